@@ -39,7 +39,6 @@ constexpr uint32_t kPush = 0, kPull = 1;
 constexpr int32_t kPullLight = 32;  // rows up to this length are scanned by one lane
 constexpr int kPullPer = 8;         // vertices per thread per pull pass
 constexpr int kPullIlp = 8;         // row entries a lane loads at once
-constexpr int32_t kSmallPush = 1 << 18;  // push levels up to this many edges prefetch rows
 
 // ctl layout (uint64 words): [0..2] frontier counters (ring), [4] edges
 // traversed, [5] entries expanded, [6] levels, [16 + 16 i] edges scanned by
@@ -96,11 +95,16 @@ struct BfsOp {
     int32_t *depth;
     uint32_t *fb_next;  // next-frontier bitmap (null when only pushing)
     int32_t nd;
-    __device__ __forceinline__ bool edge(int32_t, int32_t, int32_t v) const {
-        uint32_t *w = vis + (v >> 5);
+    // seen at the level's start (possibly stale: the claim decides)
+    __device__ __forceinline__ bool probe(int32_t, int32_t, int32_t v, int32_t &) const {
+        return !((vis[v >> 5] >> (v & 31)) & 1u);
+    }
+    __device__ __forceinline__ uint32_t claim(int32_t v, int32_t) const {
+        return dev::atomic_or_dev(vis + (v >> 5), 1u << (v & 31));
+    }
+    __device__ __forceinline__ bool appends(int32_t) const { return true; }
+    __device__ __forceinline__ bool won(int32_t v, uint32_t old) const {
         const uint32_t bit = 1u << (v & 31);
-        if (*w & bit) return false;  // seen (possibly stale: the atomic decides)
-        const uint32_t old = dev::atomic_or_dev(w, bit);
         if (old & bit) return false;
         depth[v] = nd;
         if (fb_next)
@@ -196,18 +200,16 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(8))) voi
         return;
     }
     const uint32_t mode = decide(level, p, prev, explored, F, E);
-    __syncthreads();  // every thread has read the shared state before block 0 writes
+    // (no word read above is written by a block of this level)
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         level_books(c, level, mode, F, E, explored);
         if (mode == kPush) c.w[12] += (uint64_t)E;  // entries read by push levels
     }
     clear_slice(fb_clear, p.m / 32 + 1);
     if (mode == kPush) {
-        // small levels are latency-bound: row extents loaded with the columns
-        const bool small = E <= kSmallPush;
         BfsOp op{vis, depth, fb_next, level + 1};
         expand_tiles<kBlock, TILE, false, false, true>(op, rowptr, col, (int32_t)p.nnz, cur, F,
-                                                       E, nxt, c.cnt(level + 1), small);
+                                                       E, nxt, c.cnt(level + 1));
         return;
     }
     // pull: each thread takes kPullPer vertices of a pass; for every k the

@@ -144,6 +144,35 @@ __device__ __forceinline__ uint32_t block_exclusive_add32(uint32_t x, uint32_t *
     return r;
 }
 
+// Block-wide exclusive scan of two 32-bit values at once (each block total
+// below 2^32).  Every wave scans its lanes with DPP shifts, leaves its totals
+// in LDS and, after the only barrier, scans the block's (at most 16) wave
+// totals itself, so no thread walks them alone.  `lds` needs BLOCK / 64 words;
+// the caller puts a barrier between two scans through the same words.
+struct Pair32 {
+    uint32_t a, b;
+};
+template <int BLOCK>
+__device__ __forceinline__ Pair32 block_exclusive_add_pair(uint32_t a, uint32_t b, uint64_t *lds,
+                                                           Pair32 &total) {
+    constexpr int NW = BLOCK / 64;
+    static_assert(NW <= 64, "one lane per wave total");
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+    const uint32_t ia = wave_inclusive_add(a), ib = wave_inclusive_add(b);
+    if (lane_id() == 63) lds[w] = (uint64_t(ia) << 32) | ib;
+    __syncthreads();
+    const uint64_t t = lane_id() < NW ? lds[lane_id()] : 0;
+    const uint32_t ta = wave_inclusive_add(uint32_t(t >> 32)), tb = wave_inclusive_add(uint32_t(t));
+    total.a = wave_read_lane(ta, NW - 1);
+    total.b = wave_read_lane(tb, NW - 1);
+    Pair32 r{ia - a, ib - b};
+    if (w > 0) {
+        r.a += wave_read_lane(ta, w - 1);
+        r.b += wave_read_lane(tb, w - 1);
+    }
+    return r;
+}
+
 // Slot of `key` in an open-addressing table of mask + 1 (a power of two)
 // slots: Fibonacci hashing, the HIGH bits of key * 2^32 / phi.  (The low bits
 // of the product depend only on the key's low bits, and R-MAT hub ids share

@@ -38,10 +38,12 @@ struct FrontierBufs {
 __host__ __device__ inline uint32_t cnt_entries(uint64_t c) { return uint32_t(c >> 32); }
 __host__ __device__ inline uint32_t cnt_edges(uint64_t c) { return uint32_t(c); }
 
-constexpr uint64_t kLow40 = (uint64_t(1) << 40) - 1;
-
 // Block-wide append of up to K entries per thread.  cd[k] == 0 means "no
-// entry".  All threads of the block must call it.
+// entry"; the entries of one level are distinct vertices, so their degrees
+// add up to less than 2^31.  All threads of the block must call it, and a
+// barrier separates the call from earlier uses of s_scan and s_base (the two
+// barriers inside also order the caller's earlier LDS reads before whatever
+// LDS writes follow the call).
 template <int BLOCK, int K, int TILE, bool STORE_V>
 __device__ __forceinline__ void produce(const int32_t (&cv)[K], const int32_t (&crs)[K],
                                         const int32_t (&cd)[K], FrontierBufs nxt,
@@ -53,20 +55,15 @@ __device__ __forceinline__ void produce(const int32_t (&cv)[K], const int32_t (&
         c += cd[k] > 0 ? 1u : 0u;
         dsum += (uint32_t)cd[k];
     }
-    uint64_t packed = (uint64_t(c) << 40) | uint64_t(dsum);
-    uint64_t total;
-    uint64_t excl = dev::block_exclusive_add64<BLOCK>(packed, s_scan, total);
-    if (total == 0) return;  // uniform across the block
-    if (threadIdx.x == 0) {
-        uint64_t add = ((total >> 40) << 32) | (total & kLow40);
-        *s_base = dev::atomic_add_dev(cnt_next, add);
-    }
+    dev::Pair32 total;
+    const dev::Pair32 excl = dev::block_exclusive_add_pair<BLOCK>(c, dsum, s_scan, total);
+    if (threadIdx.x == 0 && total.a)
+        *s_base = dev::atomic_add_dev(cnt_next, (uint64_t(total.a) << 32) | total.b);
     __syncthreads();
-    uint64_t base = *s_base;
-    __syncthreads();  // s_base is reused by the next call
     if (c == 0) return;
-    uint32_t slot = cnt_entries(base) + uint32_t(excl >> 40);
-    int64_t o = (int64_t)cnt_edges(base) + (int64_t)(excl & kLow40);
+    const uint64_t base = *s_base;
+    uint32_t slot = cnt_entries(base) + excl.a;
+    int64_t o = (int64_t)cnt_edges(base) + (int64_t)excl.b;
 #pragma unroll
     for (int k = 0; k < K; ++k) {
         int32_t d = cd[k];
@@ -82,6 +79,8 @@ __device__ __forceinline__ void produce(const int32_t (&cv)[K], const int32_t (&
         }
     }
 }
+
+constexpr int kMinChunk = 256;  // edges of the smallest share of a tile (see expand_tiles)
 
 // Generic load-balanced expansion over one frontier.  Op supplies:
 //   __device__ bool edge(int32_t u, int32_t e, int32_t v)
@@ -124,22 +123,42 @@ __device__ __forceinline__ int32_t row_end_of(const Op &op, const int32_t *rowpt
     else return rowptr[v + 1];
 }
 
-// prefetch loads the row extent of every edge's endpoint together with the
-// column instead of after a successful claim: one dependent round trip less
-// per level for 8 extra bytes per edge, worth it on small (latency-bound)
-// frontiers only.  (A runtime flag: a second instantiation would duplicate
-// the LDS.)
+// An Op that claims its edges' heads with an atomic supplies it in phases
+// instead of edge(), which expand_tiles runs one after another over all of a
+// thread's edges:
+//   bool probe(u, e, v, x)   loads: is v a candidate (x: the Op's own word)
+//   uint32_t claim(v, x)     the atomics; returns the claim word's old value
+//   bool appends(x)          whether a won candidate joins the frontier
+//   bool won(v, old)         whether this claim was the first, and its stores
+template <class Op, class = void>
+struct is_phased : std::false_type {};
+template <class Op>
+struct is_phased<Op, std::void_t<decltype(&Op::claim)>> : std::true_type {};
+
 template <int BLOCK, int TILE, bool STORE_V_IN, bool STORE_V_OUT, bool PRODUCE, class Op>
 __device__ __forceinline__ void expand_tiles(ExpandLds<BLOCK, TILE, STORE_V_IN> &L, Op &op,
                                              const int32_t *__restrict__ rowptr,
                                              const int32_t *__restrict__ col, int32_t nnz,
                                              FrontierBufs cur, int32_t F, int32_t E,
-                                             FrontierBufs nxt, uint64_t *cnt_next,
-                                             bool prefetch = false) {
+                                             FrontierBufs nxt, uint64_t *cnt_next) {
     constexpr int K = TILE / BLOCK;
     int32_t *s_off = L.off, *s_start = L.start, *s_v = L.v;
-    const int32_t ntiles = (int32_t)((E + TILE - 1) / TILE);
-    for (int32_t t = blockIdx.x; t < ntiles; t += gridDim.x) {
+    const int32_t ntiles = (int32_t)(((int64_t)E + TILE - 1) / TILE);
+    // A frontier that does not fill the grid with whole tiles is walked in
+    // chunks of a tile, down to kMinChunk edges: a lane's probes go to
+    // unrelated lines, which one CU serves about one a cycle, so a tile on one
+    // CU costs 12 us however few tiles there are.  (The smallest share was set
+    // with the append's cost in view: one same-address atomic, about 10 ns, per
+    // share.)  With the phases below, 2048^2 lattice BFS 2.40 -> 1.94 ms, SSSP
+    // 1024^2 3.04 -> 2.49 ms, MIS R-MAT-20 0.42 -> 0.38 ms.
+    static_assert(TILE % kMinChunk == 0, "whole chunks per tile");
+    int32_t chunk = TILE;
+    while (chunk > kMinChunk && ((int64_t)E + chunk / 2 - 1) / (chunk / 2) <= gridDim.x)
+        chunk >>= 1;
+    const int32_t nunits = (int32_t)(((int64_t)E + chunk - 1) / chunk);
+    for (int32_t x = blockIdx.x; x < nunits; x += gridDim.x) {
+        const int32_t e0 = x * chunk, ne = min(chunk, E - e0);
+        const int32_t t = e0 / TILE;
         // entries owning this tile; every degree is >= 1, so at most TILE + 1.
         // The clamps only guard memory if the frontier were inconsistent.  A
         // frontier of one tile owns it whole (no partition lookup).
@@ -152,41 +171,65 @@ __device__ __forceinline__ void expand_tiles(ExpandLds<BLOCK, TILE, STORE_V_IN> 
             if (STORE_V_IN) s_v[j] = cur.v[i0 + j];
         }
         __syncthreads();
-        const int32_t e0 = t * TILE;
-        int32_t cv[K], crs[K], cd[K];
+        int32_t cv[K], crs[K], cd[K], idx[K], u[K];
+        // the columns of all the thread's edges first: their loads are in
+        // flight together
 #pragma unroll
         for (int k = 0; k < K; ++k) {
-            cv[k] = 0;
+            const int32_t r = threadIdx.x + k * BLOCK;
+            cv[k] = -1;
             crs[k] = 0;
             cd[k] = 0;
-            const int32_t e = e0 + threadIdx.x + k * BLOCK;
-            if (e < E) {
+            idx[k] = 0;
+            u[k] = -1;
+            if (r < ne) {
+                const int32_t e = e0 + r;
                 const int j = dev::upper_bound_m1(s_off, 0, nv, e);
-                const int32_t idx = s_start[j] + (e - s_off[j]);
-                if ((uint32_t)idx >= (uint32_t)nnz) continue;
-                int32_t v;
-                if constexpr (streams_columns<Op>::value) v = __builtin_nontemporal_load(col + idx);
-                else v = col[idx];
-                const int32_t u = STORE_V_IN ? s_v[j] : -1;
-                int32_t prs = 0, pre = 0;
-                if (PRODUCE && prefetch) {
-                    prs = rowptr[v];
-                    pre = row_end_of(op, rowptr, v);
+                idx[k] = s_start[j] + (e - s_off[j]);
+                if (STORE_V_IN) u[k] = s_v[j];
+                if ((uint32_t)idx[k] >= (uint32_t)nnz) continue;  // guard only
+                if constexpr (streams_columns<Op>::value)
+                    cv[k] = __builtin_nontemporal_load(col + idx[k]);
+                else cv[k] = col[idx[k]];
+            }
+        }
+        if constexpr (is_phased<Op>::value) {
+            // phase by phase over all the thread's edges, so that each
+            // phase's loads and atomics are in flight together and the row
+            // extents come back while the claims do
+            int32_t x[K], pre[K];
+            uint32_t old[K];
+            bool cand[K];
+#pragma unroll
+            for (int k = 0; k < K; ++k) cand[k] = cv[k] >= 0 && op.probe(u[k], idx[k], cv[k], x[k]);
+#pragma unroll
+            for (int k = 0; k < K; ++k)
+                if (cand[k]) old[k] = op.claim(cv[k], x[k]);
+#pragma unroll
+            for (int k = 0; k < K; ++k)
+                if (cand[k] && op.appends(x[k])) {
+                    crs[k] = rowptr[cv[k]];
+                    pre[k] = row_end_of(op, rowptr, cv[k]);
                 }
-                if (op.edge(u, idx, v) && PRODUCE) {
-                    if (!prefetch) {
-                        prs = rowptr[v];
-                        pre = row_end_of(op, rowptr, v);
-                    }
-                    cv[k] = v;
-                    crs[k] = prs;
-                    cd[k] = pre - prs;
+#pragma unroll
+            for (int k = 0; k < K; ++k)
+                if (cand[k] && op.appends(x[k]) && op.won(cv[k], old[k])) cd[k] = pre[k] - crs[k];
+        } else {
+#pragma unroll
+            for (int k = 0; k < K; ++k) {
+                const int32_t v = cv[k];
+                if (v >= 0 && op.edge(u[k], idx[k], v) && PRODUCE) {
+                    crs[k] = rowptr[v];
+                    cd[k] = row_end_of(op, rowptr, v) - crs[k];
                 }
             }
         }
+        // s_off / s_start are overwritten by the next chunk: produce's
+        // barriers come after their last read
         if (PRODUCE)
             produce<BLOCK, K, TILE, STORE_V_OUT>(cv, crs, cd, nxt, cnt_next, L.scan, &L.base);
-        __syncthreads();  // s_off / s_start are overwritten by the next tile
+        else
+            __syncthreads();
     }
 }
 
@@ -194,11 +237,10 @@ template <int BLOCK, int TILE, bool STORE_V_IN, bool STORE_V_OUT, bool PRODUCE, 
 __device__ __forceinline__ void expand_tiles(Op &op, const int32_t *__restrict__ rowptr,
                                              const int32_t *__restrict__ col, int32_t nnz,
                                              FrontierBufs cur, int32_t F, int32_t E,
-                                             FrontierBufs nxt, uint64_t *cnt_next,
-                                             bool prefetch = false) {
+                                             FrontierBufs nxt, uint64_t *cnt_next) {
     __shared__ ExpandLds<BLOCK, TILE, STORE_V_IN> L;
     expand_tiles<BLOCK, TILE, STORE_V_IN, STORE_V_OUT, PRODUCE>(L, op, rowptr, col, nnz, cur, F,
-                                                                 E, nxt, cnt_next, prefetch);
+                                                                 E, nxt, cnt_next);
 }
 
 template <int BLOCK, int TILE, bool STORE_V_IN, bool STORE_V_OUT, bool PRODUCE, class Op>

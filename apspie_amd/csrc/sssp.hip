@@ -83,11 +83,17 @@ struct SsspPushOp {
     const float *w;
     int32_t *dist;  // float bits
     uint32_t *fb_next;
-    __device__ __forceinline__ bool edge(int32_t u, int32_t e, int32_t v) const {
-        const int32_t nd = dev::fbits(dev::bitsf(dist[u]) + __builtin_nontemporal_load(w + e));
-        if (nd >= dist[v]) return false;
+    __device__ __forceinline__ bool probe(int32_t u, int32_t e, int32_t v, int32_t &nd) const {
+        nd = dev::fbits(dev::bitsf(dist[u]) + __builtin_nontemporal_load(w + e));
+        return nd < dist[v];
+    }
+    __device__ __forceinline__ uint32_t claim(int32_t v, int32_t nd) const {
         __hip_atomic_fetch_min(dist + v, nd, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        return claim_bit(fb_next, v);
+        return dev::atomic_or_dev(fb_next + (v >> 5), 1u << (v & 31));
+    }
+    __device__ __forceinline__ bool appends(int32_t) const { return true; }
+    __device__ __forceinline__ bool won(int32_t v, uint32_t old) const {
+        return !((old >> (v & 31)) & 1u);
     }
 };
 
@@ -100,6 +106,9 @@ struct HeavyLds {
 union DoLds {
     ExpandLds<kDoBlock, kDoTile, true> ex;
     HeavyLds hv;
+};
+struct PushLds {
+    ExpandLds<kDoBlock, kDoTile, true> ex;
 };
 
 struct HeavyOp {
@@ -124,17 +133,20 @@ __global__ void k_do_seed(const int32_t *rowptr, int32_t src, int32_t *dist, uin
     for (int32_t t = threadIdx.x; (int64_t)t * kDoTile < d; t += blockDim.x) f0.tfirst[t] = 0;
 }
 
-// two 1024-thread blocks per CU resident: at most 64 VGPRs
+// two 1024-thread blocks per CU resident: at most 64 VGPRs.  Rounds of a call
+// that never pulls (PULL false, the default) are a kernel of their own, which
+// the pull branch's registers and LDS do not weigh on.
+template <bool PULL>
 __global__ __launch_bounds__(kDoBlock) __attribute__((amdgpu_waves_per_eu(8))) void
 k_sssp_do_round(const int32_t *__restrict__ rowptr, const int32_t *__restrict__ col,
                 const float *__restrict__ w, int32_t nnz, int32_t m, int32_t *dist,
                 const uint32_t *__restrict__ fb_cur, uint32_t *fb_next, uint32_t *fb_clear,
                 FrontierBufs cur, FrontierBufs nxt, FrontierBufs heavy, uint64_t heavy_cnt,
                 int32_t pull_div, uint64_t *ctl, int32_t r) {
-    __shared__ DoLds lds;
+    __shared__ std::conditional_t<PULL, DoLds, PushLds> lds;
     const uint64_t cc = ctl[r % 3];
     const int32_t F = (int32_t)cnt_entries(cc), E = (int32_t)cnt_edges(cc);
-    const bool pull = pull_div > 0 && (int64_t)E * pull_div > (int64_t)nnz;
+    const bool pull = PULL && (int64_t)E * pull_div > (int64_t)nnz;
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         ctl[(r + 2) % 3] = 0;  // the counter of round r + 1's output
         if (F > 0) {
@@ -155,6 +167,7 @@ k_sssp_do_round(const int32_t *__restrict__ rowptr, const int32_t *__restrict__ 
                                                           E, nxt, cnt_next);
         return;
     }
+    if constexpr (PULL) {
     const int lane = dev::lane_id();
     // short rows: one lane per vertex
     for (int64_t pbase = (int64_t)blockIdx.x * kDoBlock * kDoPer; pbase < m;
@@ -284,6 +297,7 @@ k_sssp_do_round(const int32_t *__restrict__ rowptr, const int32_t *__restrict__ 
         produce<kDoBlock, 1, kDoTile, true>(hc, hrs, hcd, nxt, cnt_next, L.scan, &L.base);
         __syncthreads();  // the tile's LDS is refilled next
     }
+    }
 }
 
 // The long-row list of a graph (rows longer than kLight, with tile owners
@@ -336,7 +350,8 @@ void sssp_do(Ctx *c, const Graph *g0, int32_t source, float *dist_out, int32_t p
     for (;;) {
         kt.begin();
         for (int k = 0; k < chunk; ++k, ++r) {
-            k_sssp_do_round<<<grid, kDoBlock, 0, c->stream>>>(
+            const auto round = pull_div > 0 ? k_sssp_do_round<true> : k_sssp_do_round<false>;
+            round<<<grid, kDoBlock, 0, c->stream>>>(
                 g->rowptr, g->col, g->val, (int32_t)g->nnz, g->m, dist, fb + (r % 3) * words,
                 fb + ((r + 1) % 3) * words, fb + ((r + 2) % 3) * words, fs.f[r & 1],
                 fs.f[(r + 1) & 1], heavy, g->heavy_cnt, pull_div, fs.ctl, r);
@@ -416,15 +431,21 @@ struct SsspNearOp {
     const int32_t *rend;  // end of the row part a claimed vertex expands next
     uint32_t *hb;         // light / heavy mode: bit per vertex whose heavy entries are due
     __device__ __forceinline__ int32_t row_end(int32_t v) const { return rend[v]; }
-    __device__ __forceinline__ bool edge(int32_t u, int32_t e, int32_t v) const {
-        const int32_t nd = dev::fbits(dev::bitsf(dist[u]) + __builtin_nontemporal_load(w + e));
-        if (nd >= dist[v]) return false;
+    __device__ __forceinline__ bool probe(int32_t u, int32_t e, int32_t v, int32_t &nd) const {
+        nd = dev::fbits(dev::bitsf(dist[u]) + __builtin_nontemporal_load(w + e));
+        return nd < dist[v];
+    }
+    __device__ __forceinline__ uint32_t claim(int32_t v, int32_t nd) const {
         __hip_atomic_fetch_min(dist + v, nd, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         if (nd >= tbits) {  // far: expanded by a later split round
             pend[v] = 1;
-            return false;
+            return 0;
         }
-        if (!claim_bit(fb_next, v)) return false;
+        return dev::atomic_or_dev(fb_next + (v >> 5), 1u << (v & 31));
+    }
+    __device__ __forceinline__ bool appends(int32_t nd) const { return nd < tbits; }
+    __device__ __forceinline__ bool won(int32_t v, uint32_t old) const {
+        if ((old >> (v & 31)) & 1u) return false;
         // its light entries come next; the heavy ones once the frontier empties
         if (hb) __hip_atomic_fetch_or(hb + (v >> 5), 1u << (v & 31), __ATOMIC_RELAXED,
                                       __HIP_MEMORY_SCOPE_AGENT);
@@ -447,15 +468,16 @@ k_sssp_nf_round(const int32_t *__restrict__ rowptr, const int32_t *__restrict__ 
     const int32_t F = (int32_t)cnt_entries(cc), E = (int32_t)cnt_edges(cc);
     const int32_t tbits = (int32_t)ctl[12 + (r & 1)];
     const bool split_last = ctl[14 + (r & 1)] != 0;
-    const uint64_t left_before = nf_left(ctl, r + 2);  // left by the previous round's split
     const bool split = F == 0;
+    // left by the previous round's split (only a split round asks)
+    const uint64_t left_before = split ? nf_left(ctl, r + 2) : 0;
     const bool done = split && split_last && left_before == 0;
-    const uint64_t min_before = nf_min_left(ctl, r + 2);
+    const uint64_t min_before = split ? nf_min_left(ctl, r + 2) : ~0ull;
     const bool jump = split && !done && split_last && min_before != ~0ull;
     const float step = nf_next_step(dev::bitsf((int32_t)ctl[10 + (r & 1)]), jump);
     const int32_t tnext =
         split && !done ? nf_next_threshold(tbits, step, split_last, min_before) : tbits;
-    __syncthreads();  // every thread has read the control words
+    // (no word read above is written by a block of this round)
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         ctl[(r + 2) % 3] = 0;
         ctl[10 + ((r + 1) & 1)] = (uint64_t)(uint32_t)dev::fbits(step);
