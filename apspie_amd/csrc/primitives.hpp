@@ -19,6 +19,12 @@ void scan_exclusive_i32_async(Ctx *c, const int32_t *in, int32_t *out, int64_t n
 // be null.  Sorts in place (uses scratch ping-pong buffers).
 void radix_sort_pairs(Ctx *c, uint32_t *keys, uint32_t *vals, int64_t n, int bits);
 
+// stable LSD radix sort of (key, val) by the `bits` bits of key from bit `lo`
+// on, between two buffer pairs; vals may be null.  Returns whether the result
+// is in (kb, vb).  K: uint32_t or uint64_t.
+template <class K>
+bool radix_sort(Ctx *c, K *ka, uint32_t *va, K *kb, uint32_t *vb, int64_t n, int lo, int bits);
+
 // idx_out = the i in [0, n) with flag[i] != 0, in increasing order; returns count
 int64_t compact_flags(Ctx *c, const int32_t *flag, int64_t n, int32_t *idx_out);
 
