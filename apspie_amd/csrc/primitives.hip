@@ -12,40 +12,12 @@ constexpr int kItems = 8;        // items per thread
 constexpr int kTileN = kB * kItems;
 
 // ------------------------------------------------------------------- scan
-// Single-pass scan with decoupled look-back.  Tiles take ids from a ticket
-// counter in launch order, so every tile a block waits on belongs to a block
-// that started earlier and never waits on a later one: every wait ends.
-// status word per tile: bits 62-63 = 0 nothing, 1 aggregate, 2 inclusive
-// prefix; bits 0-61 = value.  A tile looks back with a whole wave, 64 status
-// words at a time: one dependent read per word, as one thread would make,
-// cost more than the data (a 2M-element scan 14 us; 4M elements took 58 us).
-constexpr uint64_t kFlagAgg = uint64_t(1) << 62;
-constexpr uint64_t kFlagPre = uint64_t(2) << 62;
-constexpr uint64_t kValMask = (uint64_t(1) << 62) - 1;
+// Single-pass scan with decoupled look-back (dev::chain_tiles).  Tiles take
+// ids from a ticket counter in launch order.
 // elements per thread: 16, or 4 for up to kScanSmall elements, which then
 // spread over four times the blocks (and one look-back window holds them all)
 constexpr int kScanItems = 16, kScanItemsSmall = 4;
 constexpr int64_t kScanSmall = 64 * kB * kScanItemsSmall;
-
-// sum of the tiles before `tile` (called by one whole wave; tile > 0)
-__device__ __forceinline__ uint64_t look_back(const uint64_t *status, int64_t tile) {
-    uint64_t prefix = 0;
-    for (int64_t top = tile - 1;;) {
-        const int64_t j = top - dev::lane_id();
-        const uint64_t s = j >= 0 ? dev::load_relaxed(status + j) : kFlagPre;
-        const uint64_t pre = __ballot((s & ~kValMask) == kFlagPre);
-        const int last = pre ? __ffsll((unsigned long long)pre) - 1 : 63;
-        // every word up to the nearest prefix must be there
-        const bool need = dev::lane_id() <= last;
-        if (__ballot(need && (s & ~kValMask) == 0)) {
-            __builtin_amdgcn_s_sleep(1);
-            continue;
-        }
-        prefix += dev::wave_sum_u64(need ? s & kValMask : 0);
-        if (pre) return prefix;
-        top -= 64;
-    }
-}
 
 template <int ITEMS>
 __global__ __launch_bounds__(kB) void k_scan(const int32_t *in, int32_t *out, int64_t n,
@@ -82,16 +54,8 @@ __global__ __launch_bounds__(kB) void k_scan(const int32_t *in, int32_t *out, in
     uint64_t agg;
     const uint64_t excl = dev::block_exclusive_add64<kB>(sum, s_scan, agg);
     if (threadIdx.x < 64) {
-        uint64_t prefix = 0;
-        if (tile > 0) {
-            if (threadIdx.x == 0)
-                __hip_atomic_store(status + tile, kFlagAgg | (agg & kValMask), __ATOMIC_RELAXED,
-                                   __HIP_MEMORY_SCOPE_AGENT);
-            prefix = look_back(status, tile);
-        }
+        const uint64_t prefix = dev::chain_tiles(status, tile, agg);
         if (threadIdx.x == 0) {
-            __hip_atomic_store(status + tile, kFlagPre | ((prefix + agg) & kValMask),
-                               __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             s_prefix = prefix;
             const int64_t ntiles = (n + TILE - 1) / TILE;
             if (tile == ntiles - 1 && total_dev) *total_dev = (int64_t)(prefix + agg);
