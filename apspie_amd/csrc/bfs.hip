@@ -25,6 +25,7 @@
 #include "common.hpp"
 #include "device.hpp"
 #include "frontier.hpp"
+#include "levels.hpp"
 #include "timing.hpp"
 
 namespace apspie {
@@ -37,7 +38,7 @@ namespace {
 constexpr int kBlock = 1024;
 constexpr uint32_t kPush = 0, kPull = 1;
 constexpr int32_t kPullLight = 32;  // rows up to this length are scanned by one lane
-constexpr int kPullPer = 8;         // vertices per thread per pull pass
+constexpr int kPullPer = 8;         // vertices per thread per pull pass, at most
 constexpr int kPullIlp = 8;         // row entries a lane loads at once
 
 // ctl layout (uint64 words): [0..2] frontier counters (ring), [4] edges
@@ -184,7 +185,8 @@ template <int TILE>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(8))) void k_bfs_level(
     const int32_t *__restrict__ rowptr, const int32_t *__restrict__ col, int32_t *depth,
     uint32_t *vis, const uint32_t *__restrict__ fb_cur, uint32_t *fb_next, uint32_t *fb_clear,
-    FrontierBufs cur, FrontierBufs nxt, uint64_t *ctlw, int32_t level, DoParams p) {
+    FrontierBufs cur, FrontierBufs nxt, uint64_t *ctlw, int32_t level, DoParams p,
+    Progress *prog) {
     __shared__ uint64_t s_scan[kBlock / 64 + 1];
     __shared__ uint64_t s_base;
     __shared__ uint64_t s_scanned[kBlock / 64];
@@ -194,11 +196,14 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(8))) voi
     const uint64_t prev = *c.slot(level + 1), explored = *c.expl(level + 1);
     const int32_t F = (int32_t)cnt_entries(cc), E = (int32_t)cnt_edges(cc);
     if (F == 0) {
+        if (blockIdx.x > 0) return;
         // keep the counter ring clean after the last level: the entry two
         // slots ahead still holds an old frontier and would revive it
-        if (blockIdx.x == 0 && threadIdx.x == 0) *c.cnt(level + 2) = 0;
+        if (threadIdx.x == 0) *c.cnt(level + 2) = 0;
+        report_done(prog, ctlw);
         return;
     }
+    if (blockIdx.x == 0) report_level(prog, level);
     const uint32_t mode = decide(level, p, prev, explored, F, E);
     // (no word read above is written by a block of this level)
     if (blockIdx.x == 0 && threadIdx.x == 0) {
@@ -217,10 +222,13 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(8))) voi
     // consecutive vertices (two bitmap words) and writes them without atomics.
     // All loads of a pass are issued before any of them is needed, and the
     // claims of the pass are appended with one block-wide reservation.
+    // A graph too small to fill the grid at kPullPer vertices per thread takes
+    // fewer (16,384 vertices would be two blocks' work).
     const int lane = dev::lane_id();
     uint64_t scanned = 0;
-    for (int64_t pbase = (int64_t)blockIdx.x * kBlock * kPullPer; pbase < p.m;
-         pbase += (int64_t)gridDim.x * kBlock * kPullPer) {
+    const int64_t width = (int64_t)gridDim.x * kBlock;
+    const int per = (int)min<int64_t>(kPullPer, (p.m + width - 1) / width);
+    for (int64_t pbase = (int64_t)blockIdx.x * kBlock * per; pbase < p.m; pbase += width * per) {
         int32_t cv[kPullPer], crs[kPullPer], cd[kPullPer];
         int32_t rs[kPullPer], re[kPullPer];
         bool open[kPullPer], hit[kPullPer];
@@ -233,7 +241,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(8))) voi
             hit[k] = false;
             // row extents are loaded with the visited bits, not after them
             // (coalesced, and one dependent round trip less)
-            const bool in = v < p.m;
+            const bool in = k < per && v < p.m;
             open[k] = in && !((vis[v >> 5] >> (v & 31)) & 1u);
             rs[k] = in ? rowptr[v] : 0;
             re[k] = in ? rowptr[v + 1] : 0;
@@ -390,44 +398,30 @@ void bfs_levels(Ctx *c, const Graph *g, int32_t source, int32_t *depth, const Bf
         c, kBlock, (int)std::max<int64_t>(1, opt(c, "bfs_blocks_per_cu", 8) * 256 / kBlock));
     const DoParams dp{direction, (int32_t)opt(c, "bfs_alpha", 14), (int32_t)opt(c, "bfs_beta", 24),
                       g->nnz, g->m};
-    int chunk = (int)std::max<int64_t>(1, opt(c, "bfs_levels_per_sync", 8));
     KernelTimer kt(c, b.kernel_timer);
-    uint64_t *h = (uint64_t *)c->pinned;  // copy of the control block
+    LevelFeed feed(c, levels_ahead(c));
     int level = 0;
-    for (;;) {
-        kt.begin();
-        for (int k = 0; k < chunk; ++k, ++level) {
-            const int cur = level & 1;
-            if (!do_bfs) {
-                k_expand<kBlock, TILE, false, false, true><<<grid, kBlock, 0, c->stream>>>(
-                    BfsOp{vis, depth, nullptr, level + 1}, g->rowptr, g->col, (int32_t)g->nnz,
-                    fs.f[cur], fs.ctl + (level % 3), fs.f[cur ^ 1], fs.ctl + ((level + 1) % 3),
-                    fs.ctl + ((level + 2) % 3), fs.ctl + 4);
-            } else {
-                uint32_t *fcur = fb + (level % 3) * words, *fnext = fb + ((level + 1) % 3) * words,
-                         *fclr = fb + ((level + 2) % 3) * words;
-                k_bfs_level<TILE><<<grid, kBlock, 0, c->stream>>>(
-                    g->rowptr, g->col, depth, vis, fcur, fnext, fclr, fs.f[cur], fs.f[cur ^ 1],
-                    fs.ctl, level, dp);
-            }
-            APSPIE_LAUNCH_CHECK();
+    kt.begin();
+    for (; feed.more(level); ++level) {
+        APSPIE_CHECK(level <= g->m + 256, APSPIE_ERR_DEVICE, "BFS did not converge");
+        const int cur = level & 1;
+        if (!do_bfs) {
+            k_expand<kBlock, TILE, false, false, true><<<grid, kBlock, 0, c->stream>>>(
+                BfsOp{vis, depth, nullptr, level + 1}, g->rowptr, g->col, (int32_t)g->nnz,
+                fs.f[cur], fs.ctl + (level % 3), fs.f[cur ^ 1], fs.ctl + ((level + 1) % 3),
+                fs.ctl + ((level + 2) % 3), fs.ctl + 4,
+                LevelReport{feed.device(), fs.ctl, level});
+        } else {
+            uint32_t *fcur = fb + (level % 3) * words, *fnext = fb + ((level + 1) % 3) * words,
+                     *fclr = fb + ((level + 2) % 3) * words;
+            k_bfs_level<TILE><<<grid, kBlock, 0, c->stream>>>(
+                g->rowptr, g->col, depth, vis, fcur, fnext, fclr, fs.f[cur], fs.f[cur ^ 1],
+                fs.ctl, level, dp, feed.device());
         }
-        kt.end(chunk);
-        // the whole control block in one copy: counters and statistics
-        APSPIE_HIP(hipMemcpyAsync(h, fs.ctl, kCtlWords * sizeof(uint64_t),
-                                  hipMemcpyDeviceToHost, c->stream));
-        // wait on the context's end-of-call event: when this chunk was the
-        // last, the call's timing ends here without a second round trip
-        APSPIE_HIP(hipEventRecord(c->ev1, c->stream));
-        APSPIE_HIP(hipEventSynchronize(c->ev1));
-        c->stats.host_syncs++;
-        if (cnt_entries(h[level % 3]) == 0) {
-            c->ev1_recorded = true;
-            break;
-        }
-        APSPIE_CHECK(level <= g->m + 1, APSPIE_ERR_DEVICE, "BFS did not converge");
-        chunk = std::min(chunk * 2, 256);
+        APSPIE_LAUNCH_CHECK();
     }
+    kt.end(level);
+    const uint64_t *h = feed.finish();
     c->stats.edges_traversed = (int64_t)h[4];
     c->stats.vertices_reached = (int64_t)h[5];
     c->stats.iterations = (int32_t)h[6];

@@ -17,6 +17,7 @@
 namespace apspie {
 
 constexpr int kWave = 64;  // CDNA wavefront width
+constexpr size_t kProgressBytes = 4096;
 
 // ------------------------------------------------------------------ errors
 struct Error {
@@ -113,6 +114,8 @@ struct Ctx {
     bool ev1_recorded = false;  // the call recorded ev1 after its last work itself
     // pinned host word for counters read back by the host
     void *pinned = nullptr;
+    // pinned, coherent host memory that level kernels report to (levels.hpp)
+    void *progress = nullptr;
     // the default MIS priorities (mt19937 seeded 5489, one draw per vertex)
     // for mis_prio_m vertices, kept between calls: the stream is sequential
     // and generated on the host

@@ -11,7 +11,8 @@ namespace apspie {
 static const char *kOptionNames[] = {
     "bfs_tile",          // edges per expansion tile (power of two)
     "bfs_blocks_per_cu", // resident 256-thread groups per CU for the level kernels
-    "bfs_levels_per_sync", // levels launched between host checks
+    "bfs_levels_per_sync", // levels between host checks: batched chunks of this many (rounded
+                           // up to 6), the other loops run 3/8 of it ahead of the device
     "bfs_direction",     // 0 push only, 1 direction-optimising
     "bfs_alpha",         // push->pull switch: frontier edges * alpha > unexplored edges
     "bfs_beta",          // pull->push switch: frontier vertices * beta < m
@@ -314,6 +315,8 @@ int apspie_ctx_create(int device, apspie_ctx **out) {
         APSPIE_HIP(hipEventCreate(&c->ev0));
         APSPIE_HIP(hipEventCreate(&c->ev1));
         APSPIE_HIP(hipHostMalloc(&c->pinned, 4096, hipHostMallocDefault));
+        APSPIE_HIP(hipHostMalloc(&c->progress, kProgressBytes,
+                                 hipHostMallocMapped | hipHostMallocCoherent));
         noalloc_init(device);  // the no-alloc BFS's static array, once per device
     });
     if (st != APSPIE_OK) {
@@ -341,6 +344,7 @@ int apspie_ctx_destroy(apspie_ctx *c) {
     if (c->ev0) (void)hipEventDestroy(c->ev0);
     if (c->ev1) (void)hipEventDestroy(c->ev1);
     if (c->pinned) (void)hipHostFree(c->pinned);
+    if (c->progress) (void)hipHostFree(c->progress);
     if (c->mis_prio.ptr) (void)hipFree(c->mis_prio.ptr);
     // graphs outliving their context keep their memory but lose the accounting
     for (Graph *g : c->graphs) g->owner = nullptr;

@@ -243,12 +243,66 @@ __device__ __forceinline__ void expand_tiles(Op &op, const int32_t *__restrict__
                                                                  E, nxt, cnt_next);
 }
 
+// Control block: 16 words of counters / statistics, then 16 accumulators
+// 128 bytes apart (their first eight words used, the ninth of the first is
+// kCtlReported), which blocks pick by block index so that a per-block
+// statistic does not serialise thousands of atomics on one address.
+constexpr int kCtlWords = 16 + 16 * 16;
+constexpr int kSpread = 16;
+__device__ __forceinline__ uint64_t *spread_slot(uint64_t *ctl) {
+    return ctl + 16 + (blockIdx.x % kSpread) * 16;
+}
+inline uint64_t spread_sum(const uint64_t *h) {
+    uint64_t t = 0;
+    for (int i = 0; i < kSpread; ++i) t += h[16 + i * 16];
+    return t;
+}
+
+// In pinned, coherent host memory (one per context).
+struct Progress {
+    uint64_t started;  // levels whose kernel has begun
+    uint64_t done;     // a level found nothing to do; ctl is complete
+    uint64_t pad[6];
+    uint64_t ctl[kCtlWords];
+};
+static_assert(sizeof(Progress) <= kProgressBytes, "the context's block holds it");
+
+// block 0 of level l's kernel
+__device__ __forceinline__ void report_level(Progress *p, int32_t l) {
+    if (threadIdx.x == 0)
+        __hip_atomic_store(&p->started, (uint64_t)l + 1, __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// block 0, in a kernel after the one that last wrote ctl's statistics.  One
+// wave: a system-scope release by each of a block's 16 took 7 us, in every
+// launch queued after the last level, so the first of them marks ctl too.
+constexpr int kCtlReported = 24;
+__device__ __forceinline__ void report_done(Progress *p, uint64_t *ctl) {
+    if (threadIdx.x >= 64 || ctl[kCtlReported]) return;
+    for (int i = threadIdx.x; i < kCtlWords; i += 64)
+        __hip_atomic_store(p->ctl + i, ctl[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "");
+    if (threadIdx.x == 0) {
+        __hip_atomic_store(&p->done, (uint64_t)1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        ctl[kCtlReported] = 1;
+    }
+}
+
+// What a k_expand launch of a level loop reports (progress null: nothing).
+struct LevelReport {
+    Progress *progress = nullptr;
+    uint64_t *ctl = nullptr;
+    int32_t level = 0;
+};
+
 template <int BLOCK, int TILE, bool STORE_V_IN, bool STORE_V_OUT, bool PRODUCE, class Op>
 __global__ __launch_bounds__(BLOCK) void k_expand(Op op, const int32_t *__restrict__ rowptr,
                                                   const int32_t *__restrict__ col, int32_t nnz,
                                                   FrontierBufs cur, const uint64_t *cnt_cur,
                                                   FrontierBufs nxt, uint64_t *cnt_next,
-                                                  uint64_t *cnt_clear, uint64_t *stats) {
+                                                  uint64_t *cnt_clear, uint64_t *stats,
+                                                  LevelReport rep = LevelReport{}) {
     const uint64_t cc = *cnt_cur;
     const int32_t F = (int32_t)cnt_entries(cc);
     const int32_t E = (int32_t)cnt_edges(cc);
@@ -259,6 +313,10 @@ __global__ __launch_bounds__(BLOCK) void k_expand(Op op, const int32_t *__restri
             stats[1] += (uint64_t)F;  // entries expanded
             stats[2] += 1;            // levels with work
         }
+    }
+    if (rep.progress && blockIdx.x == 0) {
+        if (F > 0) report_level(rep.progress, rep.level);
+        else report_done(rep.progress, rep.ctl);
     }
     if (F == 0) return;
     expand_tiles<BLOCK, TILE, STORE_V_IN, STORE_V_OUT, PRODUCE>(op, rowptr, col, nnz, cur, F, E,
@@ -275,8 +333,10 @@ __global__ __launch_bounds__(BLOCK) void k_build(Op op, const int32_t *__restric
     __shared__ uint64_t s_scan[BLOCK / 64 + 1];
     __shared__ uint64_t s_base;
     if (n_from_counter) n = (int32_t)cnt_entries(*n_from_counter);
-    const int64_t per_block = (int64_t)BLOCK * K;
-    for (int64_t b0 = (int64_t)blockIdx.x * per_block; b0 < n; b0 += (int64_t)gridDim.x * per_block) {
+    // at most K per thread, fewer where that would leave blocks without work
+    const int64_t width = (int64_t)gridDim.x * BLOCK;
+    const int per = (int)min<int64_t>(K, (n + width - 1) / width);
+    for (int64_t b0 = (int64_t)blockIdx.x * BLOCK * per; b0 < n; b0 += width * per) {
         int32_t cv[K], crs[K], cd[K];
 #pragma unroll
         for (int k = 0; k < K; ++k) {
@@ -284,7 +344,7 @@ __global__ __launch_bounds__(BLOCK) void k_build(Op op, const int32_t *__restric
             crs[k] = 0;
             cd[k] = 0;
             const int64_t i = b0 + threadIdx.x + (int64_t)k * BLOCK;
-            if (i < n) {
+            if (k < per && i < n) {
                 const int32_t v = list ? list[i] : (int32_t)i;
                 if (op.keep(v)) {
                     const int32_t rs = rowptr[v];
@@ -296,20 +356,6 @@ __global__ __launch_bounds__(BLOCK) void k_build(Op op, const int32_t *__restric
         }
         produce<BLOCK, K, TILE, STORE_V>(cv, crs, cd, nxt, cnt_next, s_scan, &s_base);
     }
-}
-
-// Control block: 16 words of counters / statistics, then 16 accumulators
-// 128 bytes apart, which blocks pick by block index so that a per-block
-// statistic does not serialise thousands of atomics on one address.
-constexpr int kCtlWords = 16 + 16 * 16;
-constexpr int kSpread = 16;
-__device__ __forceinline__ uint64_t *spread_slot(uint64_t *ctl) {
-    return ctl + 16 + (blockIdx.x % kSpread) * 16;
-}
-inline uint64_t spread_sum(const uint64_t *h) {
-    uint64_t t = 0;
-    for (int i = 0; i < kSpread; ++i) t += h[16 + i * 16];
-    return t;
 }
 
 // Near-far split bookkeeping in the spread slots: the split of round r adds

@@ -18,6 +18,7 @@
 #include "common.hpp"
 #include "device.hpp"
 #include "frontier.hpp"
+#include "levels.hpp"
 #include "timing.hpp"
 
 namespace apspie {
@@ -142,7 +143,7 @@ k_sssp_do_round(const int32_t *__restrict__ rowptr, const int32_t *__restrict__ 
                 const float *__restrict__ w, int32_t nnz, int32_t m, int32_t *dist,
                 const uint32_t *__restrict__ fb_cur, uint32_t *fb_next, uint32_t *fb_clear,
                 FrontierBufs cur, FrontierBufs nxt, FrontierBufs heavy, uint64_t heavy_cnt,
-                int32_t pull_div, uint64_t *ctl, int32_t r) {
+                int32_t pull_div, uint64_t *ctl, int32_t r, Progress *prog) {
     __shared__ std::conditional_t<PULL, DoLds, PushLds> lds;
     const uint64_t cc = ctl[r % 3];
     const int32_t F = (int32_t)cnt_entries(cc), E = (int32_t)cnt_edges(cc);
@@ -155,6 +156,10 @@ k_sssp_do_round(const int32_t *__restrict__ rowptr, const int32_t *__restrict__ 
             ctl[6] += 1;
             ctl[7] += pull ? (uint64_t)nnz : (uint64_t)E;  // CSR entries read
         }
+    }
+    if (blockIdx.x == 0) {
+        if (F > 0) report_level(prog, r);
+        else report_done(prog, ctl);
     }
     if (F == 0) return;
     for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < m / 32 + 1;
@@ -340,33 +345,21 @@ void sssp_do(Ctx *c, const Graph *g0, int32_t source, float *dist_out, int32_t p
     const FrontierBufs heavy{g->heavy_v, g->heavy_start, g->heavy_off, g->heavy_tfirst};
     const int grid = fill_grid(
         c, kDoBlock, (int)std::max<int64_t>(1, opt(c, "bfs_blocks_per_cu", 8) * 256 / kDoBlock));
-    // rounds between host checks: the option first, then 4, 8, 16, ... (the
-    // idle tail of the last chunk is a launch per round)
-    int chunk = (int)std::max<int64_t>(1, opt(c, "bfs_levels_per_sync", 8));
-    int grow = 4;
     KernelTimer kt(c);
-    uint64_t *h = (uint64_t *)c->pinned;
+    LevelFeed feed(c, levels_ahead(c));
+    const auto round = pull_div > 0 ? k_sssp_do_round<true> : k_sssp_do_round<false>;
     int r = 0;
-    for (;;) {
-        kt.begin();
-        for (int k = 0; k < chunk; ++k, ++r) {
-            const auto round = pull_div > 0 ? k_sssp_do_round<true> : k_sssp_do_round<false>;
-            round<<<grid, kDoBlock, 0, c->stream>>>(
-                g->rowptr, g->col, g->val, (int32_t)g->nnz, g->m, dist, fb + (r % 3) * words,
-                fb + ((r + 1) % 3) * words, fb + ((r + 2) % 3) * words, fs.f[r & 1],
-                fs.f[(r + 1) & 1], heavy, g->heavy_cnt, pull_div, fs.ctl, r);
-            APSPIE_LAUNCH_CHECK();
-        }
-        kt.end(chunk);
-        APSPIE_HIP(hipMemcpyAsync(h, fs.ctl, 16 * sizeof(uint64_t), hipMemcpyDeviceToHost,
-                                  c->stream));
-        sync(c);
-        c->stats.host_syncs++;
-        if (cnt_entries(h[r % 3]) == 0) break;
-        APSPIE_CHECK(r <= 4 * g->m + 64, APSPIE_ERR_DEVICE, "SSSP did not converge");
-        chunk = grow;
-        grow = std::min(grow * 2, 256);
+    kt.begin();
+    for (; feed.more(r); ++r) {
+        APSPIE_CHECK(r <= 4 * (int64_t)g->m + 256, APSPIE_ERR_DEVICE, "SSSP did not converge");
+        round<<<grid, kDoBlock, 0, c->stream>>>(
+            g->rowptr, g->col, g->val, (int32_t)g->nnz, g->m, dist, fb + (r % 3) * words,
+            fb + ((r + 1) % 3) * words, fb + ((r + 2) % 3) * words, fs.f[r & 1],
+            fs.f[(r + 1) & 1], heavy, g->heavy_cnt, pull_div, fs.ctl, r, feed.device());
+        APSPIE_LAUNCH_CHECK();
     }
+    kt.end(r);
+    const uint64_t *h = feed.finish();
     c->stats.edges_traversed = (int64_t)h[4];
     c->stats.vertices_reached = (int64_t)h[5];
     c->stats.iterations = (int32_t)h[6];
@@ -460,7 +453,7 @@ k_sssp_nf_round(const int32_t *__restrict__ rowptr, const int32_t *__restrict__ 
                 const float *w, int32_t nnz, int32_t m, int32_t *dist, uint32_t *fb_next,
                 uint32_t *fb_clear, uint8_t *pend, FrontierBufs cur,
                 FrontierBufs nxt, uint64_t *ctl, int32_t r, const int32_t *rend,
-                uint32_t *hb) {
+                uint32_t *hb, Progress *prog) {
     __shared__ ExpandLds<kNfBlock, TILE, true> lds;
     __shared__ uint64_t s_part[kNfBlock / 64];
     __shared__ uint32_t s_min[kNfBlock / 64];
@@ -493,6 +486,12 @@ k_sssp_nf_round(const int32_t *__restrict__ rowptr, const int32_t *__restrict__ 
             ctl[6] += 1;  // split rounds count as rounds
         }
     }
+    // finished: the last round was a split that left nothing pending and
+    // found nothing below the new threshold
+    if (blockIdx.x == 0) {
+        if (!done) report_level(prog, r);
+        else report_done(prog, ctl);
+    }
     if (done) return;
     // the bitmap round r + 1 claims into (round r claims into another)
     for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < m / 32 + 1;
@@ -512,8 +511,9 @@ k_sssp_nf_round(const int32_t *__restrict__ rowptr, const int32_t *__restrict__ 
     // has read it (nothing marks during a split).
     uint64_t left = 0;
     uint32_t min_left = ~0u;  // smallest distance left pending (bits)
-    for (int64_t pbase = (int64_t)blockIdx.x * kNfBlock * kNfPer; pbase < m;
-         pbase += (int64_t)gridDim.x * kNfBlock * kNfPer) {
+    const int64_t width = (int64_t)gridDim.x * kNfBlock;
+    const int per = (int)min<int64_t>(kNfPer, (m + width - 1) / width);
+    for (int64_t pbase = (int64_t)blockIdx.x * kNfBlock * per; pbase < m; pbase += width * per) {
         int32_t cv[kNfPer], crs[kNfPer], cd[kNfPer], hrs[kNfPer], hd[kNfPer];
         bool take[kNfPer], drop[kNfPer], marked[kNfPer];
 #pragma unroll
@@ -522,6 +522,7 @@ k_sssp_nf_round(const int32_t *__restrict__ rowptr, const int32_t *__restrict__ 
             cv[k] = (int32_t)v;
             crs[k] = cd[k] = hrs[k] = hd[k] = 0;
             take[k] = drop[k] = marked[k] = false;
+            if (k >= per) continue;
             if (v < m && pend[v]) {
                 const int32_t dv = dist[v];
                 if (dv < tbits) drop[k] = true;  // lowered below T since: already expanded
@@ -684,34 +685,20 @@ void sssp_near_far(Ctx *c, const Graph *g, int32_t source, float *dist_out, floa
     APSPIE_LAUNCH_CHECK();
     const int grid = fill_grid(
         c, kNfBlock, (int)std::max<int64_t>(1, opt(c, "bfs_blocks_per_cu", 8) * 256 / kNfBlock));
-    // rounds between host checks: the option first, then 4, 8, 16, ... (the
-    // idle tail of the last chunk is a launch per round)
-    int chunk = (int)std::max<int64_t>(1, opt(c, "bfs_levels_per_sync", 8));
-    int grow = 4;
     KernelTimer kt(c);
-    uint64_t *h = (uint64_t *)c->pinned;
+    LevelFeed feed(c, levels_ahead(c));
     int r = 0;
-    for (;;) {
-        kt.begin();
-        for (int k = 0; k < chunk; ++k, ++r) {
-            k_sssp_nf_round<TILE><<<grid, kNfBlock, 0, c->stream>>>(
-                g->rowptr, col, val, (int32_t)g->nnz, g->m, dist,
-                fb + ((r + 1) % 3) * words, fb + ((r + 2) % 3) * words, pend, fs.f[r & 1],
-                fs.f[(r + 1) & 1], fs.ctl, r, rend, hb);
-            APSPIE_LAUNCH_CHECK();
-        }
-        kt.end(chunk);
-        APSPIE_HIP(hipMemcpyAsync(h, fs.ctl, kCtlWords * sizeof(uint64_t), hipMemcpyDeviceToHost,
-                                  c->stream));
-        sync(c);
-        c->stats.host_syncs++;
-        // finished when the last round was a split that left nothing pending
-        // and found nothing below the new threshold
-        if (cnt_entries(h[r % 3]) == 0 && h[14 + (r & 1)] != 0 && nf_left(h, r + 2) == 0) break;
-        APSPIE_CHECK(r <= 8 * g->m + 1024, APSPIE_ERR_DEVICE, "SSSP did not converge");
-        chunk = grow;
-        grow = std::min(grow * 2, 256);
+    kt.begin();
+    for (; feed.more(r); ++r) {
+        APSPIE_CHECK(r <= 8 * (int64_t)g->m + 1024, APSPIE_ERR_DEVICE, "SSSP did not converge");
+        k_sssp_nf_round<TILE><<<grid, kNfBlock, 0, c->stream>>>(
+            g->rowptr, col, val, (int32_t)g->nnz, g->m, dist, fb + ((r + 1) % 3) * words,
+            fb + ((r + 2) % 3) * words, pend, fs.f[r & 1], fs.f[(r + 1) & 1], fs.ctl, r, rend,
+            hb, feed.device());
+        APSPIE_LAUNCH_CHECK();
     }
+    kt.end(r);
+    const uint64_t *h = feed.finish();
     c->stats.edges_traversed = (int64_t)h[4];
     c->stats.vertices_reached = (int64_t)h[5];
     c->stats.iterations = (int32_t)h[6];

@@ -42,3 +42,27 @@ def test_shares_of_a_level(k, d, extra):
         assert np.array_equal(ctx.bfs_batch(G, [0, 1])[0], want)
         assert np.array_equal(ctx.sssp_batch(G, [0, 1])[0], wd)
         G.close()
+
+
+@pytest.mark.parametrize("ahead", [1, 2, 8, 64])
+@pytest.mark.parametrize("key", ["lattice64", "rmat12", "path300", "one"])
+def test_loops_at_any_run_ahead(ahead, key):
+    """Level loops whose host side runs 1 to 24 levels ahead of the device,
+    from a single vertex (no level has work) to hundreds of levels, call after
+    call on one context."""
+    g = {"lattice64": lambda: T.lattice(64), "rmat12": lambda: T.rmat(12),
+         "path300": lambda: T.path_graph(300), "one": lambda: T.empty_graph(1)}[key]()
+    with A.Context(0) as ctx:
+        ctx.set_option("bfs_levels_per_sync", ahead)
+        G = ctx.upload(g.rowptr32, g.col, g.w)
+        for src in (0, g.m // 2, g.m - 1):
+            want, _ = O.bfs(g.m, g.rowptr, g.col, src)
+            wd = O.sssp(g.m, g.rowptr, g.col, g.w, src)
+            wd = np.where(wd == -1, A.SSSP_INF, wd).astype(np.float32)
+            for direction in (1, 0):
+                ctx.set_option("bfs_direction", direction)
+                assert np.array_equal(ctx.bfs(G, src), want)
+            for delta in (0, 32, 200):
+                ctx.set_option("sssp_delta", delta)
+                assert np.array_equal(ctx.sssp(G, src), wd)
+        G.close()
