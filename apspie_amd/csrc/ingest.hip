@@ -387,19 +387,37 @@ __device__ __forceinline__ uint32_t f_order(float f) {
     return (b & 0x80000000u) ? ~b : (b | 0x80000000u);
 }
 
-__global__ void k_weight_range(const float *w, int64_t n, uint32_t *out) {
+// One pair of atomics per block: one per wave on the same two words took 80 us
+// whatever the size.
+__global__ __launch_bounds__(kBlock) void k_weight_range(const float *w, int64_t n,
+                                                         uint32_t *out) {
+    constexpr int U = 8;
+    __shared__ uint32_t s_lo[kBlock / 64], s_hi[kBlock / 64];
     uint32_t lo = 0xffffffffu, hi = 0;
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
-         i += (int64_t)gridDim.x * blockDim.x) {
-        const uint32_t k = f_order(w[i]);
-        lo = min(lo, k);
-        hi = max(hi, k);
+    const int64_t stride = (int64_t)gridDim.x * kBlock;
+    for (int64_t i0 = blockIdx.x * (int64_t)kBlock + threadIdx.x; i0 < n; i0 += stride * U) {
+        float x[U];
+#pragma unroll
+        for (int k = 0; k < U; ++k) x[k] = w[min(i0 + k * stride, n - 1)];
+#pragma unroll
+        for (int k = 0; k < U; ++k) {
+            const uint32_t q = f_order(x[k]);
+            lo = min(lo, q);
+            hi = max(hi, q);
+        }
     }
-    for (int off = 32; off > 0; off >>= 1) {
-        lo = min(lo, (uint32_t)__shfl_xor((int)lo, off, 64));
-        hi = max(hi, (uint32_t)__shfl_xor((int)hi, off, 64));
-    }
+    lo = dev::wave_min_u32(lo);
+    hi = dev::wave_max_u32(hi);
     if (dev::lane_id() == 0) {
+        s_lo[threadIdx.x / 64] = lo;
+        s_hi[threadIdx.x / 64] = hi;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int q = 1; q < kBlock / 64; ++q) {
+            lo = min(lo, s_lo[q]);
+            hi = max(hi, s_hi[q]);
+        }
         atomicMin(out, lo);
         atomicMax(out + 1, hi);
     }

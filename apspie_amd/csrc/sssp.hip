@@ -15,6 +15,8 @@
 // the next frontier's bitmap).
 // With integer-valued weights every sum is exact, so the fixed point does not
 // depend on the relaxation order.
+#include <cmath>
+
 #include "common.hpp"
 #include "device.hpp"
 #include "frontier.hpp"
@@ -574,41 +576,188 @@ k_sssp_nf_round(const int32_t *__restrict__ rowptr, const int32_t *__restrict__ 
     }
 }
 
-// Rows split by value for the light / heavy mode: one wave per row counts
-// its light entries (value below delta), then writes them first and the
-// heavy ones after them, each part in CSR order (ballot ranks), and records
-// where the light part ends.
+// Rows split by value for the light / heavy mode: the light entries (value
+// below delta) first and the heavy ones after them, each part in CSR order
+// (ballot ranks), and where the light part ends.  kLfLanes lanes take a row of
+// up to kLfShort entries at once, all its columns and values in flight; the
+// wave then takes its longer rows one by one, counting before it writes; and
+// rows above kLfWave go to a list for whole blocks, 8192 entries a step.  (One
+// wave walked a hub's 200,000 entries twice, 64 at a time: R-MAT-22 6.1 -> 1.8
+// ms, R-MAT-20 2.25 -> 0.49.)
 constexpr int kLfBlock = 256;
+constexpr int kLfLanes = 16, kLfPer = 4, kLfShort = kLfLanes * kLfPer;
+constexpr int32_t kLfStep = 64 * kLfPer, kLfWave = 2048;
 __global__ __launch_bounds__(kLfBlock) void k_light_first(const int32_t *__restrict__ rowptr,
                                                           const int32_t *__restrict__ col,
                                                           const float *__restrict__ val,
                                                           int32_t m, float delta, int32_t *lcol,
-                                                          float *lval, int32_t *lend) {
-    const int lane = dev::lane_id();
+                                                          float *lval, int32_t *lend,
+                                                          int32_t *hubs, uint32_t *nhubs) {
+    constexpr int kRows = 64 / kLfLanes;
+    const int lane = dev::lane_id(), sub = lane % kLfLanes;
     const uint64_t below = (1ull << lane) - 1;
-    const int64_t nwaves = (int64_t)gridDim.x * (blockDim.x / 64);
-    for (int64_t v = blockIdx.x * (int64_t)(blockDim.x / 64) + threadIdx.x / 64; v < m;
-         v += nwaves) {
-        const int32_t rs = rowptr[v], re = rowptr[v + 1];
-        uint64_t nl = 0;
-        for (int32_t e = rs + lane; e < re; e += 64) nl += val[e] < delta ? 1 : 0;
-        nl = dev::wave_sum_u64(nl);
-        int32_t lpos = rs, hpos = rs + (int32_t)nl;
-        for (int32_t e0 = rs; e0 < re; e0 += 64) {
-            const int32_t e = e0 + lane;
-            const bool in = e < re;
-            const float x = in ? val[e] : 0.0f;
-            const bool light = in && x < delta;
-            const uint64_t bl = __ballot(light), bh = __ballot(in && !light);
+    const uint64_t group = ((1ull << kLfLanes) - 1) << (lane - sub);
+    const int64_t step = (int64_t)gridDim.x * (kLfBlock / 64) * kRows;
+    for (int64_t v0 = (blockIdx.x * (int64_t)(kLfBlock / 64) + threadIdx.x / 64) * kRows; v0 < m;
+         v0 += step) {
+        const int64_t v = v0 + lane / kLfLanes;
+        const int32_t rs = v < m ? rowptr[v] : 0, re = v < m ? rowptr[v + 1] : 0;
+        const bool mine = re - rs <= kLfShort;
+        float x[kLfPer];
+        int32_t c[kLfPer];
+#pragma unroll
+        for (int k = 0; k < kLfPer; ++k) {
+            const int32_t e = rs + k * kLfLanes + sub;
+            const bool in = mine && e < re;
+            x[k] = in ? val[e] : 0.0f;
+            c[k] = in ? col[e] : 0;
+        }
+        uint64_t bl[kLfPer];
+        int32_t nl = 0;
+#pragma unroll
+        for (int k = 0; k < kLfPer; ++k) {
+            const bool in = mine && rs + k * kLfLanes + sub < re;
+            bl[k] = __ballot(in && x[k] < delta) & group;
+            nl += __popcll(bl[k]);
+        }
+        int32_t lpos = rs, hpos = rs + nl;
+#pragma unroll
+        for (int k = 0; k < kLfPer; ++k) {
+            const bool in = mine && rs + k * kLfLanes + sub < re;
+            const bool light = in && x[k] < delta;
+            const uint64_t bh = __ballot(in && !light) & group;
             if (in) {
-                const int32_t p = light ? lpos + __popcll(bl & below) : hpos + __popcll(bh & below);
-                lcol[p] = col[e];
-                lval[p] = x;
+                const int32_t p = light ? lpos + __popcll(bl[k] & below) : hpos + __popcll(bh & below);
+                lcol[p] = c[k];
+                lval[p] = x[k];
             }
-            lpos += __popcll(bl);
+            lpos += __popcll(bl[k]);
             hpos += __popcll(bh);
         }
-        if (lane == 0) lend[v] = rs + (int32_t)nl;
+        if (mine && sub == 0 && v < m) lend[v] = rs + nl;
+        if (re - rs > kLfWave && sub == 0) hubs[dev::atomic_add_dev(nhubs, 1u)] = (int32_t)v;
+        uint64_t longm = __ballot(!mine && re - rs <= kLfWave && sub == 0);
+        while (longm) {
+            const int from = __ffsll((unsigned long long)longm) - 1;
+            longm &= longm - 1;
+            const int32_t ls = __shfl(rs, from, 64), le = __shfl(re, from, 64);
+            // kLfStep entries a step, their loads in flight; a row of one
+            // step is counted from the registers it is written from
+            uint32_t cnt = 0;
+            if (le - ls > kLfStep) {
+                for (int32_t e0 = ls; e0 < le; e0 += kLfStep)
+#pragma unroll
+                    for (int k = 0; k < kLfPer; ++k) {
+                        const int32_t e = e0 + k * 64 + lane;
+                        cnt += e < le && val[e] < delta ? 1u : 0u;
+                    }
+                cnt = (uint32_t)dev::wave_sum_u64(cnt);
+            }
+            int32_t lp = ls, hp = ls + (int32_t)cnt;
+            for (int32_t e0 = ls; e0 < le; e0 += kLfStep) {
+                float y[kLfPer];
+                int32_t d[kLfPer];
+                uint64_t ml[kLfPer], mh[kLfPer];
+#pragma unroll
+                for (int k = 0; k < kLfPer; ++k) {
+                    const int32_t e = e0 + k * 64 + lane;
+                    y[k] = e < le ? val[e] : 0.0f;
+                    d[k] = e < le ? col[e] : 0;
+                }
+                uint32_t step = 0;
+#pragma unroll
+                for (int k = 0; k < kLfPer; ++k) {
+                    const bool in = e0 + k * 64 + lane < le, light = y[k] < delta;
+                    ml[k] = __ballot(in && light);
+                    mh[k] = __ballot(in && !light);
+                    step += __popcll(ml[k]);
+                }
+                if (le - ls <= kLfStep) {
+                    cnt = step;
+                    hp = ls + (int32_t)cnt;
+                }
+#pragma unroll
+                for (int k = 0; k < kLfPer; ++k) {
+                    if (e0 + k * 64 + lane < le) {
+                        const int32_t p = (ml[k] >> lane) & 1u ? lp + __popcll(ml[k] & below)
+                                                               : hp + __popcll(mh[k] & below);
+                        lcol[p] = d[k];
+                        lval[p] = y[k];
+                    }
+                    lp += __popcll(ml[k]);
+                    hp += __popcll(mh[k]);
+                }
+            }
+            if (lane == from) lend[v] = ls + (int32_t)cnt;
+        }
+    }
+}
+
+constexpr int kLfHubBlock = 1024, kLfHubPer = 8;
+__global__ __launch_bounds__(kLfHubBlock) void k_light_first_hubs(
+    const int32_t *__restrict__ rowptr, const int32_t *__restrict__ col,
+    const float *__restrict__ val, float delta, int32_t *lcol, float *lval, int32_t *lend,
+    const int32_t *hubs, const uint32_t *nhubs) {
+    constexpr int kStep = kLfHubBlock * kLfHubPer;
+    __shared__ uint64_t s_scan[kLfHubBlock / 64];
+    const int lane = dev::lane_id();
+    const uint64_t below = (1ull << lane) - 1;
+    const uint32_t n = *nhubs;
+    for (uint32_t q = blockIdx.x; q < n; q += gridDim.x) {
+        const int32_t v = hubs[q], rs = rowptr[v], re = rowptr[v + 1];
+        // a wave takes kLfHubPer * 64 consecutive entries of a step
+        const int32_t first = rs + (threadIdx.x & ~63) * kLfHubPer + lane;
+        uint32_t cnt = 0;
+        for (int32_t e0 = 0; first - lane + e0 < re; e0 += kStep)
+#pragma unroll
+            for (int k = 0; k < kLfHubPer; ++k) {
+                const int32_t e = first + e0 + k * 64;
+                cnt += e < re && val[e] < delta ? 1u : 0u;
+            }
+        dev::Pair32 tot;
+        (void)dev::block_exclusive_add_pair<kLfHubBlock>(cnt, 0u, s_scan, tot);
+        const int32_t nl = (int32_t)tot.a;
+        if (threadIdx.x == 0) lend[v] = rs + nl;
+        int32_t lp = rs, hp = rs + nl;
+        for (int32_t e0 = 0; rs + e0 < re; e0 += kStep) {
+            float x[kLfHubPer];
+            int32_t c[kLfHubPer];
+            uint64_t ml[kLfHubPer], mh[kLfHubPer];
+            uint32_t wl = 0, wh = 0;
+#pragma unroll
+            for (int k = 0; k < kLfHubPer; ++k) {
+                const int32_t e = first + e0 + k * 64;
+                x[k] = e < re ? val[e] : 0.0f;
+                c[k] = e < re ? col[e] : 0;
+            }
+#pragma unroll
+            for (int k = 0; k < kLfHubPer; ++k) {
+                const bool in = first + e0 + k * 64 < re, light = x[k] < delta;
+                ml[k] = __ballot(in && light);
+                mh[k] = __ballot(in && !light);
+                wl += __popcll(ml[k]);
+                wh += __popcll(mh[k]);
+            }
+            __syncthreads();  // s_scan's last readers
+            const dev::Pair32 ex = dev::block_exclusive_add_pair<kLfHubBlock>(
+                lane == 0 ? wl : 0u, lane == 0 ? wh : 0u, s_scan, tot);
+            int32_t l = lp + (int32_t)dev::wave_read_lane(ex.a, 0);
+            int32_t h = hp + (int32_t)dev::wave_read_lane(ex.b, 0);
+#pragma unroll
+            for (int k = 0; k < kLfHubPer; ++k) {
+                if (first + e0 + k * 64 < re) {
+                    const int32_t p = (ml[k] >> lane) & 1u ? l + __popcll(ml[k] & below)
+                                                           : h + __popcll(mh[k] & below);
+                    lcol[p] = c[k];
+                    lval[p] = x[k];
+                }
+                l += __popcll(ml[k]);
+                h += __popcll(mh[k]);
+            }
+            lp += (int32_t)tot.a;
+            hp += (int32_t)tot.b;
+        }
+        __syncthreads();  // s_scan is written by the next row
     }
 }
 
@@ -631,11 +780,17 @@ Graph::LightFirst graph_light_first(Ctx *c, Graph *g, float delta) {
     int32_t *lend = (int32_t *)((char *)mem + 2 * ecol);
     try {
         if (g->m > 0) {
-            // a wave per row and every row its own wave: the two passes over
-            // a row are a few dependent loads, so the grid covers the rows
-            const int grid = (int)std::min<int64_t>(ceil_div(g->m, kLfBlock / 64), 1 << 24);
-            k_light_first<<<grid, kLfBlock, 0, c->stream>>>(g->rowptr, g->col, g->val, g->m,
-                                                            delta, lcol, lval, lend);
+            // every group of rows its own wave: a few dependent loads each
+            const int grid = (int)std::min<int64_t>(
+                ceil_div(g->m, kLfBlock / kLfLanes), 1 << 24);
+            uint32_t *nhubs = (uint32_t *)scratch(
+                c, "sssp_hubs", sizeof(int32_t) * ((size_t)(g->nnz / kLfWave) + 2));
+            fill_i32(c, (int32_t *)nhubs, 0, 1);
+            k_light_first<<<grid, kLfBlock, 0, c->stream>>>(
+                g->rowptr, g->col, g->val, g->m, delta, lcol, lval, lend, (int32_t *)nhubs + 1,
+                nhubs);
+            k_light_first_hubs<<<fill_grid(c, kLfHubBlock, 2), kLfHubBlock, 0, c->stream>>>(
+                g->rowptr, g->col, g->val, delta, lcol, lval, lend, (int32_t *)nhubs + 1, nhubs);
             APSPIE_LAUNCH_CHECK();
         }
         sync(c);
@@ -727,21 +882,35 @@ double sssp_weight_delta(Ctx *c, Graph *g) {
     return d;
 }
 
-// The width used when sssp_delta is left at -1: the width the weights
-// suggest from 2^22 vertices on, and from 2^20 on where that width splits
-// the weights into light and heavy entries (light / heavy rounds on);
-// Bellman-Ford rounds (0) otherwise, where the rounds' fixed cost outweighs
-// the re-expansions near-far saves.  Measured at weights 1..255, ms per
-// source, Bellman-Ford / width 64 with light / heavy rounds: R-MAT-18
-// 0.58 / 0.94, R-MAT-20 1.42 / 1.33, R-MAT-21 2.21 / 1.91, R-MAT-22 4.03 /
-// 2.90; the lattices' width (512) is above every weight, and 512^2-1024^2
-// run faster without splits.
+// The width used when sssp_delta is left at -1.
+//
+// Sparse rows (the weights' width above every weight, so that no entry is
+// heavy): four times that width from kNfSparse vertices on -- the rounds'
+// fixed cost (about 8 us) weighs more than the re-expansions a wider bucket
+// adds -- and Bellman-Ford rounds (0) below.  Lattices at weights 1..255, ms
+// per source, Bellman-Ford / 512 / 2048 / 8192: 512^2 1.14 / 1.76 / 1.30 /
+// 1.28, 724^2 1.43 / - / 1.51 / -, 887^2 1.76 / - / 1.62 / -, 1024^2 2.06 / 2.28
+// / 1.73 / 2.17, 1500^2 3.40 / 2.87 / 2.33 / 3.36, 2048^2 5.68 / 3.27 / 2.84 /
+// 4.45.
+//
+// Longer rows (light / heavy rounds): 1.42 * largest weight / sqrt(mean row),
+// narrower on large graphs by (2^20 / m)^0.4, from kNfHeavy vertices on (below
+// it they gain less than the light-first copy costs a graph's first call).
+// R-MAT, edge factor 16, Bellman-Ford / 32 / 48 / 64 / 96: 2^17 0.45 / 0.52 /
+// 0.46 / 0.44 / 0.44, 2^18 0.67 / 0.67 / 0.52 / 0.55 / 0.57, 2^20 1.39 / 1.15 /
+// 1.08 / 1.07 / 1.12, 2^22 4.44 / 2.67 / 2.76 / 2.93 / 3.23; edge factor 8: 2^20
+// 1.09 / 0.99 / 0.87 / 0.92 / 0.78, 2^22 2.95 / 1.99 / 1.94 / 2.00 / 2.19.
+constexpr int32_t kNfSparse = 3 << 18, kNfHeavy = 1 << 20;
 double sssp_auto_delta(Ctx *c, Graph *g) {
-    if (g->m >= (1 << 22)) return sssp_weight_delta(c, g);
-    if (g->m < (1 << 20) || opt(c, "sssp_light_heavy", 1) == 0) return 0;
+    if (g->m < std::min(kNfSparse, kNfHeavy)) return 0;
     const double d = sssp_weight_delta(c, g);
     float lo = 0.0f, hi = 0.0f;
-    return d > 0 && graph_weight_range(c, g, &lo, &hi) && lo < d && hi >= d ? d : 0;
+    if (!(d > 0) || !graph_weight_range(c, g, &lo, &hi)) return 0;
+    if (d > hi) return g->m >= kNfSparse ? 4 * d : 0;
+    if (opt(c, "sssp_light_heavy", 1) == 0) return g->m >= (1 << 22) ? d : 0;
+    const double w = 1.42 * hi / std::sqrt(std::max(1.0, (double)g->nnz / g->m)) *
+                     std::min(1.0, std::pow((double)(1 << 20) / g->m, 0.4));
+    return w > lo && w <= hi ? w : d;
 }
 
 // The batched SSSP width when batch_sssp_delta is left at -1: the weights'
