@@ -99,26 +99,20 @@ struct BfsBatchOp {
     }
 };
 
-// Claims of a pull level are collected in an LDS queue and appended to the
-// next frontier kQueue at a time: one 64-bit reservation per flush instead of
-// one per pass (a pass covers only 256 / W * 4 vertices, and thousands of
+// Claims of a pulled SSSP round are collected in an LDS queue and appended to
+// the next frontier kQueue at a time: one 64-bit reservation per flush instead
+// of one per pass (a pass covers only 256 / W * 4 vertices, and thousands of
 // reservations on one counter serialise in the L2).
 constexpr int kQueue = 1536;
-// rows longer than kLongRow still open after their first probes are finished
-// after the pass by a whole wave each (kLongCap per block and pass, every
-// vertex of a pass at W = 1)
-constexpr int32_t kLongRow = 64;
-constexpr int kLongCap = 1024;
 struct PullQueue {
     int32_t v[kQueue], rs[kQueue], d[kQueue];
-    int32_t lv[kLongCap];
-    uint32_t n, nl;
+    uint32_t n;
     uint32_t scan32[kBlock / 64 + 1];
     uint64_t scan[kBlock / 64 + 1];
     uint64_t base;
 };
 
-// LDS of the level kernel: the push branch's expansion or the pull's queue
+// LDS of a near-far round: the push's expansion or the pull's queue
 union BatchLds {
     ExpandLds<kBlock, kTile, true> ex;
     PullQueue pq;
@@ -142,19 +136,63 @@ __device__ __forceinline__ void queue_flush(PullQueue &q, FrontierBufs nxt, uint
     __syncthreads();
 }
 
+// A wave's claims of one pass join the block's LDS queue with one LDS atomic;
+// no barrier.  The caller flushes the queue before it can overflow.
+template <int KP>
+__device__ __forceinline__ void wave_enqueue(PullQueue &q, const int32_t (&cv)[KP],
+                                             const int32_t (&crs)[KP], const int32_t (&cd)[KP]) {
+    uint64_t bm[KP];
+    uint32_t c = 0;
+#pragma unroll
+    for (int k = 0; k < KP; ++k) {
+        bm[k] = __ballot(cd[k] > 0);
+        c += __popcll(bm[k]);
+    }
+    if (c == 0) return;  // uniform in the wave
+    uint32_t pos = 0;
+    if (dev::lane_id() == 0) pos = atomicAdd(&q.n, c);
+    pos = dev::wave_read_lane(pos, 0);
+#pragma unroll
+    for (int k = 0; k < KP; ++k) {
+        if (cd[k] > 0) {
+            const uint32_t to = pos + __popcll(bm[k] & dev::lanemask_lt());
+            q.v[to] = cv[k];
+            q.rs[to] = crs[k];
+            q.d[to] = cd[k];
+        }
+        pos += __popcll(bm[k]);
+    }
+}
+
+// rows longer than kLongRow still open after their first probes are finished
+// after the pass by a whole wave each (kLongCap per block and pass, every
+// vertex of a pass at W = 1)
+constexpr int32_t kLongRow = 64;
+constexpr int kLongCap = 1024;
+struct LongRows {
+    int32_t v[kLongCap];
+    uint32_t n;
+};
+
+// LDS of a pulled level
+template <bool LONG>
+struct PullLds {
+    std::conditional_t<LONG, LongRows, int32_t> rows;
+    uint64_t scan[kBlock / 64];
+};
+
 // Writes one pulled vertex's word w: nw = the bits found and not yet visited
-// (uv = the word's unvisited bits).  Returns whether anything was found.
+// (uv = the word's unvisited bits).  Every row of dst is written, so that it
+// needs no clearing; with `kept` it is a snapshot, from which the depths are
+// read at the end.
 template <int W>
 __device__ __forceinline__ void pull_finish(int64_t i, uint32_t nw, uint32_t uv, uint32_t *vis,
-                                            uint32_t *next, uint32_t *snap, int32_t *depth,
+                                            uint32_t *dst, bool kept, int32_t *depth,
                                             int32_t level, int64_t v, int w) {
-    // with a snapshot the level's discoveries are one full bit row per
-    // vertex (the depths are read back from it at the end)
-    if (snap) snap[i] = nw;
-    next[i] = nw;  // every row: the buffer needs no clearing before a pull
+    dst[i] = nw;
     if (nw) {
         vis[i] = ~uv | nw;
-        if (!snap)
+        if (!kept)
             while (nw) {
                 const int b = __ffs(nw) - 1;
                 nw &= nw - 1;
@@ -163,23 +201,23 @@ __device__ __forceinline__ void pull_finish(int64_t i, uint32_t nw, uint32_t uv,
     }
 }
 
-// The deferred long rows of a pull pass (q.lv[0 .. nl)), one wave per row:
-// lane l ORs the frontier rows of entries l, l + 64, ...; every kLongStep
-// entries the wave checks whether every unvisited bit of every word has been
-// found.  Lane w < W then writes word w like pull_finish, and lane 0 appends
-// a claim to the queue (room was made for nl claims).
+// The deferred long rows of a pull pass, one wave per row: lane l ORs the
+// frontier rows of entries l, l + 64, ...; every kLongStep entries the wave
+// checks whether every unvisited bit of every word has been found.  Lane w <
+// W then writes word w like pull_finish, and lane 0 counts a claim.
 constexpr int kLongStep = 256;
 template <int W>
-__device__ __noinline__ void pull_long(PullQueue &q, uint32_t nl,
-                                       const int32_t *__restrict__ rowptr,
-                                       const int32_t *__restrict__ col,
-                                       const uint32_t *__restrict__ front, uint32_t *vis,
-                                       uint32_t *next, uint32_t *snap, int32_t *depth,
-                                       int32_t level) {
+__device__ __noinline__ dev::Pair32 pull_long(const LongRows &q, uint32_t nl,
+                                              const int32_t *__restrict__ rowptr,
+                                              const int32_t *__restrict__ col,
+                                              const uint32_t *__restrict__ front, uint32_t *vis,
+                                              uint32_t *dst, bool kept, int32_t *depth,
+                                              int32_t level) {
     const int lane = dev::lane_id();
     const int wave = threadIdx.x / 64, nwaves = kBlock / 64;
+    dev::Pair32 found{0, 0};
     for (uint32_t j = wave; j < nl; j += nwaves) {
-        const int64_t v = q.lv[j];
+        const int64_t v = q.v[j];
         const int32_t rs = rowptr[v], re = rowptr[v + 1];
         uint32_t uv[W], acc[W];
         load_row<W>(vis + v * W, uv);
@@ -214,55 +252,65 @@ __device__ __noinline__ void pull_long(PullQueue &q, uint32_t nl,
                 my_uv = uv[w];
             }
         }
-        if (lane < W) pull_finish<W>(v * W + lane, mine, my_uv, vis, next, snap, depth, level, v, lane);
+        if (lane < W)
+            pull_finish<W>(v * W + lane, mine, my_uv, vis, dst, kept, depth, level, v, lane);
         if (lane == 0 && any) {
-            const uint32_t pos = atomicAdd(&q.n, 1u);
-            q.v[pos] = (int32_t)v;
-            q.rs[pos] = rs;
-            q.d[pos] = re - rs;
+            found.a += 1;
+            found.b += (uint32_t)(re - rs);
         }
     }
+    return found;
 }
 
 // Pull form of one batched BFS level, for symmetric CSR (a row lists the
 // vertex's in-neighbours): a group of W lanes owns vertex v, lane w its source
 // word w.  The lane ORs word w of its neighbours' frontier rows (coalesced:
 // the group reads a W-word row at once), keeps the bits not yet visited, and
-// writes the visited / next words and the depths itself -- no atomics.  The
-// loads of KP vertices per thread are issued stage by stage.  A row longer
-// than kLongRow that is still open after its first Q neighbours (a hub whose
-// sources are not all in reach at this level would otherwise be walked entry
-// by entry by its own lanes: 30 ms levels at R-MAT-22) is queued in LDS and
-// finished after the pass by one wave, its 64 lanes striding the row and
-// checking every 256 entries whether every unvisited bit has been found.
-template <int W>
-__device__ __forceinline__ void batch_pull(PullQueue &q, const int32_t *__restrict__ rowptr,
+// writes the visited word and its row of dst itself -- no atomics.  The loads
+// of KP vertices per thread are issued stage by stage.
+//
+// The level only counts its claims (vertices and the edges of their rows, which
+// the next level's direction needs): the rows of dst are the next frontier,
+// and its queue is built from them only when a push follows (k_bfs_between).
+// Queueing every claim wrote 48 MB of a level's 470 on the 2048^2 lattice at
+// 128 sources, and a next row beside the snapshot another 67: 185 -> 120 us a
+// level, 17.9 -> 12.8 ms a batch.
+//
+// LONG (some row has more than kLongRow entries): a row longer than that still
+// open after its first Q neighbours (a hub whose sources are not all in reach
+// at this level would otherwise be walked entry by entry by its own lanes:
+// 30 ms levels at R-MAT-22) is queued in LDS and finished after the pass by
+// one wave, its 64 lanes striding the row and checking every 256 entries
+// whether every unvisited bit has been found.
+template <int W, bool LONG>
+__device__ __forceinline__ void batch_pull(PullLds<LONG> &lds, const int32_t *__restrict__ rowptr,
                                            const int32_t *__restrict__ col, int32_t m,
                                            const uint32_t *__restrict__ front, uint32_t *vis,
-                                           uint32_t *next, int32_t *depth, int32_t level,
-                                           uint32_t *snap, FrontierBufs nxt, uint64_t *cnt_next) {
+                                           uint32_t *dst, bool kept, int32_t *depth,
+                                           int32_t level, uint64_t *count) {
     constexpr int VPB = kBlock / W;  // vertices per block row
-    constexpr int KP = 4;            // block rows per pass
+    // block rows per pass: two keep a wave to 64 VGPRs and every wave resident
+    // (2048^2 lattice, 128 sources, one / two / three / four: 13.2 / 12.8 /
+    // 13.0 / 14.0 ms); with long rows three, for their list's barriers (R-MAT-20,
+    // 128 sources, two / three / four: 9.5 / 8.1 / 8.8 ms)
+    constexpr int KP = LONG ? 3 : 2;
     constexpr int Q = 4;             // neighbours loaded at once
-    if (threadIdx.x == 0) {
-        q.n = 0;
-        q.nl = 0;
+    if constexpr (LONG) {
+        if (threadIdx.x == 0) lds.rows.n = 0;
+        __syncthreads();
     }
-    __syncthreads();
     const int g = threadIdx.x / W, w = threadIdx.x % W;
     const int lane = dev::lane_id();
-    const uint64_t gmask = W == 64 ? ~0ull : (((1ull << W) - 1) << ((lane / W) * W));
+    const uint64_t gmask = ((1ull << W) - 1) << ((lane / W) * W);
     const int leader = (lane / W) * W;  // the group's first lane
+    dev::Pair32 found{0, 0};
     for (int64_t pbase = (int64_t)blockIdx.x * VPB * KP; pbase < m;
          pbase += (int64_t)gridDim.x * VPB * KP) {
-        int32_t cv[KP], crs[KP], cd[KP], rs[KP], re[KP];
+        int32_t rs[KP], re[KP];
         uint32_t uv[KP], acc[KP];
 #pragma unroll
         for (int k = 0; k < KP; ++k) {
             const int64_t v = pbase + (int64_t)k * VPB + g;
-            cv[k] = (int32_t)v;
-            crs[k] = 0;
-            cd[k] = 0;
             acc[k] = 0;
             const bool in = v < m;
             uv[k] = in ? ~vis[v * W + w] : 0u;
@@ -274,107 +322,115 @@ __device__ __forceinline__ void batch_pull(PullQueue &q, const int32_t *__restri
 #pragma unroll
         for (int k = 0; k < KP; ++k)
 #pragma unroll
-            for (int q = 0; q < Q; ++q)
-                u[k][q] = uv[k] && rs[k] + q < re[k] ? col[rs[k] + q] : -1;
+            for (int t = 0; t < Q; ++t)
+                u[k][t] = uv[k] && rs[k] + t < re[k] ? col[rs[k] + t] : -1;
 #pragma unroll
         for (int k = 0; k < KP; ++k)
 #pragma unroll
-            for (int q = 0; q < Q; ++q)
-                if (u[k][q] >= 0) acc[k] |= front[(int64_t)u[k][q] * W + w];
+            for (int t = 0; t < Q; ++t)
+                if (u[k][t] >= 0) acc[k] |= front[(int64_t)u[k][t] * W + w];
 #pragma unroll
         for (int k = 0; k < KP; ++k) {
-            // an open long row goes to the LDS list (the group's leader
-            // reserves a slot); the pass then finishes it as if nothing was
-            // found -- no more entries, no bits -- and the long-row pass after
-            // the block's next barrier rewrites its words
-            if (__ballot(re[k] - rs[k] > kLongRow) != 0) {  // uniform: a long row in this wave
-                const bool open = (__ballot((acc[k] & uv[k]) != uv[k]) & gmask) != 0;
-                int slot = -1;
-                if (open && re[k] - rs[k] > kLongRow && w == 0)
-                    slot = (int)atomicAdd(&q.nl, 1u);
-                slot = __shfl(slot, leader, 64);
-                if (slot >= 0 && slot < kLongCap) {
-                    if (w == 0) q.lv[slot] = cv[k];
-                    acc[k] = 0;
-                    re[k] = rs[k] + Q;
+            const int32_t v = (int32_t)(pbase + (int64_t)k * VPB + g);
+            if constexpr (LONG) {
+                // an open long row goes to the LDS list (the group's leader
+                // reserves a slot); the pass then finishes it as if nothing
+                // was found -- no more entries, no bits -- and the long-row
+                // pass after the block's next barrier rewrites its words
+                if (__ballot(re[k] - rs[k] > kLongRow) != 0) {  // uniform in the wave
+                    const bool open = (__ballot((acc[k] & uv[k]) != uv[k]) & gmask) != 0;
+                    int slot = -1;
+                    if (open && re[k] - rs[k] > kLongRow && w == 0)
+                        slot = (int)atomicAdd(&lds.rows.n, 1u);
+                    slot = __shfl(slot, leader, 64);
+                    if (slot >= 0 && slot < kLongCap) {
+                        if (w == 0) lds.rows.v[slot] = v;
+                        acc[k] = 0;
+                        re[k] = rs[k] + Q;
+                    }
                 }
             }
             for (int32_t e = rs[k] + Q; e < re[k] && (acc[k] & uv[k]) != uv[k]; e += Q) {
                 int32_t uu[Q];
 #pragma unroll
-                for (int q = 0; q < Q; ++q) uu[q] = e + q < re[k] ? col[e + q] : -1;
+                for (int t = 0; t < Q; ++t) uu[t] = e + t < re[k] ? col[e + t] : -1;
 #pragma unroll
-                for (int q = 0; q < Q; ++q)
-                    if (uu[q] >= 0) acc[k] |= front[(int64_t)uu[q] * W + w];
+                for (int t = 0; t < Q; ++t)
+                    if (uu[t] >= 0) acc[k] |= front[(int64_t)uu[t] * W + w];
             }
         }
 #pragma unroll
         for (int k = 0; k < KP; ++k) {
+            const int64_t v = pbase + (int64_t)k * VPB + g;
             const uint32_t nw = acc[k] & uv[k];
-            if (cv[k] < m)
-                pull_finish<W>((int64_t)cv[k] * W + w, nw, uv[k], vis, next, snap, depth, level,
-                               cv[k], w);
+            if (v < m)
+                pull_finish<W>(v * W + w, nw, uv[k], vis, dst, kept, depth, level, v, w);
             const uint64_t bm = __ballot(nw != 0);
             if (w == 0 && (bm & gmask)) {
-                crs[k] = rs[k];
-                cd[k] = re[k] - rs[k];
+                found.a += 1;
+                found.b += (uint32_t)(re[k] - rs[k]);
             }
         }
-        // append this pass's claims to the queue (flushing it first if full)
-        uint32_t c = 0;
-#pragma unroll
-        for (int k = 0; k < KP; ++k) c += cd[k] > 0 ? 1u : 0u;
-        uint32_t total;
-        uint32_t pos = dev::block_exclusive_add32<kBlock>(c, q.scan32, total);
-        if (q.n + total > (uint32_t)kQueue) queue_flush(q, nxt, cnt_next);
-        pos += q.n;
-#pragma unroll
-        for (int k = 0; k < KP; ++k)
-            if (cd[k] > 0) {
-                q.v[pos] = cv[k];
-                q.rs[pos] = crs[k];
-                q.d[pos] = cd[k];
-                ++pos;
+        if constexpr (LONG) {
+            __syncthreads();  // the pass's list is complete
+            const uint32_t nl = min(lds.rows.n, (uint32_t)kLongCap);
+            if (nl > 0) {
+                const dev::Pair32 f = pull_long<W>(lds.rows, nl, rowptr, col, front, vis, dst,
+                                                   kept, depth, level);
+                found.a += f.a;
+                found.b += f.b;
+                __syncthreads();  // every wave is done with the list
+                if (threadIdx.x == 0) lds.rows.n = 0;
             }
-        __syncthreads();  // every thread has read q.n
-        if (threadIdx.x == 0) q.n += total;
-        __syncthreads();
-        // the pass's long rows, one wave each; their claims join the queue
-        const uint32_t nl = min(q.nl, (uint32_t)kLongCap);
-        if (nl > 0) {
-            if (q.n + nl > (uint32_t)kQueue) queue_flush(q, nxt, cnt_next);
-            pull_long<W>(q, nl, rowptr, col, front, vis, next, snap, depth, level);
-            __syncthreads();  // every wave is done with q.lv and q.n
-            if (threadIdx.x == 0) q.nl = 0;
             __syncthreads();
         }
     }
-    if (q.n > 0) queue_flush(q, nxt, cnt_next);
+    dev::Pair32 all;
+    (void)dev::block_exclusive_add_pair<kBlock>(found.a, found.b, lds.scan, all);
+    if (threadIdx.x == 0 && all.a)
+        dev::atomic_add_dev(count, (uint64_t(all.a) << 32) | all.b);
 }
 
 // Snapshots of pulled levels: the j-th pulled level writes its discovered
 // bits for every vertex to snap + j * stride and its level number to
-// level_of[j], up to cap levels (later pulled levels write depths directly):
-// one full bit row per vertex instead of a scattered 4-byte depth store per
-// discovered (vertex, source) pair.  npull[l & 1] holds the number of
-// snapshots taken before level l (two slots: a level reads one and block 0
-// writes the other).
+// level_of[j], up to cap levels (later pulled levels write the next frontier
+// buffer and depths directly): one full bit row per vertex instead of a
+// scattered 4-byte depth store per discovered (vertex, source) pair.  The
+// snapshot is also the next level's frontier.  Per level parity (a level
+// reads its own words and block 0 writes the next level's): npull = snapshots
+// taken before the level, src = where its frontier rows are (0 the front
+// buffer, j + 1 snapshot j), pulled = the level before it was pulled.
 struct BatchSnap {
     uint32_t *snap;
     int64_t stride;
     int32_t cap;
     int32_t *level_of;
-    uint64_t *npull;
+    uint64_t *npull;   // [2]
+    uint64_t *src;     // [2]
+    uint64_t *pulled;  // [2]
+    uint64_t *build;   // counter of the queue built before a push
+    // a pulled level's claims, per parity, in kSpread words 128 bytes apart
+    // (one word for the grid's 2048 blocks cost 20 us a level); k_bfs_between
+    // sums them into the next level's counter
+    uint64_t *claims;
+    __device__ const uint32_t *front_of(int32_t level, const uint32_t *buffer) const {
+        const uint64_t j = src[level & 1];
+        return j ? snap + (int64_t)(j - 1) * stride : buffer;
+    }
 };
 
+// Both forms of a level and k_bfs_between choose by the same rule: pull when
+// the union frontier's edges E * pull_div > nnz (pull_div 0: never).
+__device__ __forceinline__ bool batch_pulls(uint64_t cnt, int32_t pull_div, int32_t nnz) {
+    return pull_div > 0 && (int64_t)cnt_edges(cnt) * pull_div > (int64_t)nnz;
+}
+
 // One batched BFS level: push (load-balanced expansion of the union
-// frontier) or pull, chosen identically by every block from the union
-// frontier's edge count: pull when E * pull_div > nnz (pull_div 0: never).
-// The two forms are separate kernels (each level launches both; the one
-// whose form was not chosen returns at once), so the pull kernel is not held
-// to the push expansion's register count.
-template <int W, bool PULL>
-__device__ __forceinline__ void batch_level(BatchLds &lds, const int32_t *__restrict__ rowptr,
+// frontier) or pull.  The two forms are separate kernels (each level launches
+// both; the one whose form was not chosen returns at once), so the pull
+// kernel is not held to the push expansion's register count.
+template <int W, bool PULL, bool LONG, class Lds>
+__device__ __forceinline__ void batch_level(Lds &lds, const int32_t *__restrict__ rowptr,
                                             const int32_t *__restrict__ col, int32_t nnz,
                                             int32_t m, BfsBatchOp<W> &op, uint32_t *next_w,
                                             int32_t pull_div, FrontierBufs cur,
@@ -384,29 +440,33 @@ __device__ __forceinline__ void batch_level(BatchLds &lds, const int32_t *__rest
     const uint64_t cc = *cnt_cur;
     const int32_t F = (int32_t)cnt_entries(cc);
     const int32_t E = (int32_t)cnt_edges(cc);
-    const bool pull = pull_div > 0 && (int64_t)E * pull_div > (int64_t)nnz;
-    if (pull != PULL) return;
+    if (batch_pulls(cc, pull_div, nnz) != PULL) return;
     const int32_t level = *op.lvl;
     const uint64_t j = sn.npull[level & 1];
-    const bool take = pull && (int64_t)j < (int64_t)sn.cap;
+    const bool take = PULL && (int64_t)j < (int64_t)sn.cap;
+    op.front = sn.front_of(level, op.front);
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         *cnt_clear = 0;
         if (F > 0) {
             stats[0] += (uint64_t)E;  // union-frontier edges
             stats[1] += (uint64_t)F;  // union-frontier entries
             stats[2] += 1;            // levels with work
-            if (pull) stats[3] += 1;  // of which pulled
+            if (PULL) stats[3] += 1;  // of which pulled
             sn.npull[(level + 1) & 1] = j + (take ? 1 : 0);
+            sn.src[(level + 1) & 1] = take ? j + 1 : 0;
+            sn.pulled[(level + 1) & 1] = PULL ? 1 : 0;
+            *sn.build = 0;
             if (take) sn.level_of[j] = level;
         }
     }
     if (F == 0) return;
     if constexpr (PULL)
-        batch_pull<W>(lds.pq, rowptr, col, m, op.front, op.vis, next_w, op.depth, level,
-                      take ? sn.snap + (int64_t)j * sn.stride : nullptr, nxt, cnt_next);
+        batch_pull<W, LONG>(lds, rowptr, col, m, op.front, op.vis,
+                            take ? sn.snap + (int64_t)j * sn.stride : next_w, take, op.depth,
+                            level, sn.claims + (blockIdx.x % kSpread) * 16 + (level & 1));
     else
-        expand_tiles<kBlock, kTile, true, true, true>(lds.ex, op, rowptr, col, nnz, cur, F, E,
-                                                       nxt, cnt_next);
+        expand_tiles<kBlock, kTile, true, true, true>(lds, op, rowptr, col, nnz, cur, F, E, nxt,
+                                                       cnt_next);
 }
 
 template <int W>
@@ -415,20 +475,93 @@ __global__ __launch_bounds__(kBlock) void k_batch_bfs_push(
     BfsBatchOp<W> op, uint32_t *next_w, int32_t pull_div, FrontierBufs cur,
     const uint64_t *cnt_cur, FrontierBufs nxt, uint64_t *cnt_next, uint64_t *cnt_clear,
     uint64_t *stats, BatchSnap sn) {
-    __shared__ BatchLds lds;
-    batch_level<W, false>(lds, rowptr, col, nnz, m, op, next_w, pull_div, cur, cnt_cur, nxt,
-                          cnt_next, cnt_clear, stats, sn);
+    __shared__ ExpandLds<kBlock, kTile, true> lds;
+    batch_level<W, false, false>(lds, rowptr, col, nnz, m, op, next_w, pull_div, cur, cnt_cur,
+                                 nxt, cnt_next, cnt_clear, stats, sn);
 }
 
-template <int W>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(6))) void k_batch_bfs_pull(
+template <int W, bool LONG>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(8))) void k_batch_bfs_pull(
     const int32_t *__restrict__ rowptr, const int32_t *__restrict__ col, int32_t nnz, int32_t m,
     BfsBatchOp<W> op, uint32_t *next_w, int32_t pull_div, FrontierBufs cur,
     const uint64_t *cnt_cur, FrontierBufs nxt, uint64_t *cnt_next, uint64_t *cnt_clear,
     uint64_t *stats, BatchSnap sn) {
-    __shared__ BatchLds lds;
-    batch_level<W, true>(lds, rowptr, col, nnz, m, op, next_w, pull_div, cur, cnt_cur, nxt,
-                         cnt_next, cnt_clear, stats, sn);
+    __shared__ PullLds<LONG> lds;
+    batch_level<W, true, LONG>(lds, rowptr, col, nnz, m, op, next_w, pull_div, cur, cnt_cur, nxt,
+                               cnt_next, cnt_clear, stats, sn);
+}
+
+// After a BFS level: advances the level, makes the buffers ready for the next
+// level and builds its queue if it needs one.  A level's front buffer must be
+// zero again before a push writes into it as the next one:
+//   - its frontier was in a snapshot: the buffer was not written;
+//   - its queue exists (the level before it pushed, or it pushed itself):
+//     the rows of the queue's vertices;
+//   - otherwise (pulled after a pulled level without a snapshot): all of it,
+//     unless the next level pulls too, and then overwrites every row.
+// A push after a pulled level gets its queue from the rows that level wrote.
+// par: the level's parity (levels of a captured chunk keep theirs).
+template <int W>
+__global__ __launch_bounds__(kBlock) void k_bfs_between(
+    const int32_t *__restrict__ rowptr, int32_t m, int32_t nnz, int32_t pull_div,
+    FrontierBufs cur, FrontierBufs nxt, const uint64_t *cnt, uint64_t *cnt_next,
+    uint32_t *front, const uint32_t *next, int32_t *lvl, int32_t par, BatchSnap sn) {
+    constexpr int K = 4;
+    __shared__ uint64_t s_scan[kBlock / 64];
+    __shared__ uint64_t s_base;
+    const uint64_t cc = *cnt;
+    const int32_t F = (int32_t)cnt_entries(cc);
+    if (F == 0) return;
+    const bool pulled = batch_pulls(cc, pull_div, nnz);
+    uint64_t cn = 0;
+    if (pulled) {
+#pragma unroll
+        for (int q = 0; q < kSpread; ++q) cn += sn.claims[q * 16 + par];
+    } else {
+        cn = *cnt_next;
+    }
+    if (blockIdx.x == 0) {
+        if (threadIdx.x == 0) {
+            *lvl += 1;
+            if (pulled) *cnt_next = cn;
+        }
+        if (threadIdx.x < kSpread) sn.claims[threadIdx.x * 16 + (par ^ 1)] = 0;
+    }
+    const bool pulls_next = batch_pulls(cn, pull_div, nnz);
+    if (sn.src[par] == 0) {
+        if (!pulled || !sn.pulled[par]) {
+            for (int64_t i = blockIdx.x * (int64_t)kBlock + threadIdx.x; i < (int64_t)F * W;
+                 i += (int64_t)gridDim.x * kBlock)
+                front[(int64_t)cur.v[i / W] * W + (i % W)] = 0;
+        } else if (!pulls_next) {
+            for (int64_t i = blockIdx.x * (int64_t)kBlock + threadIdx.x; i < (int64_t)m * W;
+                 i += (int64_t)gridDim.x * kBlock)
+                front[i] = 0;
+        }
+    }
+    if (!pulled || pulls_next || cnt_entries(cn) == 0) return;
+    const uint32_t *rows = sn.front_of(par ^ 1, next);
+    const int64_t width = (int64_t)gridDim.x * kBlock;
+    for (int64_t b0 = (int64_t)blockIdx.x * kBlock * K; b0 < m; b0 += width * K) {
+        int32_t cv[K], crs[K], cd[K];
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+            const int64_t v = b0 + k * kBlock + threadIdx.x;
+            cv[k] = (int32_t)v;
+            crs[k] = cd[k] = 0;
+            if (v < m) {
+                uint32_t x[W], any = 0;
+                load_row<W>(rows + v * W, x);
+#pragma unroll
+                for (int w = 0; w < W; ++w) any |= x[w];
+                if (any) {
+                    crs[k] = rowptr[v];
+                    cd[k] = rowptr[v + 1] - crs[k];
+                }
+            }
+        }
+        produce<kBlock, K, kTile, true>(cv, crs, cd, nxt, sn.build, s_scan, &s_base);
+    }
 }
 
 // Near-far rounds for the batch (the single-source scheme with one threshold
@@ -442,16 +575,31 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(6))) voi
 // ctl: [10 + (r & 1)] the step of round r, [12 + (r & 1)] T of round r,
 // [14 + (r & 1)] round r - 1 was a split,
 // pending bits left by the split of round r in the spread slots (r % 3).
-template <int W>
+//
+// SM: distances are source-major ([nsrc][m], the caller's result itself)
+// instead of vertex-major ([m][32W], transposed at the end).  Graphs with
+// short rows and long paths have few sources near any vertex at a time (1.6 of
+// 32 on the 2048^2 lattice), each on a ring of neighbouring vertices: a
+// vertex-major line then holds one or two useful distances, a source-major one
+// those of the ring's next vertices: 32 sources 22.9 -> 19.0 ms, pulled both
+// ways.  Where many sources relax an edge at once (R-MAT) vertex-major is one
+// line per end.
+template <int W, bool SM>
 struct SsspBatchNearOp {
     const uint32_t *front;
     uint32_t *next;
     uint32_t *pend;  // null: no threshold (every improvement is near)
     int32_t *stamp;
-    int32_t *dist;  // [m][32W] float bits
+    int32_t *dist;  // float bits
+    int64_t m;
     const float *wt;
     const int32_t *lvl;  // device round counter
     int32_t tbits;
+    // distance of source 32 w + b at v: word_of(v, w)[b * stride()]
+    __device__ __forceinline__ int32_t *word_of(int64_t v, int w) const {
+        return SM ? dist + (int64_t)(w * 32) * m + v : dist + v * (32 * W) + w * 32;
+    }
+    __device__ __forceinline__ int64_t stride() const { return SM ? m : 1; }
     // the edge u -> v (e = CSR position): relax every source of front[u]
     // (the row read at once), four sources at a time with their distance
     // loads in flight.  An improvement is judged against the distance read,
@@ -459,7 +607,7 @@ struct SsspBatchNearOp {
     // write can leave a spurious frontier bit, which costs a re-expansion,
     // never a wrong result.
     __device__ __forceinline__ bool edge(int32_t u, int32_t e, int32_t v) const {
-        constexpr int B = 32 * W;
+        const int64_t st = stride();
         uint32_t fr[W];
         load_row<W>(front + (int64_t)u * W, fr);
         uint32_t anyf = 0;
@@ -471,8 +619,8 @@ struct SsspBatchNearOp {
         for (int w = 0; w < W; ++w) {
             uint32_t f = fr[w];
             if (!f) continue;
-            const int32_t *du_row = dist + (int64_t)u * B + w * 32;
-            int32_t *dv_row = dist + (int64_t)v * B + w * 32;
+            const int32_t *du_row = word_of(u, w);
+            int32_t *dv_row = word_of(v, w);
             uint32_t near = 0, far = 0;
             while (f) {
                 int b[4];
@@ -484,15 +632,15 @@ struct SsspBatchNearOp {
                 int32_t du[4], dv[4];
 #pragma unroll
                 for (int q = 0; q < 4; ++q) {
-                    du[q] = b[q] >= 0 ? du_row[b[q]] : 0;
-                    dv[q] = b[q] >= 0 ? dv_row[b[q]] : 0;
+                    du[q] = b[q] >= 0 ? du_row[b[q] * st] : 0;
+                    dv[q] = b[q] >= 0 ? dv_row[b[q] * st] : 0;
                 }
 #pragma unroll
                 for (int q = 0; q < 4; ++q) {
                     if (b[q] < 0) continue;
                     const int32_t nd = dev::fbits(dev::bitsf(du[q]) + we);
                     if (nd >= dv[q]) continue;
-                    __hip_atomic_fetch_min(dv_row + b[q], nd, __ATOMIC_RELAXED,
+                    __hip_atomic_fetch_min(dv_row + b[q] * st, nd, __ATOMIC_RELAXED,
                                            __HIP_MEMORY_SCOPE_AGENT);
                     if (!pend || nd < tbits) near |= 1u << b[q];
                     else far |= 1u << b[q];
@@ -525,12 +673,17 @@ struct SsspBatchNearOp {
 // the buffer needs no clearing before a pulled round.  A neighbour's
 // distance read while its owner lowers it is either value, both upper
 // bounds: the relaxations are those of the push, and so is the fixed point.
-template <int W>
+//
+// The sources of a row are relaxed four at a time over four neighbours: the
+// 16 neighbour distances and v's own four are in flight together, and v's are
+// written once.  (Neighbour by neighbour, the loads of one waited for the
+// stores of the one before.)
+template <int W, bool SM>
 __device__ __forceinline__ void batch_sssp_pull(PullQueue &q, const int32_t *__restrict__ rowptr,
                                                 const int32_t *__restrict__ col, int32_t m,
-                                                const SsspBatchNearOp<W> &op, int32_t tbits,
+                                                const SsspBatchNearOp<W, SM> &op, int32_t tbits,
                                                 FrontierBufs nxt, uint64_t *cnt_next) {
-    constexpr int B = 32 * W;
+    const int64_t st = op.stride();
     constexpr int VPB = kBlock / W;
     // vertices per group and pass, measured on the 2048^2 lattice (ms per
     // query): one for rows of one word (32 sources: 0.826 with two, 0.812
@@ -538,13 +691,15 @@ __device__ __forceinline__ void batch_sssp_pull(PullQueue &q, const int32_t *__r
     // four from four words on (128 / 256 / 512 sources: 0.616 / 0.598 /
     // 0.597 with two, 0.611 / 0.591 / 0.579 with four)
     constexpr int KP = W == 1 ? 1 : W == 2 ? 2 : 4;
-    static_assert(KP * kBlock <= kQueue, "one pass's claims fit the LDS queue");
     constexpr int Q = 4;  // row entries loaded at once
+    constexpr int S = 4;  // sources relaxed at once
+    constexpr int kPasses = kQueue / (VPB * KP);
+    static_assert(kPasses >= 1, "one pass's claims fit the LDS queue");
     if (threadIdx.x == 0) q.n = 0;
     __syncthreads();
     const int g = threadIdx.x / W, w = threadIdx.x % W;
-    const int lane = dev::lane_id();
-    const uint64_t gmask = W == 64 ? ~0ull : (((1ull << W) - 1) << ((lane / W) * W));
+    const uint64_t gmask = ((1ull << W) - 1) << ((dev::lane_id() / W) * W);
+    int pass = 0;
     for (int64_t pbase = (int64_t)blockIdx.x * VPB * KP; pbase < m;
          pbase += (int64_t)gridDim.x * VPB * KP) {
         int32_t cv[KP], crs[KP], cd[KP];
@@ -559,42 +714,48 @@ __device__ __forceinline__ void batch_sssp_pull(PullQueue &q, const int32_t *__r
             if (v < m) {
                 rs = rowptr[v];
                 re = rowptr[v + 1];
-                int32_t *dv_row = op.dist + v * B + w * 32;
+                int32_t *dv_row = op.word_of(v, w);
                 for (int32_t e0 = rs; e0 < re; e0 += Q) {
                     int32_t u[Q];
-                    uint32_t f[Q];
+                    uint32_t f[Q], x = 0;
+                    float we[Q];
 #pragma unroll
                     for (int t = 0; t < Q; ++t) u[t] = e0 + t < re ? col[e0 + t] : -1;
 #pragma unroll
-                    for (int t = 0; t < Q; ++t) f[t] = u[t] >= 0 ? op.front[(int64_t)u[t] * W + w] : 0u;
-#pragma unroll
                     for (int t = 0; t < Q; ++t) {
-                        if (!f[t]) continue;
-                        const float we = op.wt[e0 + t];
-                        const int32_t *du_row = op.dist + (int64_t)u[t] * B + w * 32;
-                        uint32_t x = f[t];
-                        while (x) {  // four sources at a time, their loads in flight
-                            int b[4];
+                        f[t] = u[t] >= 0 ? op.front[(int64_t)u[t] * W + w] : 0u;
+                        we[t] = u[t] >= 0 ? op.wt[e0 + t] : 0.0f;
+                        x |= f[t];
+                    }
+                    while (x) {
+                        int b[S];
+                        int32_t dv[S], du[S][Q];
 #pragma unroll
-                            for (int j = 0; j < 4; ++j) {
-                                b[j] = x ? __ffs(x) - 1 : -1;
-                                x &= x - 1;
-                            }
-                            int32_t du[4], dv[4];
+                        for (int j = 0; j < S; ++j) {
+                            b[j] = x ? __ffs(x) - 1 : -1;
+                            x &= x - 1;
+                        }
 #pragma unroll
-                            for (int j = 0; j < 4; ++j) {
-                                du[j] = b[j] >= 0 ? du_row[b[j]] : 0;
-                                dv[j] = b[j] >= 0 ? dv_row[b[j]] : 0;
-                            }
+                        for (int j = 0; j < S; ++j) {
+                            dv[j] = b[j] >= 0 ? dv_row[b[j] * st] : 0;
 #pragma unroll
-                            for (int j = 0; j < 4; ++j) {
-                                if (b[j] < 0) continue;
-                                const int32_t nd = dev::fbits(dev::bitsf(du[j]) + we);
-                                if (nd < dv[j]) {
-                                    dv_row[b[j]] = nd;
-                                    if (!op.pend || nd < tbits) near |= 1u << b[j];
-                                    else far |= 1u << b[j];
-                                }
+                            for (int t = 0; t < Q; ++t)
+                                du[j][t] = b[j] >= 0 && ((f[t] >> b[j]) & 1u)
+                                               ? op.word_of(u[t], w)[b[j] * st]
+                                               : -1;
+                        }
+#pragma unroll
+                        for (int j = 0; j < S; ++j) {
+                            if (b[j] < 0) continue;
+                            int32_t nd = 0x7fffffff;
+#pragma unroll
+                            for (int t = 0; t < Q; ++t)
+                                if (du[j][t] >= 0)
+                                    nd = min(nd, dev::fbits(dev::bitsf(du[j][t]) + we[t]));
+                            if (nd < dv[j]) {
+                                dv_row[b[j] * st] = nd;
+                                if (!op.pend || nd < tbits) near |= 1u << b[j];
+                                else far |= 1u << b[j];
                             }
                         }
                     }
@@ -610,25 +771,14 @@ __device__ __forceinline__ void batch_sssp_pull(PullQueue &q, const int32_t *__r
                 cd[k] = re - rs;
             }
         }
-        uint32_t c = 0;
-#pragma unroll
-        for (int k = 0; k < KP; ++k) c += cd[k] > 0 ? 1u : 0u;
-        uint32_t total;
-        uint32_t pos = dev::block_exclusive_add32<kBlock>(c, q.scan32, total);
-        if (q.n + total > (uint32_t)kQueue) queue_flush(q, nxt, cnt_next);
-        pos += q.n;
-#pragma unroll
-        for (int k = 0; k < KP; ++k)
-            if (cd[k] > 0) {
-                q.v[pos] = cv[k];
-                q.rs[pos] = crs[k];
-                q.d[pos] = cd[k];
-                ++pos;
-            }
-        __syncthreads();  // every thread has read q.n
-        if (threadIdx.x == 0) q.n += total;
-        __syncthreads();
+        wave_enqueue<KP>(q, cv, crs, cd);
+        if (++pass == kPasses) {
+            pass = 0;
+            __syncthreads();
+            queue_flush(q, nxt, cnt_next);
+        }
     }
+    __syncthreads();
     if (q.n > 0) queue_flush(q, nxt, cnt_next);
 }
 
@@ -636,7 +786,7 @@ __device__ __forceinline__ void batch_sssp_pull(PullQueue &q, const int32_t *__r
 template <int W>
 __global__ __launch_bounds__(kBlock) void k_batch_sssp_bf(
     const int32_t *__restrict__ rowptr, const int32_t *__restrict__ col, int32_t nnz,
-    SsspBatchNearOp<W> op, FrontierBufs cur, const uint64_t *cnt_cur, FrontierBufs nxt,
+    SsspBatchNearOp<W, false> op, FrontierBufs cur, const uint64_t *cnt_cur, FrontierBufs nxt,
     uint64_t *cnt_next, uint64_t *cnt_clear, uint64_t *stats) {
     __shared__ BatchLds lds;
     const uint64_t cc = *cnt_cur;
@@ -654,12 +804,11 @@ __global__ __launch_bounds__(kBlock) void k_batch_sssp_bf(
                                                    cnt_next);
 }
 
-template <int W>
+template <int W, bool SM>
 __global__ __launch_bounds__(kBlock) void k_batch_sssp_nf(
     const int32_t *__restrict__ rowptr, const int32_t *__restrict__ col, int32_t nnz, int32_t m,
-    SsspBatchNearOp<W> op, FrontierBufs cur, FrontierBufs nxt, uint64_t *ctl,
+    SsspBatchNearOp<W, SM> op, FrontierBufs cur, FrontierBufs nxt, uint64_t *ctl,
     int32_t r, int32_t pull_div) {
-    constexpr int B = 32 * W;
     __shared__ BatchLds lds;
     __shared__ uint64_t s_part[kBlock / 64];
     __shared__ uint32_t s_min[kBlock / 64];
@@ -690,7 +839,7 @@ __global__ __launch_bounds__(kBlock) void k_batch_sssp_nf(
     }
     if (done) return;
     if (!split && pull_div > 0 && (int64_t)E * pull_div > (int64_t)nnz) {
-        batch_sssp_pull<W>(lds.pq, rowptr, col, m, op, tbits, nxt, ctl + (r + 1) % 3);
+        batch_sssp_pull<W, SM>(lds.pq, rowptr, col, m, op, tbits, nxt, ctl + (r + 1) % 3);
         return;
     }
     if (!split) {
@@ -703,10 +852,7 @@ __global__ __launch_bounds__(kBlock) void k_batch_sssp_nf(
     constexpr int VPB = kBlock / W;
     constexpr int KP = 4;
     PullQueue &q = lds.pq;
-    if (threadIdx.x == 0) {
-        q.n = 0;
-        q.nl = 0;
-    }
+    if (threadIdx.x == 0) q.n = 0;
     __syncthreads();
     const int g = threadIdx.x / W, w = threadIdx.x % W;
     const int lane = dev::lane_id();
@@ -729,10 +875,11 @@ __global__ __launch_bounds__(kBlock) void k_batch_sssp_nf(
                 uint32_t pb = op.pend[i];
                 if (pb) {
                     uint32_t keep = 0, x = pb;
+                    const int32_t *dv_row = op.word_of(v, w);
                     while (x) {
                         const int b = __ffs(x) - 1;
                         x &= x - 1;
-                        const int32_t d = op.dist[v * B + w * 32 + b];
+                        const int32_t d = dv_row[b * op.stride()];
                         if (d < tbits) continue;  // lowered below T since: expanded
                         if (d < tnext) {
                             moved |= 1u << b;
@@ -821,7 +968,7 @@ __global__ void k_batch_vis_init(int32_t m, int32_t nsrc, const int32_t *__restr
     }
 }
 
-// zero the frontier rows of the entries just expanded; advance the level
+// SSSP: zero the frontier rows of the entries just expanded; advance the level
 // (every round when `every`: near-far rounds number their claims by round,
 // split rounds included).  The rows are left alone when the next level pulls
 // (pull_div > 0 and its union frontier has more than nnz / pull_div edges):
@@ -841,13 +988,13 @@ __global__ void k_clear_rows(FrontierBufs cur, const uint64_t *cnt, uint32_t *fr
 // seed: source i -> bit i of its vertex; depth/dist 0 at the source
 template <int W>
 __global__ void k_batch_seed(const int32_t *srcs, int32_t nsrc, uint32_t *vis, uint32_t *front,
-                             int32_t *depth, int32_t m, int32_t *dist) {
+                             int32_t *depth, int32_t m, int32_t *dist, bool source_major) {
     for (int i = threadIdx.x; i < nsrc; i += blockDim.x) {
         const int32_t s = srcs[i];
         if (vis) atomicOr(vis + (int64_t)s * W + i / 32, 1u << (i % 32));
         atomicOr(front + (int64_t)s * W + i / 32, 1u << (i % 32));
         if (depth) depth[(int64_t)s * (32 * W) + i] = 0;
-        if (dist) dist[(int64_t)s * (32 * W) + i] = 0;
+        if (dist) dist[source_major ? (int64_t)i * m + s : (int64_t)s * (32 * W) + i] = 0;
     }
 }
 
@@ -880,8 +1027,10 @@ __global__ void k_batch_npull(uint64_t *npull, const int32_t *lvl) { npull[0] = 
 // with the depth written where they were discovered (vertex-major dep
 // [m][32W]), or unreached (-1).  With comp given, pairs of a vertex and a
 // source in different components were marked visited up front and are
-// unreached.  The snapshots are read kSnapRun at a time (independent loads
-// in flight).
+// unreached.  The snapshots are read kSnapRun at a time (independent loads in
+// flight); LDS holds 16-bit snapshot numbers (at most 4096), not depths, for
+// twice the blocks per CU (128 sources of the 2048^2 lattice, 72 snapshots:
+// 2.22 -> 1.62 ms, 4.3 TB/s).
 constexpr int kSnapRun = 16;
 template <int W>
 __global__ __launch_bounds__(256) void k_batch_depths(
@@ -889,13 +1038,13 @@ __global__ __launch_bounds__(256) void k_batch_depths(
     int32_t m, int32_t nsrc, const uint32_t *snap, int64_t stride, const uint64_t *npull,
     const int32_t *level_of, int32_t *out) {
     constexpr int B = 32 * W, T = 256 / W;
-    __shared__ int32_t d[T][B + 1];
+    __shared__ uint16_t d[T][B + 2];  // snapshot + 1, 0 = in none
     __shared__ int32_t s_comp[B];
     for (int i = threadIdx.x; i < B; i += 256) s_comp[i] = comp && i < nsrc ? comp[srcs[i]] : -1;
     const int64_t v0 = (int64_t)blockIdx.x * T;
     const int t = threadIdx.x / W, w = threadIdx.x % W;
     const int64_t v = v0 + t;
-    for (int b = 0; b < 32; ++b) d[t][w * 32 + b] = -2;
+    for (int b = 0; b < 32; ++b) d[t][w * 32 + b] = 0;
     const int32_t ns = (int32_t)npull[0];
     for (int32_t j0 = 0; j0 < ns; j0 += kSnapRun) {
         uint32_t bits[kSnapRun];
@@ -904,12 +1053,10 @@ __global__ __launch_bounds__(256) void k_batch_depths(
             bits[q] = (j0 + q < ns && v < m) ? snap[(int64_t)(j0 + q) * stride + v * W + w] : 0u;
 #pragma unroll
         for (int q = 0; q < kSnapRun; ++q) {
-            if (!bits[q]) continue;
-            const int32_t L = level_of[j0 + q];
             while (bits[q]) {
                 const int b = __ffs(bits[q]) - 1;
                 bits[q] &= bits[q] - 1;
-                d[t][w * 32 + b] = L;
+                d[t][w * 32 + b] = (uint16_t)(j0 + q + 1);
             }
         }
     }
@@ -918,9 +1065,11 @@ __global__ __launch_bounds__(256) void k_batch_depths(
         const int s = x / T, tt = x % T;
         const int64_t vv = v0 + tt;
         if (vv >= m) continue;
-        int32_t r = d[tt][s];
-        if (r == -2) {
-            r = -1;
+        const int32_t j = d[tt][s];
+        int32_t r = -1;
+        if (j > 0) {
+            r = level_of[j - 1];
+        } else {
             if ((vis[vv * W + s / 32] >> (s % 32)) & 1u)
                 if (!comp || comp[vv] == s_comp[s]) r = dep[vv * B + s];
         }
@@ -940,8 +1089,6 @@ void batch_pass(Ctx *c, const Graph *g, const int32_t *src_host, int32_t nsrc, i
     uint32_t *fa = (uint32_t *)scratch(c, "batch_fa", sizeof(uint32_t) * words);
     uint32_t *fb = (uint32_t *)scratch(c, "batch_fb", sizeof(uint32_t) * words);
     int32_t *stamp = (int32_t *)scratch(c, "batch_stamp", sizeof(int32_t) * m);
-    int32_t *dist = SSSP ? (int32_t *)scratch(c, "batch_dist", sizeof(int32_t) * m * (int64_t)B)
-                         : nullptr;
     int32_t *depth = SSSP ? nullptr
                           : (int32_t *)scratch(c, "batch_dep", sizeof(int32_t) * m * (int64_t)B);
     // snapshots of pulled BFS levels, within batch_snapshot_mb (and half the
@@ -962,6 +1109,10 @@ void batch_pass(Ctx *c, const Graph *g, const int32_t *src_host, int32_t nsrc, i
                              : nullptr;
         sn.level_of = (int32_t *)scratch(c, "batch_snap_lv", sizeof(int32_t) * 4096);
         sn.npull = fs.ctl + 12;
+        sn.src = fs.ctl + 9;
+        sn.pulled = fs.ctl + 14;
+        sn.build = fs.ctl + 11;
+        sn.claims = fs.ctl + 16;
     }
     int32_t *srcs = (int32_t *)scratch(c, "batch_srcs", sizeof(int32_t) * (B + 1));
     APSPIE_HIP(hipMemcpyAsync(srcs, src_host, sizeof(int32_t) * nsrc, hipMemcpyHostToDevice,
@@ -1013,10 +1164,16 @@ void batch_pass(Ctx *c, const Graph *g, const int32_t *src_host, int32_t nsrc, i
             ? (int32_t)std::min<int64_t>(opt(c, "batch_sssp_pull_div", 4) * (W <= 2 ? 2 : 1),
                                          1 << 22)
             : 0;
+    const bool source_major = sssp_pull_div > 0;
+    int32_t *dist = !SSSP          ? nullptr
+                    : source_major ? (int32_t *)dist_out
+                                   : (int32_t *)scratch(c, "batch_dist",
+                                                        sizeof(int32_t) * m * (int64_t)B);
     if (!SSSP) {
         k_batch_vis_init<W><<<grid, kBlock, 0, c->stream>>>(m, nsrc, comp, srcs, vis);
     } else {
-        fill_i32(c, dist, __builtin_bit_cast(int32_t, APSPIE_SSSP_INF), (int64_t)m * B);
+        fill_i32(c, dist, __builtin_bit_cast(int32_t, APSPIE_SSSP_INF),
+                 (int64_t)m * (source_major ? nsrc : B));
     }
     fill_i32(c, (int32_t *)fa, 0, words);
     fill_i32(c, (int32_t *)fb, 0, words);
@@ -1029,7 +1186,7 @@ void batch_pass(Ctx *c, const Graph *g, const int32_t *src_host, int32_t nsrc, i
         fill_i32(c, (int32_t *)(fs.ctl + 12), __builtin_bit_cast(int32_t, delta), 1);
         fill_i32(c, (int32_t *)(fs.ctl + 10), __builtin_bit_cast(int32_t, delta), 1);
     }
-    k_batch_seed<W><<<1, 256, 0, c->stream>>>(srcs, nsrc, vis, fa, depth, m, dist);
+    k_batch_seed<W><<<1, 256, 0, c->stream>>>(srcs, nsrc, vis, fa, depth, m, dist, source_major);
     k_build<kBlock, 1, kTile, true><<<1, kBlock, 0, c->stream>>>(
         SeedOp{}, g->rowptr, ulist, (int32_t)uniq.size(), nullptr, fs.f[0], fs.ctl + 0);
     APSPIE_LAUNCH_CHECK();
@@ -1038,15 +1195,20 @@ void batch_pass(Ctx *c, const Graph *g, const int32_t *src_host, int32_t nsrc, i
     auto level = [&](int l) {
         const int cur = l & 1;
         uint32_t *front = cur ? fb : fa, *next = cur ? fa : fb;
-        if (near_far)
-            k_batch_sssp_nf<W><<<grid, kBlock, 0, c->stream>>>(
+        if (near_far && source_major)
+            k_batch_sssp_nf<W, true><<<grid, kBlock, 0, c->stream>>>(
                 g->rowptr, g->col, (int32_t)g->nnz, m,
-                SsspBatchNearOp<W>{front, next, pend, stamp, dist, g->val, lvl, 0}, fs.f[cur],
-                fs.f[cur ^ 1], fs.ctl, l % 6, sssp_pull_div);
+                SsspBatchNearOp<W, true>{front, next, pend, stamp, dist, m, g->val, lvl, 0},
+                fs.f[cur], fs.f[cur ^ 1], fs.ctl, l % 6, sssp_pull_div);
+        else if (near_far)
+            k_batch_sssp_nf<W, false><<<grid, kBlock, 0, c->stream>>>(
+                g->rowptr, g->col, (int32_t)g->nnz, m,
+                SsspBatchNearOp<W, false>{front, next, pend, stamp, dist, m, g->val, lvl, 0},
+                fs.f[cur], fs.f[cur ^ 1], fs.ctl, l % 6, 0);
         else if (SSSP)
             k_batch_sssp_bf<W><<<grid, kBlock, 0, c->stream>>>(
                 g->rowptr, g->col, (int32_t)g->nnz,
-                SsspBatchNearOp<W>{front, next, nullptr, stamp, dist, g->val, lvl, 0}, fs.f[cur],
+                SsspBatchNearOp<W, false>{front, next, nullptr, stamp, dist, m, g->val, lvl, 0}, fs.f[cur],
                 fs.ctl + (l % 3), fs.f[cur ^ 1], fs.ctl + ((l + 1) % 3), fs.ctl + ((l + 2) % 3),
                 fs.ctl + 4);
         else {
@@ -1055,16 +1217,22 @@ void batch_pass(Ctx *c, const Graph *g, const int32_t *src_host, int32_t nsrc, i
                 g->rowptr, g->col, (int32_t)g->nnz, m, op, next, pull_div, fs.f[cur],
                 fs.ctl + (l % 3), fs.f[cur ^ 1], fs.ctl + ((l + 1) % 3), fs.ctl + ((l + 2) % 3),
                 fs.ctl + 4, sn);
-            if (pull_div > 0)  // six 256-thread blocks per CU fit its registers and LDS
-                k_batch_bfs_pull<W><<<fill_grid(c, kBlock, 6), kBlock, 0, c->stream>>>(
+            if (pull_div > 0) {  // eight 256-thread blocks per CU fit its registers and LDS
+                const auto pull = short_rows ? k_batch_bfs_pull<W, false> : k_batch_bfs_pull<W, true>;
+                pull<<<fill_grid(c, kBlock, 8), kBlock, 0, c->stream>>>(
                     g->rowptr, g->col, (int32_t)g->nnz, m, op, next, pull_div, fs.f[cur],
                     fs.ctl + (l % 3), fs.f[cur ^ 1], fs.ctl + ((l + 1) % 3),
                     fs.ctl + ((l + 2) % 3), fs.ctl + 4, sn);
+            }
         }
-        k_clear_rows<W><<<grid, kBlock, 0, c->stream>>>(fs.f[cur], fs.ctl + (l % 3), front, lvl,
-                                                        near_far, fs.ctl + ((l + 1) % 3),
-                                                        SSSP ? sssp_pull_div : pull_div,
-                                                        (int32_t)g->nnz);
+        if (SSSP)
+            k_clear_rows<W><<<grid, kBlock, 0, c->stream>>>(
+                fs.f[cur], fs.ctl + (l % 3), front, lvl, near_far, fs.ctl + ((l + 1) % 3),
+                sssp_pull_div, (int32_t)g->nnz);
+        else
+            k_bfs_between<W><<<grid, kBlock, 0, c->stream>>>(
+                g->rowptr, m, (int32_t)g->nnz, pull_div, fs.f[cur], fs.f[cur ^ 1],
+                fs.ctl + (l % 3), fs.ctl + ((l + 1) % 3), front, next, lvl, (l + 1) & 1, sn);
     };
 
     // chunks of K levels captured once and replayed: K is a multiple of 6 so
@@ -1115,7 +1283,9 @@ void batch_pass(Ctx *c, const Graph *g, const int32_t *src_host, int32_t nsrc, i
     c->stats.vertices_reached += (int64_t)h[5];
     c->stats.iterations = std::max(c->stats.iterations, (int32_t)h[6]);
     kt.collect();
-    if (SSSP) {
+    if (SSSP && source_major) {
+        // the distances are the result already
+    } else if (SSSP) {
         dim3 grd((unsigned)ceil_div(m, 32), (unsigned)ceil_div(nsrc, 32));
         k_transpose_dist<<<grd, 256, 0, c->stream>>>(dist, m, B, nsrc, dist_out);
     } else {

@@ -45,16 +45,19 @@ __global__ void k_pack(const int32_t *row, const int32_t *col, const float *val,
 // CSR entries as keys (column << rb) | row: each thread takes kPackRun
 // consecutive entries, finds the first one's row by binary search and walks on
 constexpr int kPackRun = 8;
+__device__ __forceinline__ int32_t entry_row(const int32_t *rowptr, int32_t m, int64_t e) {
+    int32_t r = 0, hi = m;  // largest r with rowptr[r] <= e
+    while (hi - r > 1) {
+        const int32_t mid = (int32_t)(((int64_t)r + hi) >> 1);
+        if (rowptr[mid] <= e) r = mid; else hi = mid;
+    }
+    return r;
+}
 __global__ void k_pack_transposed(const int32_t *rowptr, const int32_t *col, int32_t m,
                                   int64_t nnz, int rb, uint64_t *keys) {
     for (int64_t e0 = (blockIdx.x * (int64_t)blockDim.x + threadIdx.x) * kPackRun; e0 < nnz;
          e0 += (int64_t)gridDim.x * blockDim.x * kPackRun) {
-        int32_t r = 0, hi = m;  // largest r with rowptr[r] <= e0
-        while (hi - r > 1) {
-            const int32_t mid = (int32_t)(((int64_t)r + hi) >> 1);
-            if (rowptr[mid] <= e0) r = mid; else hi = mid;
-        }
-        int32_t end = rowptr[r + 1];
+        int32_t r = entry_row(rowptr, m, e0), end = rowptr[r + 1];
         for (int64_t e = e0; e < min(e0 + kPackRun, nnz); ++e) {
             while (end <= e) end = rowptr[++r + 1];
             keys[e] = ((uint64_t)(uint32_t)col[e] << rb) | (uint32_t)r;
@@ -329,6 +332,29 @@ __global__ void k_neq(const int32_t *a, const int32_t *b, int64_t n, int32_t *fl
         if (a[i] != b[i]) flag[0] = 1;
 }
 
+// Whether every entry of a symmetric CSR with sorted rows has its mirror
+// image's value: kPackRun consecutive entries per thread, the mirror image by
+// binary search in its row.
+__global__ void k_check_mirror_values(const int32_t *rowptr, const int32_t *col,
+                                      const float *val, int32_t m, int64_t nnz, int32_t *flag) {
+    for (int64_t e0 = (blockIdx.x * (int64_t)blockDim.x + threadIdx.x) * kPackRun; e0 < nnz;
+         e0 += (int64_t)gridDim.x * blockDim.x * kPackRun) {
+        int32_t r = entry_row(rowptr, m, e0), end = rowptr[r + 1];
+        for (int64_t e = e0; e < min(e0 + kPackRun, nnz); ++e) {
+            while (end <= e) end = rowptr[++r + 1];
+            const int32_t v = col[e];
+            int32_t lo = rowptr[v], hi = rowptr[v + 1];  // first entry of row v not below r
+            while (lo < hi) {
+                const int32_t mid = (lo + hi) >> 1;
+                if (col[mid] < r) lo = mid + 1; else hi = mid;
+            }
+            if (lo >= rowptr[v + 1] || col[lo] != r ||
+                __float_as_int(val[lo]) != __float_as_int(val[e]))
+                flag[0] = 1;
+        }
+    }
+}
+
 // Structure (and, for a weighted graph, values) compared with the transpose,
 // once per graph.  The transpose's rows come out sorted, so with equal
 // structure the values line up position by position.
@@ -355,6 +381,24 @@ static void check_symmetry(Ctx *c, Graph *g) {
     sync(c);
     g->symmetric = h[0] == 0 ? 1 : 0;
     g->sym_weights = (g->symmetric == 1 && g->val && h[1] == 0) ? 1 : 0;
+}
+
+// A graph built symmetrized is known to be symmetric (and its rows sorted),
+// but not in its values: an edge listed both ways round keeps each one's own.
+// Checked in place, with no scratch but a flag: the callers may have none left.
+static void check_mirror_values(Ctx *c, Graph *g) {
+    if (g->symmetric != 1 || g->sym_weights >= 0) return;
+    int32_t *flag = (int32_t *)scratch(c, "sym_flag", 256);
+    fill_i32(c, flag, 0, 1);
+    if (g->val && g->nnz > 0) {
+        k_check_mirror_values<<<fill_grid(c, kBlock, 8), kBlock, 0, c->stream>>>(
+            g->rowptr, g->col, g->val, g->m, g->nnz, flag);
+        APSPIE_LAUNCH_CHECK();
+    }
+    int32_t h = 1;
+    APSPIE_HIP(hipMemcpyAsync(&h, flag, 4, hipMemcpyDeviceToHost, c->stream));
+    sync(c);
+    g->sym_weights = g->val && h == 0 ? 1 : 0;
 }
 
 __global__ void k_iso_bits(const int32_t *rowptr, int32_t m, uint32_t *bits) {
@@ -629,6 +673,7 @@ bool graph_is_symmetric(Ctx *c, Graph *g) {
 bool graph_is_symmetric_weighted(Ctx *c, Graph *g) {
     std::lock_guard<std::mutex> lock(g->derived_mu);
     check_symmetry(c, g);
+    check_mirror_values(c, g);
     return g->sym_weights == 1;
 }
 
