@@ -26,6 +26,16 @@ __device__ __forceinline__ void wave_sync() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// Inclusive scan (+) of each row of 16 lanes.
+__device__ __forceinline__ uint32_t row16_inclusive_add(uint32_t x) {
+    uint32_t t;
+    t = __builtin_amdgcn_update_dpp(0u, x, 0x111, 0xf, 0xf, false); x += t;
+    t = __builtin_amdgcn_update_dpp(0u, x, 0x112, 0xf, 0xf, false); x += t;
+    t = __builtin_amdgcn_update_dpp(0u, x, 0x114, 0xf, 0xf, false); x += t;
+    t = __builtin_amdgcn_update_dpp(0u, x, 0x118, 0xf, 0xf, false); x += t;
+    return x;
+}
+
 // Inclusive wave-wide scan (+) of 32-bit values.  Uses the DPP row shifts
 // within each 16-lane row and row broadcasts across rows, the CDNA idiom.
 __device__ __forceinline__ uint32_t wave_inclusive_add(uint32_t x) {
