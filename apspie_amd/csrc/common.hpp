@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <deque>
 #include <cstdio>
 #include <cstring>
 #include <map>
@@ -121,6 +122,13 @@ struct Ctx {
     // and generated on the host
     Buffer mis_prio;
     int32_t mis_prio_m = -1;
+    // arrays of destroyed graphs, kept for the next ones (graph_alloc): oldest
+    // first, at most kSpareBytes, not counted as used but given back before
+    // the budget or the device runs short
+    std::mutex spare_mu;
+    std::deque<Buffer> spares;
+    size_t spare_bytes = 0;
+    std::map<void *, size_t> spare_sizes;  // handed out again: bytes of the block
     // graphs whose memory is accounted to this context
     std::set<Graph *> graphs;
     // event pairs of the kernel timer (option "profiling"), reused by calls
@@ -136,6 +144,13 @@ void *scratch(Ctx *c, const std::string &name, size_t bytes);
 int64_t scratch_room(Ctx *c);
 void *dev_alloc(Ctx *c, size_t bytes);  // counted against the budget
 void dev_free(Ctx *c, void *p, size_t bytes);
+// hipMalloc that gives the context's spare blocks back before it fails.
+hipError_t device_malloc(Ctx *c, void **p, size_t bytes);
+// A graph's arrays: counted as dev_alloc's are, from the spare blocks where one
+// fits.  graph_free is for a device with no pending work on the block.
+void *graph_alloc(Ctx *c, size_t bytes);
+void graph_free(Ctx *c, void *p, size_t bytes);
+void drop_spares(Ctx *c);
 
 // Run `f` translating exceptions into status codes and recording the message.
 template <class F>

@@ -40,8 +40,10 @@ static const char *kOptionNames[] = {
     "tc_medium_row",     // TC: rows with |L_r| up to this go to the 256-thread LDS tier, longer
                          // ones to the 1024-thread tier (128..2048; 512 measured best or within
                          // 4 % on R-MAT-18/20/22: 1.2-1.6x faster than 2048)
-    "spgemm_wave_ub",    // SpGEMM: rows with at most this many products to the wave tier (<= 256)
-    "spgemm_block_ub",   // SpGEMM: up to this to the block LDS tier (<= 4096)
+    "spgemm_wave_ub",    // SpGEMM: rows with at most this many products to the wave tier (<= 256; with the
+                         // dense accumulator and up to 16384 columns, at most 64 of them)
+    "spgemm_block_ub",   // SpGEMM: up to this to the block LDS tier (<= 4096) where B has more than
+                         // 16384 columns or the dense accumulator is off
     "spgemm_dense",      // SpGEMM: longer rows to the dense accumulator when B has <= 32768
                          // columns (1) or always to global tables (0)
     "profiling",         // 1 = time the dominant kernel with hipEvents
@@ -99,13 +101,13 @@ void sync(Ctx *c) { APSPIE_HIP(hipStreamSynchronize(c->stream)); }
 
 void *dev_alloc(Ctx *c, size_t bytes) {
     if (bytes == 0) bytes = 256;
+    if (c->budget > 0 && c->used + (int64_t)(c->spare_bytes + bytes) > c->budget) drop_spares(c);
     if (c->budget > 0 && c->used + (int64_t)bytes > c->budget)
         throw Error{APSPIE_ERR_BUDGET, "HBM budget exceeded: need " + std::to_string(bytes) +
                                            " more bytes, " + std::to_string(c->budget - c->used) +
                                            " left"};
     void *p = nullptr;
-    hipError_t e = hipMalloc(&p, bytes);
-    if (e != hipSuccess) {
+    if (device_malloc(c, &p, bytes) != hipSuccess) {
         (void)hipGetLastError();
         throw Error{APSPIE_ERR_OOM, "hipMalloc(" + std::to_string(bytes) + ") failed"};
     }
@@ -118,6 +120,84 @@ void dev_free(Ctx *c, void *p, size_t bytes) {
     (void)hipFree(p);
     if (bytes == 0) bytes = 256;
     c->used -= (int64_t)bytes;
+}
+
+hipError_t device_malloc(Ctx *c, void **p, size_t bytes) {
+    hipError_t e = hipMalloc(p, bytes);
+    if (e != hipSuccess && c->spare_bytes) {
+        (void)hipGetLastError();
+        drop_spares(c);
+        e = hipMalloc(p, bytes);
+    }
+    return e;
+}
+
+// Freeing the 320 MB of an R-MAT-14 square took 0.48 ms, and 8 ms once a loop of
+// products had freed some 100 GB (the freed memory has to be cleared before it
+// can be given out); a block kept costs neither.  Blocks below 1 MB are not
+// worth keeping, and one is not given to a request below 8/9 of its size.
+constexpr size_t kSpareMin = (size_t)1 << 20, kSpareBytes = (size_t)512 << 20;
+
+void drop_spares(Ctx *c) {
+    std::lock_guard<std::mutex> lock(c->spare_mu);
+    for (const Buffer &b : c->spares) (void)hipFree(b.ptr);
+    c->spares.clear();
+    c->spare_bytes = 0;
+}
+
+void *graph_alloc(Ctx *c, size_t bytes) {
+    if (bytes >= kSpareMin) {
+        std::lock_guard<std::mutex> lock(c->spare_mu);
+        auto best = c->spares.end();
+        for (auto it = c->spares.begin(); it != c->spares.end(); ++it)
+            if (it->bytes >= bytes && it->bytes <= bytes + bytes / 8 &&
+                (best == c->spares.end() || it->bytes < best->bytes))
+                best = it;
+        if (best != c->spares.end() &&
+            (c->budget == 0 || c->used + (int64_t)best->bytes <= c->budget)) {
+            const Buffer b = *best;
+            c->spare_sizes[b.ptr] = b.bytes;
+            c->spares.erase(best);
+            c->spare_bytes -= b.bytes;
+            c->used += (int64_t)b.bytes;
+            return b.ptr;
+        }
+    }
+    return dev_alloc(c, bytes);
+}
+
+void graph_free(Ctx *c, void *p, size_t bytes) {
+    if (!p) return;
+    {
+        std::lock_guard<std::mutex> lock(c->spare_mu);
+        const auto it = c->spare_sizes.find(p);
+        if (it != c->spare_sizes.end()) {
+            bytes = it->second;
+            c->spare_sizes.erase(it);
+        }
+        if (bytes >= kSpareMin && bytes <= kSpareBytes) {
+            while (c->spare_bytes + bytes > kSpareBytes) {
+                (void)hipFree(c->spares.front().ptr);
+                c->spare_bytes -= c->spares.front().bytes;
+                c->spares.pop_front();
+            }
+            Buffer b;
+            b.ptr = p;
+            b.bytes = bytes;
+            bool kept = true;  // no exception leaves a destroy
+            try {
+                c->spares.push_back(b);
+            } catch (...) {
+                kept = false;
+            }
+            if (kept) {
+                c->spare_bytes += bytes;
+                c->used -= (int64_t)bytes;
+                return;
+            }
+        }
+    }
+    dev_free(c, p, bytes);
 }
 
 namespace {
@@ -336,6 +416,7 @@ int apspie_ctx_destroy(apspie_ctx *c) {
     else
         for (auto &kv : c->scratch)
             if (kv.second.ptr) (void)hipFree(kv.second.ptr);
+    drop_spares(c);
     for (auto &p : c->timer_events) {
         (void)hipEventDestroy(p.first);
         (void)hipEventDestroy(p.second);
@@ -362,6 +443,8 @@ void *apspie_ctx_stream(apspie_ctx *c) { return c ? (void *)c->stream : nullptr;
 
 int apspie_ctx_set_hbm_budget(apspie_ctx *c, int64_t bytes) {
     if (!c || bytes < 0) return APSPIE_ERR_INVALID;
+    (void)hipSetDevice(c->device);
+    if (bytes > 0 && c->used + (int64_t)c->spare_bytes > bytes) drop_spares(c);
     c->budget = bytes;
     return APSPIE_OK;
 }
@@ -409,6 +492,7 @@ int apspie_ctx_trim(apspie_ctx *c) {
         set_device(c);
         sync(c);
         drop_scratch(c);
+        drop_spares(c);
     });
 }
 
@@ -500,9 +584,9 @@ int apspie_graph_upload(apspie_ctx *c, const apspie_csr *h, apspie_graph **out) 
         const bool has_val = h->val != nullptr;  // a weighted graph, even if edgeless
         size_t rb = sizeof(int32_t) * (h->m + 1), cb = sizeof(int32_t) * h->nnz,
                vb = has_val ? sizeof(float) * h->nnz : 0;
-        g->rowptr = (int32_t *)dev_alloc(c, rb);
-        g->col = (int32_t *)dev_alloc(c, cb);
-        if (has_val) g->val = (float *)dev_alloc(c, vb);
+        g->rowptr = (int32_t *)graph_alloc(c, rb);
+        g->col = (int32_t *)graph_alloc(c, cb);
+        if (has_val) g->val = (float *)graph_alloc(c, vb);
         g->bytes = (int64_t)(std::max<size_t>(rb, 256) + std::max<size_t>(cb, 256) +
                              (has_val ? std::max<size_t>(vb, 256) : 0));
         copy_to_device(c, g->rowptr, h->rowptr, rb, APSPIE_MEM_HOST);
@@ -511,9 +595,10 @@ int apspie_graph_upload(apspie_ctx *c, const apspie_csr *h, apspie_graph **out) 
         sync(c);
     });
     if (st != APSPIE_OK) {
-        if (g->rowptr) dev_free(c, g->rowptr, sizeof(int32_t) * (h->m + 1));
-        if (g->col) dev_free(c, g->col, sizeof(int32_t) * h->nnz);
-        if (g->val) dev_free(c, g->val, sizeof(float) * h->nnz);
+        (void)hipDeviceSynchronize();
+        graph_free(c, g->rowptr, sizeof(int32_t) * (h->m + 1));
+        graph_free(c, g->col, sizeof(int32_t) * h->nnz);
+        graph_free(c, g->val, sizeof(float) * h->nnz);
         delete g;
         return st;
     }
@@ -588,14 +673,16 @@ int apspie_graph_destroy(apspie_graph *g) {
     Ctx *c = g->owner;
     (void)hipSetDevice(g->device);
     if (c) {
-        (void)hipStreamSynchronize(c->stream);
+        // every stream, as hipFree waits: another context or the caller's own
+        // stream may still read the arrays, and they are given out again
+        (void)hipDeviceSynchronize();
         c->graphs.erase(g);
     }
     if (g->owns) {
         if (c) {
-            dev_free(c, g->rowptr, sizeof(int32_t) * (g->m + 1));
-            dev_free(c, g->col, sizeof(int32_t) * g->nnz);
-            if (g->val) dev_free(c, g->val, sizeof(float) * g->nnz);
+            graph_free(c, g->rowptr, sizeof(int32_t) * (g->m + 1));
+            graph_free(c, g->col, sizeof(int32_t) * g->nnz);
+            graph_free(c, g->val, sizeof(float) * g->nnz);
         } else {
             (void)hipFree(g->rowptr);
             (void)hipFree(g->col);

@@ -318,9 +318,9 @@ void graph_from_coo_dev(Ctx *c, Graph *g, const int32_t *row, const int32_t *col
     APSPIE_CHECK(h[1] == 0, APSPIE_ERR_INVALID, "COO index out of range");
     const int64_t k = symmetrize ? h[0] : E;
     g->nnz = k;
-    g->rowptr = (int32_t *)dev_alloc(c, sizeof(int32_t) * (g->m + 1));
-    g->col = (int32_t *)dev_alloc(c, sizeof(int32_t) * std::max<int64_t>(k, 1));
-    g->val = (float *)dev_alloc(c, sizeof(float) * std::max<int64_t>(k, 1));
+    g->rowptr = (int32_t *)graph_alloc(c, sizeof(int32_t) * (g->m + 1));
+    g->col = (int32_t *)graph_alloc(c, sizeof(int32_t) * std::max<int64_t>(k, 1));
+    g->val = (float *)graph_alloc(c, sizeof(float) * std::max<int64_t>(k, 1));
     g->bytes = (int64_t)(sizeof(int32_t) * (g->m + 1) + 8 * std::max<int64_t>(k, 1));
     if (symmetrize) emit_csr<true>(c, g, ka, va, E, cb, offsets);
     else emit_csr<false>(c, g, ka, va, E, cb, nullptr);
@@ -518,7 +518,7 @@ const uint32_t *graph_iso_bits(Ctx *c, Graph *g) {
     const int64_t words = ((int64_t)g->m + 31) / 32;
     uint32_t *bits = nullptr;
     // owned by the graph (freed with it), like its other derived arrays
-    APSPIE_HIP(hipMalloc(&bits, sizeof(uint32_t) * std::max<int64_t>(words, 1)));
+    APSPIE_HIP(device_malloc(c, (void **)&bits, sizeof(uint32_t) * std::max<int64_t>(words, 1)));
     if (words > 0) {
         k_iso_bits<<<(int)std::min<int64_t>(ceil_div(words, kBlock), 4 * c->cus), kBlock, 0,
                      c->stream>>>(g->rowptr, g->m, bits);
@@ -639,7 +639,7 @@ const int32_t *graph_components(Ctx *c, Graph *g) {
     if (g->comp) return g->comp;
     int32_t *label = nullptr;
     // owned by the graph (freed with it), like its other derived arrays
-    APSPIE_HIP(hipMalloc(&label, sizeof(int32_t) * std::max<int64_t>(g->m, 1)));
+    APSPIE_HIP(device_malloc(c, (void **)&label, sizeof(int32_t) * std::max<int64_t>(g->m, 1)));
     components_into(c, g, label);
     sync(c);
     g->comp = label;
@@ -713,9 +713,9 @@ void graph_transpose_dev(Ctx *c, const Graph *g, Graph *t, const char *in_scratc
         t->col = (int32_t *)scratch(c, p + "_col", sizeof(int32_t) * Ea);
         t->val = g->val ? (float *)scratch(c, p + "_val", sizeof(float) * Ea) : nullptr;
     } else {
-        t->rowptr = (int32_t *)dev_alloc(c, sizeof(int32_t) * (t->m + 1));
-        t->col = (int32_t *)dev_alloc(c, sizeof(int32_t) * Ea);
-        t->val = g->val ? (float *)dev_alloc(c, sizeof(float) * Ea) : nullptr;
+        t->rowptr = (int32_t *)graph_alloc(c, sizeof(int32_t) * (t->m + 1));
+        t->col = (int32_t *)graph_alloc(c, sizeof(int32_t) * Ea);
+        t->val = g->val ? (float *)graph_alloc(c, sizeof(float) * Ea) : nullptr;
     }
     t->bytes = (int64_t)(sizeof(int32_t) * (t->m + 1) + (g->val ? 8 : 4) * Ea);
     emit_csr<false>(c, t, ka, va, E, rb, nullptr);

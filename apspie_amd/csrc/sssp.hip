@@ -315,7 +315,7 @@ void graph_prepare_heavy(Ctx *c, Graph *g) {
     const int64_t ent = g->nnz / (kLight + 1) + 2, tiles = g->nnz / kHvTile + 2;
     const size_t bytes = sizeof(int32_t) * (3 * ent + tiles) + 64;
     // owned by the graph (freed with it), like its other derived arrays
-    APSPIE_HIP(hipMalloc(&g->heavy_mem, bytes));
+    APSPIE_HIP(device_malloc(c, (void **)&g->heavy_mem, bytes));
     int32_t *p = (int32_t *)g->heavy_mem;
     g->heavy_v = p;
     g->heavy_start = p + ent;
@@ -774,7 +774,7 @@ Graph::LightFirst graph_light_first(Ctx *c, Graph *g, float delta) {
     const size_t bytes = 2 * ecol + sizeof(int32_t) * ((size_t)g->m + 1);
     void *mem = nullptr;
     // owned by the graph (freed with it), like its other derived arrays
-    APSPIE_HIP(hipMalloc(&mem, bytes));
+    APSPIE_HIP(device_malloc(c, (void **)&mem, bytes));
     int32_t *lcol = (int32_t *)mem;
     float *lval = (float *)((char *)mem + ecol);
     int32_t *lend = (int32_t *)((char *)mem + 2 * ecol);

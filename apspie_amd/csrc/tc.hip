@@ -684,7 +684,7 @@ void graph_prepare_tc(Ctx *c, Graph *g) {
         APSPIE_CHECK(flag == 0, APSPIE_ERR_INVALID, "TC needs sorted, duplicate-free rows");
         // owned by the graph (freed with it), not charged to this context
         int32_t *lc = nullptr;
-        APSPIE_HIP(hipMalloc(&lc, sizeof(int32_t) * std::max(m, 1)));
+        APSPIE_HIP(device_malloc(c, (void **)&lc, sizeof(int32_t) * std::max(m, 1)));
         k_lowcnt<<<grid, kBlock, 0, c->stream>>>(g->rowptr, g->col, m, lc);
         APSPIE_LAUNCH_CHECK();
         sync(c);

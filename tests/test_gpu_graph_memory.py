@@ -1,0 +1,68 @@
+"""Arrays of destroyed graphs are kept for the next ones: the accounting, the
+budget and the results are those of arrays freed at once."""
+import numpy as np
+import pytest
+
+import apspie_amd as A
+
+pytestmark = pytest.mark.gpu
+
+
+def _csr(m, k, seed):
+    rng = np.random.default_rng(seed)
+    col = np.sort(rng.integers(0, m, (m, k)), axis=1).astype(np.int32).reshape(-1)
+    return (np.arange(m + 1) * k).astype(np.int32), col, rng.random(m * k, dtype=np.float32)
+
+
+def _check(g, csr):
+    rp, col, val = g.download(values=True)
+    assert np.array_equal(rp, csr[0]) and np.array_equal(col, csr[1])
+    assert np.array_equal(val, csr[2])
+
+
+def test_reuse_keeps_contents_and_accounting():
+    with A.Context(0) as c:
+        base = c.hbm_used()
+        for i, (m, k) in enumerate([(100_000, 8), (100_000, 8), (100_000, 7), (90_000, 8),
+                                    (1000, 4), (100_000, 9), (262_144, 1), (100_000, 8)]):
+            csr = _csr(m, k, i)
+            a, b = c.upload(*csr), c.upload(*csr)
+            _check(a, csr)
+            a.close()
+            other = _csr(m, k, 100 + i)
+            a = c.upload(*other)  # on the blocks of the first
+            _check(a, other)
+            _check(b, csr)
+            a.close()
+            b.close()
+            assert c.hbm_used() == base
+        c.trim()
+        assert c.hbm_used() == base
+
+
+def test_budget_and_other_contexts():
+    csr = _csr(200_000, 16, 1)  # 26 MB
+    small = _csr(150_000, 2, 2)
+    with A.Context(0) as c, A.Context(0) as other:
+        g = c.upload(*csr)
+        size = c.hbm_used()
+        g.close()
+        c.set_hbm_budget(size + 1000)  # kept blocks do not count against a new graph
+        s = c.upload(*small)
+        _check(s, small)
+        with pytest.raises(A.ApspieError):
+            c.upload(*csr)
+        s.close()
+        g = c.upload(*csr)
+        h = other.upload(*csr)
+        _check(g, csr)
+        g.close()
+        _check(h, csr)
+        h.close()
+    g = None
+    with A.Context(0) as c:
+        keep = c.upload(*csr)
+        c.upload(*csr).close()
+        g = c.upload(*csr)  # outlives its context, on a block given out twice
+        keep.close()
+    g.close()
