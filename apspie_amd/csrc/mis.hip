@@ -160,6 +160,124 @@ struct UndecidedOp {
     __device__ __forceinline__ bool keep(int32_t v) const { return state[v] == -1; }
 };
 
+// The last rounds in one block: a round of the whole grid is four launches,
+// 18-20 us however few candidates are left, and R-MAT and lattice graphs end
+// in two to four rounds of at most some thousand (R-MAT-20: 646786, 379269,
+// 67914, 7977, 592, 18 candidates).  Up to kTailRows candidates with kTailEdges
+// entries are finished here, 40-44 us for the last two or three rounds: their
+// rows are read into LDS once, and a round is two passes over the entries (who
+// loses, who leaves), each a single dependent read per entry with all of a
+// thread's reads in flight (8 lanes a row and their chains of reads: 51 us at
+// R-MAT-20).  More candidates are left to the grid.  Each round decides at
+// least the one with the largest key.  A call: 5,000 vertices 194 -> 94 us,
+// 15,543 vertices 160 -> 115, R-MAT-20 355 -> 345.
+constexpr int kTail = 1024, kTailRows = 2048, kTailEdges = 16384;
+
+__global__ __launch_bounds__(kTail) void k_mis_tail(const int32_t *__restrict__ rowptr,
+                                                    const int32_t *__restrict__ col,
+                                                    uint64_t *live, int32_t *state,
+                                                    FrontierBufs cur, uint64_t *cnt_cur,
+                                                    uint64_t *stats) {
+    constexpr int PER = kTailRows / kTail;
+    __shared__ int32_t s_u[kTailRows], s_rs[kTailRows], s_off[kTailRows + 1];
+    __shared__ uint64_t s_key[kTailRows];
+    __shared__ int32_t s_col[kTailEdges];
+    __shared__ uint16_t s_own[kTailEdges];
+    __shared__ uint8_t s_open[kTailRows], s_lost[kTailRows], s_won[kTailRows];
+    __shared__ uint64_t s_scan[kTail / 64];
+    __shared__ uint32_t s_n, s_edges;
+    const uint64_t cc = *cnt_cur;
+    const uint32_t F0 = cnt_entries(cc), E0 = cnt_edges(cc);
+    if (F0 == 0 || F0 > (uint32_t)kTailRows || E0 > (uint32_t)kTailEdges) return;
+    // candidate 2 t and 2 t + 1 of thread t: where their entries start
+    uint32_t deg[PER], mine = 0;
+#pragma unroll
+    for (int k = 0; k < PER; ++k) {
+        const uint32_t i = threadIdx.x * PER + k;
+        deg[k] = 0;
+        if (i < F0) {
+            const int32_t u = cur.v[i], rs = cur.start[i];
+            deg[k] = (uint32_t)(rowptr[u + 1] - rs);
+            s_u[i] = u;
+            s_rs[i] = rs;
+            s_key[i] = live[u];
+            s_open[i] = 1;
+            s_won[i] = 0;
+        }
+        mine += deg[k];
+    }
+    dev::Pair32 tot;
+    uint32_t off = dev::block_exclusive_add_pair<kTail>(mine, 0u, s_scan, tot).a;
+#pragma unroll
+    for (int k = 0; k < PER; ++k) {
+        s_off[threadIdx.x * PER + k] = (int32_t)off;
+        off += deg[k];
+    }
+    if (tot.a > (uint32_t)kTailEdges) return;  // (the counter says the same)
+    const int32_t entries = (int32_t)tot.a;
+    __syncthreads();
+#pragma unroll 4
+    for (int32_t e = threadIdx.x; e < entries; e += kTail) {
+        const int i = dev::upper_bound_m1(s_off, 0, (int)F0, e);
+        s_own[e] = (uint16_t)i;
+        s_col[e] = col[s_rs[i] + (e - s_off[i])];
+    }
+    uint64_t edges = 0, rows = 0, rounds = 0;
+    for (uint32_t F = F0, E = E0; F > 0;) {
+        edges += E;
+        rows += F;
+        rounds += 1;
+        for (uint32_t i = threadIdx.x; i < F0; i += kTail) s_lost[i] = 0;
+        __syncthreads();  // also: F and E are read, the entries are written
+        if (threadIdx.x == 0) s_n = s_edges = 0;
+#pragma unroll 4
+        for (int32_t e = threadIdx.x; e < entries; e += kTail) {
+            const int i = s_own[e];
+            if (s_open[i] && live[s_col[e]] > s_key[i]) s_lost[i] = 1;
+        }
+        __syncthreads();
+        // all winners join before any neighbour leaves: a row of a graph that is
+        // not symmetric may name another winner
+        for (uint32_t i = threadIdx.x; i < F0; i += kTail)
+            if (s_open[i] && !s_lost[i]) {
+                s_won[i] = 1;
+                s_open[i] = 0;
+                state[s_u[i]] = 1;
+                live[s_u[i]] = 0;
+            }
+        __syncthreads();
+#pragma unroll 4
+        for (int32_t e = threadIdx.x; e < entries; e += kTail) {
+            const int32_t v = s_col[e];
+            if (s_won[s_own[e]] && live[v] != 0) {
+                state[v] = 0;
+                live[v] = 0;
+            }
+        }
+        __syncthreads();
+        for (uint32_t i = threadIdx.x; i < F0; i += kTail) {
+            s_won[i] = 0;
+            if (!s_open[i]) continue;
+            if (live[s_u[i]] == 0) {
+                s_open[i] = 0;
+            } else {
+                const int32_t end = i + 1 < F0 ? s_off[i + 1] : entries;
+                atomicAdd(&s_n, 1u);
+                atomicAdd(&s_edges, (uint32_t)(end - s_off[i]));
+            }
+        }
+        __syncthreads();
+        F = s_n;
+        E = s_edges;
+    }
+    if (threadIdx.x == 0) {
+        stats[0] += edges;
+        stats[1] += rows;
+        stats[2] += rounds;
+        *cnt_cur = 0;
+    }
+}
+
 __global__ void k_mis_init(const int32_t *rowptr, const uint32_t *prio, int32_t m,
                            int32_t *state, uint64_t *live, int32_t *lose, uint64_t *ctl) {
     for (int64_t v = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; v < m;
@@ -192,8 +310,12 @@ void mis_run(Ctx *c, const Graph *g, const uint32_t *prio, int32_t *state) {
     APSPIE_LAUNCH_CHECK();
     KernelTimer kt(c);
     int round = 0;
-    int chunk = 8;  // rounds between host checks: R-MAT graphs finish in 6-7
-    int grow = 4;   // then 4, 8, 16, ... (an idle round still costs four launches)
+    // rounds of the whole grid before the tail is tried and the host looks: what
+    // R-MAT and lattice graphs of the size take to come down to kTailRows
+    // candidates (one too many costs four empty launches, one too few a round
+    // trip); then 2, 4, 8, ...
+    int chunk = g->m <= (1 << 15) ? 2 : g->m <= (1 << 18) ? 3 : 4;
+    int grow = 2;
     for (;;) {
         for (int k = 0; k < chunk; ++k, ++round) {
             const int cur = round & 1;
@@ -224,6 +346,9 @@ void mis_run(Ctx *c, const Graph *g, const uint32_t *prio, int32_t *state) {
                 UndecidedOp{state}, g->rowptr, fs.f[cur].v, 0, cnt, fs.f[cur ^ 1], nxt);
             APSPIE_LAUNCH_CHECK();
         }
+        k_mis_tail<<<1, kTail, 0, c->stream>>>(g->rowptr, g->col, live, state, fs.f[round & 1],
+                                               fs.ctl + (round % 3), fs.ctl + 4);
+        APSPIE_LAUNCH_CHECK();
         uint64_t *h = (uint64_t *)c->pinned;
         APSPIE_HIP(hipMemcpyAsync(h, fs.ctl + (round % 3), sizeof(uint64_t), hipMemcpyDeviceToHost,
                                   c->stream));
