@@ -147,9 +147,10 @@ void dev_free(Ctx *c, void *p, size_t bytes);
 // hipMalloc that gives the context's spare blocks back before it fails.
 hipError_t device_malloc(Ctx *c, void **p, size_t bytes);
 // A graph's arrays: counted as dev_alloc's are, from the spare blocks where one
-// fits.  graph_free is for a device with no pending work on the block.
+// fits.  A block is kept only where device_idle() has waited for every stream.
 void *graph_alloc(Ctx *c, size_t bytes);
-void graph_free(Ctx *c, void *p, size_t bytes);
+bool device_idle();
+void graph_free(Ctx *c, void *p, size_t bytes, bool keep);
 void drop_spares(Ctx *c);
 
 // Run `f` translating exceptions into status codes and recording the message.

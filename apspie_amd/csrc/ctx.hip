@@ -138,6 +138,12 @@ hipError_t device_malloc(Ctx *c, void **p, size_t bytes) {
 // worth keeping, and one is not given to a request below 8/9 of its size.
 constexpr size_t kSpareMin = (size_t)1 << 20, kSpareBytes = (size_t)512 << 20;
 
+bool device_idle() {
+    if (hipDeviceSynchronize() == hipSuccess) return true;
+    (void)hipGetLastError();  // refused, as during another thread's capture
+    return false;
+}
+
 void drop_spares(Ctx *c) {
     std::lock_guard<std::mutex> lock(c->spare_mu);
     for (const Buffer &b : c->spares) (void)hipFree(b.ptr);
@@ -166,7 +172,7 @@ void *graph_alloc(Ctx *c, size_t bytes) {
     return dev_alloc(c, bytes);
 }
 
-void graph_free(Ctx *c, void *p, size_t bytes) {
+void graph_free(Ctx *c, void *p, size_t bytes, bool keep) {
     if (!p) return;
     {
         std::lock_guard<std::mutex> lock(c->spare_mu);
@@ -175,7 +181,7 @@ void graph_free(Ctx *c, void *p, size_t bytes) {
             bytes = it->second;
             c->spare_sizes.erase(it);
         }
-        if (bytes >= kSpareMin && bytes <= kSpareBytes) {
+        if (keep && bytes >= kSpareMin && bytes <= kSpareBytes) {
             while (c->spare_bytes + bytes > kSpareBytes) {
                 (void)hipFree(c->spares.front().ptr);
                 c->spare_bytes -= c->spares.front().bytes;
@@ -595,10 +601,10 @@ int apspie_graph_upload(apspie_ctx *c, const apspie_csr *h, apspie_graph **out) 
         sync(c);
     });
     if (st != APSPIE_OK) {
-        (void)hipDeviceSynchronize();
-        graph_free(c, g->rowptr, sizeof(int32_t) * (h->m + 1));
-        graph_free(c, g->col, sizeof(int32_t) * h->nnz);
-        graph_free(c, g->val, sizeof(float) * h->nnz);
+        const bool idle = device_idle();
+        graph_free(c, g->rowptr, sizeof(int32_t) * (h->m + 1), idle);
+        graph_free(c, g->col, sizeof(int32_t) * h->nnz, idle);
+        graph_free(c, g->val, sizeof(float) * h->nnz, idle);
         delete g;
         return st;
     }
@@ -673,16 +679,17 @@ int apspie_graph_destroy(apspie_graph *g) {
     Ctx *c = g->owner;
     (void)hipSetDevice(g->device);
     if (c) {
-        // every stream, as hipFree waits: another context or the caller's own
-        // stream may still read the arrays, and they are given out again
-        (void)hipDeviceSynchronize();
+        (void)hipStreamSynchronize(c->stream);
         c->graphs.erase(g);
     }
     if (g->owns) {
         if (c) {
-            graph_free(c, g->rowptr, sizeof(int32_t) * (g->m + 1));
-            graph_free(c, g->col, sizeof(int32_t) * g->nnz);
-            graph_free(c, g->val, sizeof(float) * g->nnz);
+            // every stream, as hipFree waits: another context or the caller's own
+            // stream may still read the arrays, and they are given out again
+            const bool idle = device_idle();
+            graph_free(c, g->rowptr, sizeof(int32_t) * (g->m + 1), idle);
+            graph_free(c, g->col, sizeof(int32_t) * g->nnz, idle);
+            graph_free(c, g->val, sizeof(float) * g->nnz, idle);
         } else {
             (void)hipFree(g->rowptr);
             (void)hipFree(g->col);

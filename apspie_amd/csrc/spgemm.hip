@@ -54,49 +54,42 @@ enum { kCtlBin = 0, kCtlMaxU = 4, kCtlTiny = 5, kCtlTicket = 6 };
 constexpr int32_t kEmpty = 0x7fffffff;  // sorts after every column id
 
 // p[i] = products of row i.  16 lanes per row: a wave per row left 60 of its
-// lanes idle on rows of four entries.  Rows of more than kBoundRow entries go
-// to an LDS list and take a wave each, with several loads in flight (R-MAT-14,
-// a hub of 3,665 entries: 57 -> 26 us).
+// lanes idle on rows of four entries.  Rows of more than kBoundRow entries take
+// the whole wave, with several loads in flight (R-MAT-14, a hub of 3,665
+// entries: 57 -> 22 us; 512^2 lattice 70 -> 14).
 constexpr int kBoundRow = 128;
 __global__ __launch_bounds__(kBlock) void k_row_bound(const int32_t *__restrict__ arp,
                                                       const int32_t *__restrict__ acol,
                                                       const int32_t *__restrict__ brp, int32_t m,
                                                       int64_t *__restrict__ prods) {
-    constexpr int NG = kBlock / 16;
-    __shared__ int32_t s_long[NG], s_n;
     const int j = threadIdx.x & 15;
-    for (int64_t r0 = (int64_t)blockIdx.x * NG; r0 < m; r0 += (int64_t)gridDim.x * NG) {
-        if (threadIdx.x == 0) s_n = 0;
-        __syncthreads();
-        const int64_t i = r0 + threadIdx.x / 16;
-        if (i < m) {
-            const int32_t b = arp[i], e1 = arp[i + 1];
-            if (e1 - b > kBoundRow) {
-                if (j == 0) s_long[atomicAdd(&s_n, 1)] = (int32_t)i;
-            } else {
-                uint64_t s = 0;
-                for (int32_t e = b + j; e < e1; e += 16) {
-                    const int32_t k = acol[e];
-                    s += (uint64_t)(brp[k + 1] - brp[k]);
-                }
-#pragma unroll
-                for (int d = 8; d >= 1; d >>= 1) s += __shfl_xor(s, d, 16);
-                if (j == 0) prods[i] = (int64_t)s;
-            }
-        }
-        __syncthreads();
-        for (int q = threadIdx.x / 64; q < s_n; q += kBlock / 64) {
-            const int32_t r = s_long[q], e1 = arp[r + 1];
-            uint64_t s = 0;
-#pragma unroll 8
-            for (int32_t e = arp[r] + dev::lane_id(); e < e1; e += 64) {
+    const int64_t step = (int64_t)gridDim.x * (kBlock / 16);
+    const int64_t i0 = (int64_t)blockIdx.x * (kBlock / 16) + threadIdx.x / 64 * 4;
+    for (int64_t w = i0; w < m; w += step) {  // the wave's first row
+        const int64_t i = w + (threadIdx.x / 16 & 3);
+        const int32_t b = i < m ? arp[i] : 0, e1 = i < m ? arp[i + 1] : 0;
+        const bool is_long = e1 - b > kBoundRow;
+        uint64_t s = 0;
+        if (!is_long)
+            for (int32_t e = b + j; e < e1; e += 16) {
                 const int32_t k = acol[e];
                 s += (uint64_t)(brp[k + 1] - brp[k]);
             }
-            s = dev::wave_sum_u64(s);
-            if (dev::lane_id() == 0) prods[r] = (int64_t)s;
+#pragma unroll
+        for (int d = 8; d >= 1; d >>= 1) s += __shfl_xor(s, d, 16);
+        if (j == 0 && i < m && !is_long) prods[i] = (int64_t)s;
+        for (uint64_t todo = __ballot(is_long && j == 0); todo; todo &= todo - 1) {
+            const int src = __ffsll((unsigned long long)todo) - 1;
+            const int32_t lb = __shfl(b, src, 64), le = __shfl(e1, src, 64);
+            uint64_t t = 0;
+#pragma unroll 8
+            for (int32_t e = lb + dev::lane_id(); e < le; e += 64) {
+                const int32_t k = acol[e];
+                t += (uint64_t)(brp[k + 1] - brp[k]);
+            }
+            t = dev::wave_sum_u64(t);
+            if (dev::lane_id() == 0) prods[w + src / 16] = (int64_t)t;
         }
-        __syncthreads();  // s_n is reset by the next pass
     }
 }
 
@@ -397,14 +390,20 @@ __device__ __forceinline__ int wave_find(const int32_t *pre, int cn, int32_t x) 
     return c + __popcll(__ballot(lane < 16 && c + lane < cn && pre[min(c + lane, cn)] <= x)) - 1;
 }
 
+// A staged entry of A_i.
+struct Entry {
+    int32_t base;  // product x of the chunk is B's entry base + x
+    float a;
+};
+
 // One wave's share of a chunk's W products: RUN slices of 64 consecutive ones
 // from w0, a product per lane and slice, so that a long B row is read
 // coalesced and its entry found once (R-MAT-14: 91 % of the products lie in B
 // rows of 256 entries and more).  All loads of B go out before the first
 // product is applied.
 template <int RUN, class F>
-__device__ __forceinline__ void wave_products(const int32_t *pre, const int32_t *rs,
-                                              const float *av, int cn, int32_t w0, int32_t W,
+__device__ __forceinline__ void wave_products(const int32_t *pre, const Entry *ent, int cn,
+                                              int32_t w0, int32_t W,
                                               const int32_t *__restrict__ bcol,
                                               const float *__restrict__ bval, F &&f) {
     const int jl = __builtin_amdgcn_readfirstlane(wave_find(pre, cn, w0));
@@ -428,9 +427,10 @@ __device__ __forceinline__ void wave_products(const int32_t *pre, const int32_t 
     }
 #pragma unroll
     for (int q = 0; q < RUN; ++q) {
-        const int64_t e = (int64_t)rs[j[q]] + (x[q] - pre[j[q]]);
+        const Entry t = ent[j[q]];
+        const int32_t e = t.base + x[q];
         key[q] = bcol[e];
-        a[q] = av[j[q]];
+        a[q] = t.a;
         b[q] = bval ? bval[e] : 1.0f;
     }
 #pragma unroll
@@ -439,13 +439,14 @@ __device__ __forceinline__ void wave_products(const int32_t *pre, const int32_t 
 }
 
 // The products of row r, load-balanced over the block: f(col, value) per
-// product.  pre / rs / av are LDS staging of kChunk entries of A_r.
-template <int BLOCK, class F>
+// product.  pre / ent are LDS staging of kChunk entries of A_r; RUN products per
+// lane have their loads in flight together.
+template <int BLOCK, int RUN, class F>
 __device__ __forceinline__ void for_products(int32_t r, const int32_t *arp, const int32_t *acol,
                                              const float *aval, const int32_t *brp,
                                              const int32_t *bcol, const float *bval,
-                                             int32_t *pre, int32_t *rs, float *av,
-                                             uint64_t *s_scan, F &&f) {
+                                             int32_t *pre, Entry *ent, uint64_t *s_scan,
+                                             F &&f) {
     const int32_t ab = arp[r], an = arp[r + 1] - ab;
     for (int32_t c0 = 0; c0 < an; c0 += kChunk) {
         const int32_t cn = min(kChunk, an - c0);
@@ -453,17 +454,20 @@ __device__ __forceinline__ void for_products(int32_t r, const int32_t *arp, cons
         for (int32_t x0 = 0; x0 < cn; x0 += BLOCK) {
             const int32_t x = x0 + threadIdx.x;
             uint32_t len = 0;
+            int32_t b0 = 0;
             if (x < cn) {
                 const int32_t k = acol[ab + c0 + x];
-                const int32_t b0 = brp[k];
+                b0 = brp[k];
                 len = (uint32_t)(brp[k + 1] - b0);
-                rs[x] = b0;
-                av[x] = aval ? aval[ab + c0 + x] : 1.0f;
             }
             if (x0 > 0) __syncthreads();  // s_scan is free again
             dev::Pair32 tot;
-            const uint32_t ex = dev::block_exclusive_add_pair<BLOCK>(len, 0u, s_scan, tot).a;
-            if (x < cn) pre[x] = (int32_t)(carry + ex);
+            const uint32_t ex =
+                carry + dev::block_exclusive_add_pair<BLOCK>(len, 0u, s_scan, tot).a;
+            if (x < cn) {
+                pre[x] = (int32_t)ex;
+                ent[x] = Entry{b0 - (int32_t)ex, aval ? aval[ab + c0 + x] : 1.0f};
+            }
             carry += tot.a;
         }
         if (threadIdx.x == 0) pre[cn] = (int32_t)carry;
@@ -471,14 +475,17 @@ __device__ __forceinline__ void for_products(int32_t r, const int32_t *arp, cons
         const int32_t W = (int32_t)carry;
         const int32_t wave = threadIdx.x / 64;
         // a chunk that does not give every wave half a run goes out in slices
-        if (W >= BLOCK * kRun / 2) {
-            for (int32_t w0 = wave * 64 * kRun; w0 < W; w0 += BLOCK * kRun)
-                wave_products<kRun>(pre, rs, av, cn, w0, W, bcol, bval, f);
+        if (W >= BLOCK * RUN / 2) {
+            for (int32_t w0 = wave * 64 * RUN; w0 < W; w0 += BLOCK * RUN)
+                wave_products<RUN>(pre, ent, cn, w0, W, bcol, bval, f);
+        } else if (RUN > 4 && W >= BLOCK * 2) {
+            for (int32_t w0 = wave * 64 * 4; w0 < W; w0 += BLOCK * 4)
+                wave_products<4>(pre, ent, cn, w0, W, bcol, bval, f);
         } else {
             for (int32_t w0 = wave * 64; w0 < W; w0 += BLOCK)
-                wave_products<1>(pre, rs, av, cn, w0, W, bcol, bval, f);
+                wave_products<1>(pre, ent, cn, w0, W, bcol, bval, f);
         }
-        __syncthreads();  // pre / rs / av are refilled by the next chunk
+        __syncthreads();  // pre / ent are refilled by the next chunk
     }
 }
 
@@ -533,8 +540,8 @@ __global__ __launch_bounds__(BLOCK) void k_rows_table(const int32_t *rows, const
     constexpr bool LDS = TABLE > 0;
     __shared__ int32_t s_keys[LDS ? TABLE : 1];
     __shared__ float s_vals[(LDS && NUMERIC) ? TABLE : 1];
-    __shared__ int32_t pre[kChunk + 1], rs[kChunk];
-    __shared__ float av[kChunk];
+    __shared__ int32_t pre[kChunk + 1];
+    __shared__ Entry ent[kChunk];
     __shared__ uint32_t s_scan[BLOCK / 64 + 1];
     __shared__ uint64_t s_stage[BLOCK / 64];
     __shared__ uint32_t s_count;
@@ -553,7 +560,7 @@ __global__ __launch_bounds__(BLOCK) void k_rows_table(const int32_t *rows, const
         if (threadIdx.x == 0) s_count = 0;
         __syncthreads();
         uint32_t created = 0;
-        for_products<BLOCK>(r, arp, acol, aval, brp, bcol, bval, pre, rs, av, s_stage,
+        for_products<BLOCK, kRun>(r, arp, acol, aval, brp, bcol, bval, pre, ent, s_stage,
                             [&](int32_t col, float v) {
                                 uint32_t slot;
                                 created += tab_insert(keys, mask, col, &slot) ? 1u : 0u;
@@ -570,7 +577,7 @@ __global__ __launch_bounds__(BLOCK) void k_rows_table(const int32_t *rows, const
             // order by rank instead of sorting: a bit per column (the chunk
             // staging arrays, free once the products are done), the words'
             // popcount prefix, and each entry's rank from its own word
-            uint32_t *bits = (uint32_t *)pre, *wpre = (uint32_t *)rs;
+            uint32_t *bits = (uint32_t *)pre, *wpre = (uint32_t *)ent;
             const int32_t nw = (ncols + 31) / 32;
             __syncthreads();  // every thread is past the last chunk
             for (int32_t q = threadIdx.x; q < nw; q += BLOCK) bits[q] = 0;
@@ -625,8 +632,9 @@ __global__ __launch_bounds__(BLOCK) void k_rows_table(const int32_t *rows, const
 // of its own against 192 for ds_add_f32, which takes its lanes one by one.
 // DN and BLOCK are the smallest that hold the columns, so that a CU holds 16
 // to 32 waves (a 128 KB accumulator leaves room for one block).  R-MAT-14
-// squared, 156M products: 2037 -> 542 us, symbolic 465 -> 199 (a block of 256
-// for its longest rows of 340,000 products took 480).
+// squared, 156M products: 2037 -> 517 us (542 with half the loads in flight),
+// symbolic 465 -> 200 (a block of 256 for its longest rows, 340,000 products,
+// took 480).
 template <int DN, int BLOCK>
 __global__ __launch_bounds__(BLOCK) void k_rows_dense(
     const int32_t *heavy, const int32_t *rest, const uint32_t *ctl, uint32_t *ticket,
@@ -636,12 +644,14 @@ __global__ __launch_bounds__(BLOCK) void k_rows_dense(
     const int32_t *crp, int32_t *ccol, float *cval) {
     constexpr bool NUMERIC = DN > 0;
     using Acc = std::conditional_t<(DN > kDenseN / 2), float, double>;
+    // where 16 waves fill the CU's LDS, each keeps twice the loads in flight
+    constexpr int RUN = DN > kDenseN / 4 ? 2 * kRun : kRun;
     constexpr int NWORD = (NUMERIC ? DN : kDenseN) / 32;
     static_assert(NWORD <= kChunk, "the words' places share the chunk staging");
     __shared__ Acc s_val[NUMERIC ? DN : 1];
     __shared__ uint32_t s_bits[NWORD];
-    __shared__ int32_t pre[kChunk + 1], rs[kChunk];
-    __shared__ float av[kChunk];
+    __shared__ int32_t pre[kChunk + 1];
+    __shared__ Entry ent[kChunk];
     __shared__ uint64_t s_scan[BLOCK / 64];
     __shared__ uint32_t s_row;
     const int32_t nw = (ncols + 31) / 32;
@@ -655,7 +665,7 @@ __global__ __launch_bounds__(BLOCK) void k_rows_dense(
         const uint32_t i = s_row;
         if (i >= nrows) return;
         const int32_t r = i < nheavy ? heavy[i] : rest[i - nheavy];
-        for_products<BLOCK>(r, arp, acol, aval, brp, bcol, bval, pre, rs, av, s_scan,
+        for_products<BLOCK, RUN>(r, arp, acol, aval, brp, bcol, bval, pre, ent, s_scan,
                             [&](int32_t col, float v) {
                                 // a set bit needs no atomic (a stale read only costs one)
                                 const uint32_t bit = 1u << (col & 31);
@@ -814,10 +824,10 @@ Graph *spgemm_run(Ctx *c, const Graph *a, const Graph *b) {
         c->stats.edges_traversed = nnz;
         c->stats.iterations = 1;
     } catch (...) {
-        (void)hipDeviceSynchronize();
-        graph_free(c, C->rowptr, sizeof(int32_t) * (m + 1));
-        graph_free(c, C->col, sizeof(int32_t) * std::max<int64_t>(C->nnz, 1));
-        graph_free(c, C->val, sizeof(float) * std::max<int64_t>(C->nnz, 1));
+        const bool idle = device_idle();
+        graph_free(c, C->rowptr, sizeof(int32_t) * (m + 1), idle);
+        graph_free(c, C->col, sizeof(int32_t) * std::max<int64_t>(C->nnz, 1), idle);
+        graph_free(c, C->val, sizeof(float) * std::max<int64_t>(C->nnz, 1), idle);
         delete C;
         throw;
     }
