@@ -1078,6 +1078,13 @@ __global__ __launch_bounds__(256) void k_batch_depths(
 }
 
 // One batched traversal pass for up to 32*W sources.
+// near-far rounds of a batch may pull (and keep their distances source-major)
+bool sssp_rounds_pull(Ctx *c, const Graph *g) {
+    return opt(c, "batch_sssp_pull_div", 4) > 0 &&
+           graph_max_degree(c, const_cast<Graph *>(g)) <= 64 &&
+           graph_is_symmetric_weighted(c, const_cast<Graph *>(g));
+}
+
 template <int W, bool SSSP>
 void batch_pass(Ctx *c, const Graph *g, const int32_t *src_host, int32_t nsrc, int32_t *depth_out,
                 float *dist_out) {
@@ -1158,9 +1165,7 @@ void batch_pass(Ctx *c, const Graph *g, const int32_t *src_host, int32_t nsrc, i
     // lattice, 32 / 64 sources: 0.94 -> 0.88 / 0.73 -> 0.71 ms per query;
     // 128 sources are best at the option's 4)
     const int32_t sssp_pull_div =
-        near_far && opt(c, "batch_sssp_pull_div", 4) > 0 &&
-                graph_max_degree(c, const_cast<Graph *>(g)) <= 64 &&
-                graph_is_symmetric_weighted(c, const_cast<Graph *>(g))
+        near_far && sssp_rounds_pull(c, g)
             ? (int32_t)std::min<int64_t>(opt(c, "batch_sssp_pull_div", 4) * (W <= 2 ? 2 : 1),
                                          1 << 22)
             : 0;
@@ -1299,6 +1304,8 @@ void batch_pass(Ctx *c, const Graph *g, const int32_t *src_host, int32_t nsrc, i
     APSPIE_LAUNCH_CHECK();
 }
 
+constexpr int32_t kSourceMajorGroup = 128, kSourceMajorFrom = 1 << 20;
+
 template <bool SSSP>
 void batch_run(Ctx *c, const Graph *g, const int32_t *src, int32_t nsrc, int32_t *depth,
                float *dist) {
@@ -1310,11 +1317,19 @@ void batch_run(Ctx *c, const Graph *g, const int32_t *src, int32_t nsrc, int32_t
     // 0.154 ms per query on average in groups of 128 / 256 / 512 (0.107-0.165
     // in groups of 256; plain 0.206)
     static_assert(kQueue % kBlock == 0, "queue flushes take whole block rows");
-    const int32_t group =
+    int32_t group =
         !SSSP && graph_max_degree(c, const_cast<Graph *>(g)) > 64
             ? (int32_t)std::min<int64_t>(std::max<int64_t>(opt(c, "batch_long_row_group", 256), 1),
                                          kMaxBatch)
             : kMaxBatch;
+    // source-major SSSP from kSourceMajorFrom vertices on runs in groups of 128:
+    // the rings of more sources at once no longer share the caches (512 sources,
+    // ms per query in groups of 512 / 256 / 128: 2048^2 lattice 0.652 / 0.553 /
+    // 0.508, 1024^2 0.167 / 0.150 / 0.151).  On smaller graphs the rounds' fixed
+    // cost weighs more (724^2 0.067 / 0.071 / 0.077, 512^2 0.040 / 0.044 / 0.057)
+    if (SSSP && nsrc > kSourceMajorGroup && g->m >= kSourceMajorFrom &&
+        opt(c, "batch_sssp_delta", -1) != 0 && sssp_rounds_pull(c, g))
+        group = kSourceMajorGroup;
     for (int32_t s0 = 0; s0 < nsrc; s0 += group) {
         const int32_t k = std::min(group, nsrc - s0);
         int32_t *d = depth ? depth + (int64_t)s0 * g->m : nullptr;

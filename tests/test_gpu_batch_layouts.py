@@ -94,3 +94,24 @@ def test_sssp_distance_layouts(ctx, kind, nsrc):
         ctx.set_option("batch_sssp_delta", -1)
         ctx.set_option("batch_sssp_pull_div", 4)
         G.close()
+
+
+@pytest.mark.parametrize("nsrc", [128, 129, 200, 260])
+def test_groups_of_a_large_graph(nsrc):
+    """From 2^20 vertices on, source-major SSSP splits a batch in groups of
+    128: every row equals the single-source call's."""
+    w = 1024
+    ids = np.arange(w * w).reshape(w, w)
+    u = np.concatenate([ids[:, :-1].ravel(), ids[:-1].ravel()]).astype(np.int32)
+    v = np.concatenate([ids[:, 1:].ravel(), ids[1:].ravel()]).astype(np.int32)
+    rng = np.random.default_rng(nsrc)
+    keep = rng.random(len(u)) >= 0.1
+    u, v = u[keep], v[keep]
+    val = rng.integers(1, 256, len(u)).astype(np.float32)
+    src = rng.choice(w * w, nsrc, replace=False).astype(np.int32)
+    with A.Context(0) as c:
+        G = c.from_coo(w * w, u, v, val)
+        got = c.sssp_batch(G, src)
+        for i in {0, 1, 127, nsrc - 1, min(128, nsrc - 1), min(256, nsrc - 1)}:
+            assert np.array_equal(got[i], c.sssp(G, int(src[i])))
+        G.close()
