@@ -507,8 +507,11 @@ k_sssp_nf_round(const int32_t *__restrict__ rowptr, const int32_t *__restrict__ 
     }
     // split: move the pending vertices below the new threshold into the
     // frontier, and in light / heavy mode add the heavy entries of the
-    // vertices marked since the last split (a moved vertex brings its light
-    // and its heavy entries).  The 32 vertices of a mark word sit in 32
+    // vertices marked since the last split.  A moved vertex brings its light
+    // and its heavy entries as one frontier entry, its whole row: with one for
+    // each part a split could append 2 m of them, and the frontier holds m + 1
+    // (2^20 vertices joined to a hub at one weight, light and heavy entries
+    // each: 2,097,150).  The 32 vertices of a mark word sit in 32
     // consecutive lanes, and the word's first lane clears it after the wave
     // has read it (nothing marks during a split).
     uint64_t left = 0;
@@ -516,13 +519,13 @@ k_sssp_nf_round(const int32_t *__restrict__ rowptr, const int32_t *__restrict__ 
     const int64_t width = (int64_t)gridDim.x * kNfBlock;
     const int per = (int)min<int64_t>(kNfPer, (m + width - 1) / width);
     for (int64_t pbase = (int64_t)blockIdx.x * kNfBlock * per; pbase < m; pbase += width * per) {
-        int32_t cv[kNfPer], crs[kNfPer], cd[kNfPer], hrs[kNfPer], hd[kNfPer];
+        int32_t cv[kNfPer], crs[kNfPer], cd[kNfPer];
         bool take[kNfPer], drop[kNfPer], marked[kNfPer];
 #pragma unroll
         for (int k = 0; k < kNfPer; ++k) {
             const int64_t v = pbase + (int64_t)k * kNfBlock + threadIdx.x;
             cv[k] = (int32_t)v;
-            crs[k] = cd[k] = hrs[k] = hd[k] = 0;
+            crs[k] = cd[k] = 0;
             take[k] = drop[k] = marked[k] = false;
             if (k >= per) continue;
             if (v < m && pend[v]) {
@@ -543,20 +546,14 @@ k_sssp_nf_round(const int32_t *__restrict__ rowptr, const int32_t *__restrict__ 
 #pragma unroll
         for (int k = 0; k < kNfPer; ++k) {
             if (take[k] || drop[k]) pend[cv[k]] = 0;
-            if (take[k]) {  // the sweep meets each vertex once: no claim needed
-                crs[k] = rowptr[cv[k]];
-                cd[k] = rend[cv[k]] - crs[k];
-            }
+            // the sweep meets each vertex once: no claim needed
             if (take[k] || marked[k]) {
-                hrs[k] = rend[cv[k]];
-                hd[k] = hb ? rowptr[cv[k] + 1] - hrs[k] : 0;
+                crs[k] = take[k] ? rowptr[cv[k]] : rend[cv[k]];
+                cd[k] = rowptr[cv[k] + 1] - crs[k];
             }
         }
         produce<kNfBlock, kNfPer, TILE, true>(cv, crs, cd, nxt, ctl + ((r + 1) % 3), lds.scan,
                                               &lds.base);
-        if (hb)
-            produce<kNfBlock, kNfPer, TILE, true>(cv, hrs, hd, nxt, ctl + ((r + 1) % 3),
-                                                  lds.scan, &lds.base);
     }
     const uint64_t ws = dev::wave_sum_u64(left);
     const uint32_t wm = dev::wave_min_u32(min_left);

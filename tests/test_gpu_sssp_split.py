@@ -1,0 +1,42 @@
+"""Light / heavy splits that move most vertices of a graph without isolated
+ones: the frontier gets one entry per vertex, which is all it has room for."""
+import numpy as np
+import pytest
+
+import apspie_amd as A
+from oracle import oracle as O
+from tests.test_nearfar_entries import hub_graph
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("tile", [1024, 2048, 4096])
+@pytest.mark.parametrize("m", [65, 1000, 70_001])
+def test_split_moves_every_vertex(m, tile):
+    rp, c, w = hub_graph(m, 4)
+    with A.Context(0) as ctx:
+        ctx.set_option("bfs_tile", tile)
+        ctx.set_option("sssp_delta", 100)
+        G = ctx.upload(rp.astype(np.int32), c, w)
+        for src in (0, 1, m - 1):
+            assert np.array_equal(ctx.sssp(G, src), O.sssp(m, rp, c, w, src))
+            if src == 0:  # the hub, then every other vertex once
+                assert ctx.stats()["vertices_reached"] == m
+        G.close()
+
+
+@pytest.mark.parametrize("delta", [72, 80, 96])
+def test_uniform_rows(delta):
+    """Rows of about 32 entries, weights 1..255: splits that move a large part
+    of the vertices, all of them with light and heavy entries."""
+    m = 1 << 14
+    rng = np.random.default_rng(delta)
+    rp, c = O.edges_to_csr(m, rng.integers(0, m, 16 * m).astype(np.int32),
+                           rng.integers(0, m, 16 * m).astype(np.int32))
+    w = O.assign_weights(m, rp, c)
+    with A.Context(0) as ctx:
+        ctx.set_option("sssp_delta", delta)
+        G = ctx.upload(rp.astype(np.int32), c, w)
+        for src in (0, m // 2):
+            assert np.array_equal(ctx.sssp(G, src), O.sssp(m, rp, c, w, src))
+        G.close()
