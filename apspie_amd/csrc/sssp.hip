@@ -882,7 +882,7 @@ double sssp_weight_delta(Ctx *c, Graph *g) {
 // The width used when sssp_delta is left at -1.
 //
 // Sparse rows (the weights' width above every weight, so that no entry is
-// heavy): four times that width from kNfSparse vertices on -- the rounds'
+// heavy): four times that width from kNfFrom vertices on -- the rounds'
 // fixed cost (about 8 us) weighs more than the re-expansions a wider bucket
 // adds -- and Bellman-Ford rounds (0) below.  Lattices at weights 1..255, ms
 // per source, Bellman-Ford / 512 / 2048 / 8192: 512^2 1.14 / 1.76 / 1.30 /
@@ -891,19 +891,24 @@ double sssp_weight_delta(Ctx *c, Graph *g) {
 // 4.45.
 //
 // Longer rows (light / heavy rounds): 1.42 * largest weight / sqrt(mean row),
-// narrower on large graphs by (2^20 / m)^0.4, from kNfHeavy vertices on (below
-// it they gain less than the light-first copy costs a graph's first call).
-// R-MAT, edge factor 16, Bellman-Ford / 32 / 48 / 64 / 96: 2^17 0.45 / 0.52 /
-// 0.46 / 0.44 / 0.44, 2^18 0.67 / 0.67 / 0.52 / 0.55 / 0.57, 2^20 1.39 / 1.15 /
-// 1.08 / 1.07 / 1.12, 2^22 4.44 / 2.67 / 2.76 / 2.93 / 3.23; edge factor 8: 2^20
-// 1.09 / 0.99 / 0.87 / 0.92 / 0.78, 2^22 2.95 / 1.99 / 1.94 / 2.00 / 2.19.
-constexpr int32_t kNfSparse = 3 << 18, kNfHeavy = 1 << 20;
+// narrower on large graphs by (2^20 / m)^0.4, from kNfFrom vertices on too.
+// The light-first copy makes a graph's first call longer and every later one
+// shorter, ms with Bellman-Ford and with light / heavy rounds, first call /
+// later ones: 786432 vertices at edge factor 16 1.10 / 1.05 and 1.29 / 0.82,
+// 900000 1.36 / 1.31 and 1.39 / 0.97, at edge factor 8 0.99 / 0.93 and 1.12 /
+// 0.82, 2^20 at edge factor 16 1.49 / 1.44 and 1.74 / 1.04.  (Below, less is
+// gained a call: 2^18 0.67 against 0.52.)  R-MAT, edge factor 16, later calls,
+// Bellman-Ford / 32 / 48 / 64 / 96: 2^17 0.45 / 0.52 / 0.46 / 0.44 / 0.44, 2^18
+// 0.67 / 0.67 / 0.52 / 0.55 / 0.57, 2^20 1.39 / 1.15 / 1.08 / 1.07 / 1.12, 2^22
+// 4.44 / 2.67 / 2.76 / 2.93 / 3.23; edge factor 8: 2^20 1.09 / 0.99 / 0.87 / 0.92 /
+// 0.78, 2^22 2.95 / 1.99 / 1.94 / 2.00 / 2.19.
+constexpr int32_t kNfFrom = 3 << 18;
 double sssp_auto_delta(Ctx *c, Graph *g) {
-    if (g->m < std::min(kNfSparse, kNfHeavy)) return 0;
+    if (g->m < kNfFrom) return 0;
     const double d = sssp_weight_delta(c, g);
     float lo = 0.0f, hi = 0.0f;
     if (!(d > 0) || !graph_weight_range(c, g, &lo, &hi)) return 0;
-    if (d > hi) return g->m >= kNfSparse ? 4 * d : 0;
+    if (d > hi) return 4 * d;
     if (opt(c, "sssp_light_heavy", 1) == 0) return g->m >= (1 << 22) ? d : 0;
     const double w = 1.42 * hi / std::sqrt(std::max(1.0, (double)g->nnz / g->m)) *
                      std::min(1.0, std::pow((double)(1 << 20) / g->m, 0.4));

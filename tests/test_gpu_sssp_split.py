@@ -40,3 +40,16 @@ def test_uniform_rows(delta):
         for src in (0, m // 2):
             assert np.array_equal(ctx.sssp(G, src), O.sssp(m, rp, c, w, src))
         G.close()
+
+
+@pytest.mark.parametrize("m,near_far", [((3 << 18) - 1, False), (3 << 18, True)])
+def test_default_width_of_longer_rows(m, near_far):
+    """Graphs whose weights split into light and heavy take near-far rounds
+    from 3 * 2^18 vertices on.  Bellman-Ford rounds from the hub are two (the hub,
+    then all others once); a split is a round more."""
+    rp, c, w = hub_graph(m, 4)
+    with A.Context(0) as ctx:
+        G = ctx.upload(rp.astype(np.int32), c, w)
+        assert np.array_equal(ctx.sssp(G, 0), np.where(np.arange(m) == 0, 0, 200))
+        assert (ctx.stats()["iterations"] != 2) == near_far
+        G.close()
