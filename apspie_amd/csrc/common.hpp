@@ -151,6 +151,8 @@ hipError_t device_malloc(Ctx *c, void **p, size_t bytes);
 void *graph_alloc(Ctx *c, size_t bytes);
 bool device_idle();
 void graph_free(Ctx *c, void *p, size_t bytes, bool keep);
+// The arrays that a graph of context c has so far, if any.
+void graph_release(Ctx *c, Graph *g);
 void drop_spares(Ctx *c);
 
 // Run `f` translating exceptions into status codes and recording the message.

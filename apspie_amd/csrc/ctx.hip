@@ -206,6 +206,19 @@ void graph_free(Ctx *c, void *p, size_t bytes, bool keep) {
     dev_free(c, p, bytes);
 }
 
+void graph_release(Ctx *c, Graph *g) {
+    if (!g->rowptr && !g->col && !g->val) return;
+    (void)hipSetDevice(c->device);
+    // every stream, as hipFree waits: another context or the caller's own
+    // stream may still read the arrays, and they are given out again
+    const bool idle = device_idle();
+    graph_free(c, g->rowptr, sizeof(int32_t) * (g->m + 1), idle);
+    graph_free(c, g->col, sizeof(int32_t) * g->nnz, idle);
+    graph_free(c, g->val, sizeof(float) * g->nnz, idle);
+    g->rowptr = g->col = nullptr;
+    g->val = nullptr;
+}
+
 namespace {
 
 constexpr size_t kGranule = 256;
@@ -601,10 +614,7 @@ int apspie_graph_upload(apspie_ctx *c, const apspie_csr *h, apspie_graph **out) 
         sync(c);
     });
     if (st != APSPIE_OK) {
-        const bool idle = device_idle();
-        graph_free(c, g->rowptr, sizeof(int32_t) * (h->m + 1), idle);
-        graph_free(c, g->col, sizeof(int32_t) * h->nnz, idle);
-        graph_free(c, g->val, sizeof(float) * h->nnz, idle);
+        graph_release(c, g);
         delete g;
         return st;
     }
@@ -684,12 +694,7 @@ int apspie_graph_destroy(apspie_graph *g) {
     }
     if (g->owns) {
         if (c) {
-            // every stream, as hipFree waits: another context or the caller's own
-            // stream may still read the arrays, and they are given out again
-            const bool idle = device_idle();
-            graph_free(c, g->rowptr, sizeof(int32_t) * (g->m + 1), idle);
-            graph_free(c, g->col, sizeof(int32_t) * g->nnz, idle);
-            graph_free(c, g->val, sizeof(float) * g->nnz, idle);
+            graph_release(c, g);
         } else {
             (void)hipFree(g->rowptr);
             (void)hipFree(g->col);

@@ -1,5 +1,7 @@
 """Arrays of destroyed graphs are kept for the next ones: the accounting, the
 budget and the results are those of arrays freed at once."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -66,3 +68,21 @@ def test_budget_and_other_contexts():
         g = c.upload(*csr)  # outlives its context, on a block given out twice
         keep.close()
     g.close()
+
+
+def test_upload_refuses_without_arrays():
+    """A refused upload has nothing to release: no description at all, none of
+    the arrays, or a column out of range."""
+    csr = _csr(100, 3, 5)
+    with A.Context(0) as c:
+        base = c.hbm_used()
+        h = C.c_void_p()
+        for arg in (None, C.byref(A._Csr(4, 4, 0, None, None, None))):
+            assert A.lib().apspie_graph_upload(c.h, arg, C.byref(h)) != 0
+            assert not h
+        with pytest.raises(A.ApspieError):
+            c.upload(csr[0], np.full_like(csr[1], 100), csr[2])
+        assert c.hbm_used() == base
+        g = c.upload(*csr)
+        _check(g, csr)
+        g.close()
