@@ -676,6 +676,7 @@ int apspie_graph_from_coo(apspie_ctx *c, const apspie_coo *coo, int mem, int sym
         sync(c);
     });
     if (st != APSPIE_OK) {
+        graph_release(c, g);
         delete g;
         return st;
     }
@@ -798,6 +799,7 @@ int apspie_graph_transpose(apspie_ctx *c, const apspie_graph *g, apspie_graph **
         sync(c);
     });
     if (st != APSPIE_OK) {
+        graph_release(c, t);
         delete t;
         return st;
     }

@@ -824,10 +824,7 @@ Graph *spgemm_run(Ctx *c, const Graph *a, const Graph *b) {
         c->stats.edges_traversed = nnz;
         c->stats.iterations = 1;
     } catch (...) {
-        const bool idle = device_idle();
-        graph_free(c, C->rowptr, sizeof(int32_t) * (m + 1), idle);
-        graph_free(c, C->col, sizeof(int32_t) * std::max<int64_t>(C->nnz, 1), idle);
-        graph_free(c, C->val, sizeof(float) * std::max<int64_t>(C->nnz, 1), idle);
+        graph_release(c, C);
         delete C;
         throw;
     }

@@ -86,3 +86,39 @@ def test_upload_refuses_without_arrays():
         g = c.upload(*csr)
         _check(g, csr)
         g.close()
+
+
+@pytest.mark.parametrize("kind", ["from_coo", "transpose", "spgemm"])
+@pytest.mark.parametrize("room", [0, 1, 2])
+def test_refused_results_give_their_arrays_back(kind, room):
+    """A result whose first `room` arrays fit the budget and whose next one is
+    refused: nothing stays counted, and the call passes once there is room."""
+    m, k = 300_000, 8
+    rp, col, val = _csr(m, k, 3)
+    rows = np.repeat(np.arange(m, dtype=np.int32), k)
+    eye = np.arange(m + 1, dtype=np.int32)
+    with A.Context(0) as c:
+        a = c.upload(rp, col, val)
+        one = c.upload(eye, eye[:-1], np.ones(m, np.float32))
+
+        def make():
+            if kind == "from_coo":
+                return c.from_coo(m, rows, col, val, symmetrize=False)
+            return a.transpose() if kind == "transpose" else c.spgemm(one, a)
+
+        g = make()
+        nnz = len(g.download()[1])
+        g.close()  # the scratch buffers stay
+        used = c.hbm_used()
+        c.set_hbm_budget(used + sum([4 * (m + 1), 4 * nnz, 4 * nnz][:room]) + m)
+        for _ in range(2):
+            with pytest.raises(A.ApspieError):
+                make()
+            assert c.hbm_used() == used
+        c.set_hbm_budget(0)
+        g = make()
+        assert c.hbm_used() == used + 4 * (m + 1) + 8 * nnz
+        g.close()
+        assert c.hbm_used() == used
+        a.close()
+        one.close()
