@@ -146,8 +146,9 @@ void *dev_alloc(Ctx *c, size_t bytes);  // counted against the budget
 void dev_free(Ctx *c, void *p, size_t bytes);
 // hipMalloc that gives the context's spare blocks back before it fails.
 hipError_t device_malloc(Ctx *c, void **p, size_t bytes);
-// A graph's arrays: counted as dev_alloc's are, from the spare blocks where one
-// fits.  A block is kept only where device_idle() has waited for every stream.
+// A graph's arrays (of no bytes: a small one), counted as dev_alloc's are, from the
+// spare blocks where one fits.  A block is kept only where device_idle() has
+// waited for every stream.
 void *graph_alloc(Ctx *c, size_t bytes);
 bool device_idle();
 void graph_free(Ctx *c, void *p, size_t bytes, bool keep);

@@ -319,8 +319,8 @@ void graph_from_coo_dev(Ctx *c, Graph *g, const int32_t *row, const int32_t *col
     const int64_t k = symmetrize ? h[0] : E;
     g->nnz = k;
     g->rowptr = (int32_t *)graph_alloc(c, sizeof(int32_t) * (g->m + 1));
-    g->col = (int32_t *)graph_alloc(c, sizeof(int32_t) * std::max<int64_t>(k, 1));
-    g->val = (float *)graph_alloc(c, sizeof(float) * std::max<int64_t>(k, 1));
+    g->col = (int32_t *)graph_alloc(c, sizeof(int32_t) * k);
+    g->val = (float *)graph_alloc(c, sizeof(float) * k);
     g->bytes = (int64_t)(sizeof(int32_t) * (g->m + 1) + 8 * std::max<int64_t>(k, 1));
     if (symmetrize) emit_csr<true>(c, g, ka, va, E, cb, offsets);
     else emit_csr<false>(c, g, ka, va, E, cb, nullptr);
@@ -714,8 +714,8 @@ void graph_transpose_dev(Ctx *c, const Graph *g, Graph *t, const char *in_scratc
         t->val = g->val ? (float *)scratch(c, p + "_val", sizeof(float) * Ea) : nullptr;
     } else {
         t->rowptr = (int32_t *)graph_alloc(c, sizeof(int32_t) * (t->m + 1));
-        t->col = (int32_t *)graph_alloc(c, sizeof(int32_t) * Ea);
-        t->val = g->val ? (float *)graph_alloc(c, sizeof(float) * Ea) : nullptr;
+        t->col = (int32_t *)graph_alloc(c, sizeof(int32_t) * E);
+        t->val = g->val ? (float *)graph_alloc(c, sizeof(float) * E) : nullptr;
     }
     t->bytes = (int64_t)(sizeof(int32_t) * (t->m + 1) + (g->val ? 8 : 4) * Ea);
     emit_csr<false>(c, t, ka, va, E, rb, nullptr);

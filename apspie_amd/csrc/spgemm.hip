@@ -816,8 +816,8 @@ Graph *spgemm_run(Ctx *c, const Graph *a, const Graph *b) {
         const int64_t nnz = scan_exclusive_i32(c, row_nnz, C->rowptr, m + 1);
         APSPIE_CHECK(nnz < INT32_MAX, APSPIE_ERR_OVERFLOW, "product has more than 2^31 entries");
         C->nnz = nnz;
-        C->col = (int32_t *)graph_alloc(c, sizeof(int32_t) * std::max<int64_t>(nnz, 1));
-        C->val = (float *)graph_alloc(c, sizeof(float) * std::max<int64_t>(nnz, 1));
+        C->col = (int32_t *)graph_alloc(c, sizeof(int32_t) * nnz);
+        C->val = (float *)graph_alloc(c, sizeof(float) * nnz);
         C->bytes = (int64_t)(sizeof(int32_t) * (m + 1) + 8 * std::max<int64_t>(nnz, 1));
         if (nnz > 0) pass(std::true_type{}, C->rowptr, C->col, C->val);
         sync(c);

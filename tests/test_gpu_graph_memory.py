@@ -122,3 +122,20 @@ def test_refused_results_give_their_arrays_back(kind, room):
         assert c.hbm_used() == used
         a.close()
         one.close()
+
+
+def test_edgeless_graphs_are_counted_and_uncounted_alike():
+    with A.Context(0) as c:
+        none = np.zeros(0, np.int32)
+        a = c.upload(np.zeros(6, np.int32), none, np.zeros(0, np.float32))
+        for make in (lambda: c.from_coo(5, none, none, symmetrize=True),
+                     lambda: c.from_coo(5, np.arange(5), np.arange(5), symmetrize=True),
+                     a.transpose, lambda: c.spgemm(a, a)):
+            make().close()
+            used = c.hbm_used()
+            for _ in range(2):
+                g = make()
+                assert len(g.download()[1]) == 0 and c.hbm_used() > used
+                g.close()
+                assert c.hbm_used() == used
+        a.close()
