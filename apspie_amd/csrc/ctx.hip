@@ -135,7 +135,9 @@ hipError_t device_malloc(Ctx *c, void **p, size_t bytes) {
 // Freeing the 320 MB of an R-MAT-14 square took 0.48 ms, and 8 ms once a loop of
 // products had freed some 100 GB (the freed memory has to be cleared before it
 // can be given out); a block kept costs neither.  Blocks below 1 MB are not
-// worth keeping, and one is not given to a request below 8/9 of its size.
+// worth keeping, and one is not given to a request below 8/9 of its size.  What
+// counts as used is the request, so that a call is refused where it would be with
+// arrays of its own; under a budget a block has to be of the request's size.
 constexpr size_t kSpareMin = (size_t)1 << 20, kSpareBytes = (size_t)512 << 20;
 
 bool device_idle() {
@@ -154,18 +156,19 @@ void drop_spares(Ctx *c) {
 void *graph_alloc(Ctx *c, size_t bytes) {
     if (bytes >= kSpareMin) {
         std::lock_guard<std::mutex> lock(c->spare_mu);
+        const size_t most = c->budget > 0 ? bytes : bytes + bytes / 8;
         auto best = c->spares.end();
         for (auto it = c->spares.begin(); it != c->spares.end(); ++it)
-            if (it->bytes >= bytes && it->bytes <= bytes + bytes / 8 &&
+            if (it->bytes >= bytes && it->bytes <= most &&
                 (best == c->spares.end() || it->bytes < best->bytes))
                 best = it;
         if (best != c->spares.end() &&
-            (c->budget == 0 || c->used + (int64_t)best->bytes <= c->budget)) {
+            (c->budget == 0 || c->used + (int64_t)bytes <= c->budget)) {
             const Buffer b = *best;
             c->spare_sizes[b.ptr] = b.bytes;
             c->spares.erase(best);
             c->spare_bytes -= b.bytes;
-            c->used += (int64_t)b.bytes;
+            c->used += (int64_t)bytes;
             return b.ptr;
         }
     }
@@ -176,20 +179,21 @@ void graph_free(Ctx *c, void *p, size_t bytes, bool keep) {
     if (!p) return;
     {
         std::lock_guard<std::mutex> lock(c->spare_mu);
+        size_t block = bytes;
         const auto it = c->spare_sizes.find(p);
         if (it != c->spare_sizes.end()) {
-            bytes = it->second;
+            block = it->second;
             c->spare_sizes.erase(it);
         }
-        if (keep && bytes >= kSpareMin && bytes <= kSpareBytes) {
-            while (c->spare_bytes + bytes > kSpareBytes) {
+        if (keep && block >= kSpareMin && block <= kSpareBytes) {
+            while (c->spare_bytes + block > kSpareBytes) {
                 (void)hipFree(c->spares.front().ptr);
                 c->spare_bytes -= c->spares.front().bytes;
                 c->spares.pop_front();
             }
             Buffer b;
             b.ptr = p;
-            b.bytes = bytes;
+            b.bytes = block;
             bool kept = true;  // no exception leaves a destroy
             try {
                 c->spares.push_back(b);
@@ -197,7 +201,7 @@ void graph_free(Ctx *c, void *p, size_t bytes, bool keep) {
                 kept = false;
             }
             if (kept) {
-                c->spare_bytes += bytes;
+                c->spare_bytes += block;
                 c->used -= (int64_t)bytes;
                 return;
             }

@@ -139,3 +139,23 @@ def test_edgeless_graphs_are_counted_and_uncounted_alike():
                 g.close()
                 assert c.hbm_used() == used
         a.close()
+
+
+def test_larger_kept_blocks_do_not_narrow_a_budget():
+    """A graph that fits the budget to the byte fits it too where kept blocks up
+    to an eighth larger are at hand, and counts what it counts without them."""
+    large, csr = _csr(220_000, 16, 1), _csr(200_000, 16, 2)
+    with A.Context(0) as c:
+        g = c.upload(*csr)
+        size = c.hbm_used()
+        g.close()
+        c.trim()
+        for budget in (0, size):
+            c.set_hbm_budget(0)
+            c.upload(*large).close()
+            c.set_hbm_budget(budget)
+            g = c.upload(*csr)
+            assert c.hbm_used() == size
+            _check(g, csr)
+            g.close()
+            assert c.hbm_used() == 0
