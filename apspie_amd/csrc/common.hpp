@@ -3,6 +3,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <atomic>
 #include <cstdint>
 #include <deque>
 #include <cstdio>
@@ -97,7 +98,7 @@ struct Ctx {
     hipStream_t own_stream = nullptr;
     hipStream_t stream = nullptr;
     int64_t budget = 0;  // 0 = unlimited
-    int64_t used = 0;    // bytes held: uploaded graphs + scratch
+    std::atomic<int64_t> used{0};  // bytes held: uploaded graphs + scratch
     std::map<std::string, Buffer> scratch;
     // optional arena: one block of device memory the scratch buffers are
     // carved from (first fit, 256-byte granules, free ranges coalesced), so
@@ -123,9 +124,8 @@ struct Ctx {
     Buffer mis_prio;
     int32_t mis_prio_m = -1;
     // arrays of destroyed graphs, kept for the next ones (graph_alloc): oldest
-    // first, at most kSpareBytes, not counted as used but given back before
-    // the budget or the device runs short
-    std::mutex spare_mu;
+    // first, not counted as used but given back before the budget or the device
+    // runs short
     std::deque<Buffer> spares;
     size_t spare_bytes = 0;
     std::map<void *, size_t> spare_sizes;  // handed out again: bytes of the block
@@ -144,13 +144,13 @@ void *scratch(Ctx *c, const std::string &name, size_t bytes);
 int64_t scratch_room(Ctx *c);
 void *dev_alloc(Ctx *c, size_t bytes);  // counted against the budget
 void dev_free(Ctx *c, void *p, size_t bytes);
-// hipMalloc that gives the context's spare blocks back before it fails.
+// hipMalloc that gives the device's spare blocks back before it fails.
 hipError_t device_malloc(Ctx *c, void **p, size_t bytes);
 // A graph's arrays (of no bytes: a small one), counted as dev_alloc's are, from the
-// spare blocks where one fits.  A block is kept only where device_idle() has
+// spare blocks where one fits.  A block is kept only where may_keep_blocks() has
 // waited for every stream.
 void *graph_alloc(Ctx *c, size_t bytes);
-bool device_idle();
+bool may_keep_blocks();
 void graph_free(Ctx *c, void *p, size_t bytes, bool keep);
 // The arrays that a graph of context c has so far, if any.
 void graph_release(Ctx *c, Graph *g);

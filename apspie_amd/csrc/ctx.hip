@@ -99,9 +99,75 @@ void set_device(Ctx *c) { APSPIE_HIP(hipSetDevice(c->device)); }
 
 void sync(Ctx *c) { APSPIE_HIP(hipStreamSynchronize(c->stream)); }
 
+// Freeing the 320 MB of an R-MAT-14 square took 0.48 ms, and 8 ms once a loop of
+// products had freed some 100 GB (the freed memory has to be cleared before it
+// can be given out); a block kept costs neither.  Blocks below 1 MB are not
+// worth keeping, and one is not given to a request below 8/9 of its size.  What
+// counts as used is the request, so that a call is refused where it would be with
+// arrays of its own; under a budget a block has to be of the request's size.
+//
+// The blocks are the contexts' own, the rest is the device's: all its contexts
+// together keep at most kSpareBytes, none while less than 1/16 of the device's
+// memory is free, and when a hipMalloc of any of them fails, all give theirs back.
+constexpr size_t kSpareMin = (size_t)1 << 20, kSpareBytes = (size_t)512 << 20;
+
+namespace {
+
+// the contexts alive, and a lock for them and their spares, spare_bytes and
+// spare_sizes (never destroyed: a context may be closed after the statics are)
+std::mutex &spare_mu = *new std::mutex;
+std::set<Ctx *> &contexts = *new std::set<Ctx *>;
+
+void drop_spares_locked(Ctx *c) {
+    for (const Buffer &b : c->spares) (void)hipFree(b.ptr);
+    c->spares.clear();
+    c->spare_bytes = 0;
+}
+
+size_t spares_of_device(int device) {
+    size_t t = 0;
+    for (const Ctx *x : contexts)
+        if (x->device == device) t += x->spare_bytes;
+    return t;
+}
+
+}  // namespace
+
+hipError_t device_malloc(Ctx *c, void **p, size_t bytes) {
+    const hipError_t e = hipMalloc(p, bytes);
+    if (e == hipSuccess) return e;
+    std::lock_guard<std::mutex> lock(spare_mu);
+    if (spares_of_device(c->device) == 0) return e;
+    (void)hipGetLastError();
+    for (Ctx *x : contexts)
+        if (x->device == c->device) drop_spares_locked(x);
+    return hipMalloc(p, bytes);
+}
+
+// Whether the caller's device has no work left and room to spare.
+bool may_keep_blocks() {
+    size_t room = 0, total = 0;
+    if (hipDeviceSynchronize() == hipSuccess && hipMemGetInfo(&room, &total) == hipSuccess)
+        return room >= total / 16;
+    (void)hipGetLastError();  // refused, as during another thread's capture
+    return false;
+}
+
+void drop_spares(Ctx *c) {
+    std::lock_guard<std::mutex> lock(spare_mu);
+    drop_spares_locked(c);
+}
+
+// room for `bytes` more within the budget, without the spares if need be
+static void make_budget_room(Ctx *c, int64_t bytes) {
+    std::lock_guard<std::mutex> lock(spare_mu);
+    if (c->budget > 0 && c->used + (int64_t)c->spare_bytes + bytes > c->budget)
+        drop_spares_locked(c);
+}
+
 void *dev_alloc(Ctx *c, size_t bytes) {
     if (bytes == 0) bytes = 256;
-    if (c->budget > 0 && c->used + (int64_t)(c->spare_bytes + bytes) > c->budget) drop_spares(c);
+    make_budget_room(c, (int64_t)bytes);
     if (c->budget > 0 && c->used + (int64_t)bytes > c->budget)
         throw Error{APSPIE_ERR_BUDGET, "HBM budget exceeded: need " + std::to_string(bytes) +
                                            " more bytes, " + std::to_string(c->budget - c->used) +
@@ -122,40 +188,9 @@ void dev_free(Ctx *c, void *p, size_t bytes) {
     c->used -= (int64_t)bytes;
 }
 
-hipError_t device_malloc(Ctx *c, void **p, size_t bytes) {
-    hipError_t e = hipMalloc(p, bytes);
-    if (e != hipSuccess && c->spare_bytes) {
-        (void)hipGetLastError();
-        drop_spares(c);
-        e = hipMalloc(p, bytes);
-    }
-    return e;
-}
-
-// Freeing the 320 MB of an R-MAT-14 square took 0.48 ms, and 8 ms once a loop of
-// products had freed some 100 GB (the freed memory has to be cleared before it
-// can be given out); a block kept costs neither.  Blocks below 1 MB are not
-// worth keeping, and one is not given to a request below 8/9 of its size.  What
-// counts as used is the request, so that a call is refused where it would be with
-// arrays of its own; under a budget a block has to be of the request's size.
-constexpr size_t kSpareMin = (size_t)1 << 20, kSpareBytes = (size_t)512 << 20;
-
-bool device_idle() {
-    if (hipDeviceSynchronize() == hipSuccess) return true;
-    (void)hipGetLastError();  // refused, as during another thread's capture
-    return false;
-}
-
-void drop_spares(Ctx *c) {
-    std::lock_guard<std::mutex> lock(c->spare_mu);
-    for (const Buffer &b : c->spares) (void)hipFree(b.ptr);
-    c->spares.clear();
-    c->spare_bytes = 0;
-}
-
 void *graph_alloc(Ctx *c, size_t bytes) {
     if (bytes >= kSpareMin) {
-        std::lock_guard<std::mutex> lock(c->spare_mu);
+        std::lock_guard<std::mutex> lock(spare_mu);
         const size_t most = c->budget > 0 ? bytes : bytes + bytes / 8;
         auto best = c->spares.end();
         for (auto it = c->spares.begin(); it != c->spares.end(); ++it)
@@ -178,7 +213,7 @@ void *graph_alloc(Ctx *c, size_t bytes) {
 void graph_free(Ctx *c, void *p, size_t bytes, bool keep) {
     if (!p) return;
     {
-        std::lock_guard<std::mutex> lock(c->spare_mu);
+        std::lock_guard<std::mutex> lock(spare_mu);
         size_t block = bytes;
         const auto it = c->spare_sizes.find(p);
         if (it != c->spare_sizes.end()) {
@@ -186,7 +221,7 @@ void graph_free(Ctx *c, void *p, size_t bytes, bool keep) {
             c->spare_sizes.erase(it);
         }
         if (keep && block >= kSpareMin && block <= kSpareBytes) {
-            while (c->spare_bytes + block > kSpareBytes) {
+            while (!c->spares.empty() && spares_of_device(c->device) + block > kSpareBytes) {
                 (void)hipFree(c->spares.front().ptr);
                 c->spare_bytes -= c->spares.front().bytes;
                 c->spares.pop_front();
@@ -194,9 +229,10 @@ void graph_free(Ctx *c, void *p, size_t bytes, bool keep) {
             Buffer b;
             b.ptr = p;
             b.bytes = block;
-            bool kept = true;  // no exception leaves a destroy
-            try {
-                c->spares.push_back(b);
+            // (of the other contexts' blocks none is taken for this one)
+            bool kept = spares_of_device(c->device) + block <= kSpareBytes;
+            try {  // no exception leaves a destroy
+                if (kept) c->spares.push_back(b);
             } catch (...) {
                 kept = false;
             }
@@ -215,10 +251,10 @@ void graph_release(Ctx *c, Graph *g) {
     (void)hipSetDevice(c->device);
     // every stream, as hipFree waits: another context or the caller's own
     // stream may still read the arrays, and they are given out again
-    const bool idle = device_idle();
-    graph_free(c, g->rowptr, sizeof(int32_t) * (g->m + 1), idle);
-    graph_free(c, g->col, sizeof(int32_t) * g->nnz, idle);
-    graph_free(c, g->val, sizeof(float) * g->nnz, idle);
+    const bool keep = may_keep_blocks();
+    graph_free(c, g->rowptr, sizeof(int32_t) * (g->m + 1), keep);
+    graph_free(c, g->col, sizeof(int32_t) * g->nnz, keep);
+    graph_free(c, g->val, sizeof(float) * g->nnz, keep);
     g->rowptr = g->col = nullptr;
     g->val = nullptr;
 }
@@ -421,6 +457,8 @@ int apspie_ctx_create(int device, apspie_ctx **out) {
         APSPIE_HIP(hipHostMalloc(&c->progress, kProgressBytes,
                                  hipHostMallocMapped | hipHostMallocCoherent));
         noalloc_init(device);  // the no-alloc BFS's static array, once per device
+        std::lock_guard<std::mutex> lock(spare_mu);
+        contexts.insert(c);
     });
     if (st != APSPIE_OK) {
         delete c;
@@ -439,7 +477,11 @@ int apspie_ctx_destroy(apspie_ctx *c) {
     else
         for (auto &kv : c->scratch)
             if (kv.second.ptr) (void)hipFree(kv.second.ptr);
-    drop_spares(c);
+    {
+        std::lock_guard<std::mutex> lock(spare_mu);
+        drop_spares_locked(c);
+        contexts.erase(c);
+    }
     for (auto &p : c->timer_events) {
         (void)hipEventDestroy(p.first);
         (void)hipEventDestroy(p.second);
@@ -467,12 +509,12 @@ void *apspie_ctx_stream(apspie_ctx *c) { return c ? (void *)c->stream : nullptr;
 int apspie_ctx_set_hbm_budget(apspie_ctx *c, int64_t bytes) {
     if (!c || bytes < 0) return APSPIE_ERR_INVALID;
     (void)hipSetDevice(c->device);
-    if (bytes > 0 && c->used + (int64_t)c->spare_bytes > bytes) drop_spares(c);
     c->budget = bytes;
+    make_budget_room(c, 0);
     return APSPIE_OK;
 }
 
-int64_t apspie_ctx_hbm_used(apspie_ctx *c) { return c ? c->used : -1; }
+int64_t apspie_ctx_hbm_used(apspie_ctx *c) { return c ? c->used.load() : -1; }
 
 int apspie_ctx_set_option(apspie_ctx *c, const char *name, int64_t v) {
     if (!c || !name) return APSPIE_ERR_INVALID;

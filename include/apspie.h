@@ -99,7 +99,9 @@ int64_t apspie_ctx_hbm_used(apspie_ctx *ctx);
 int apspie_ctx_set_option(apspie_ctx *ctx, const char *name, int64_t value);
 int apspie_ctx_get_option(apspie_ctx *ctx, const char *name, int64_t *value);
 /* Release cached scratch memory (with an arena: mark it all free again) and the
- * arrays of destroyed graphs that are kept for the next ones (at most 512 MB). */
+ * arrays of destroyed graphs that it keeps for the next ones.  (All contexts of a
+ * device in the process keep at most 512 MB together, nothing while less than 1/16
+ * of the device's memory is free, and give it back when one of them runs short.) */
 int apspie_ctx_trim(apspie_ctx *ctx);
 /* Carve the context's scratch buffers out of one device block of `bytes`
  * (counted against the HBM budget) instead of one hipMalloc each: growing or

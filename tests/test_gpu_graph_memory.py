@@ -1,6 +1,7 @@
 """Arrays of destroyed graphs are kept for the next ones: the accounting, the
 budget and the results are those of arrays freed at once."""
 import ctypes as C
+import time
 
 import numpy as np
 import pytest
@@ -159,3 +160,45 @@ def test_larger_kept_blocks_do_not_narrow_a_budget():
             _check(g, csr)
             g.close()
             assert c.hbm_used() == 0
+
+
+def _free_bytes():
+    """Free device memory, by the runtime the library has loaded."""
+    free, total = C.c_size_t(), C.c_size_t()
+    assert C.CDLL("libamdhip64.so").hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+    return free.value
+
+
+def _settles(cond):
+    """The device returns freed memory after clearing it, a moment later."""
+    for _ in range(100):
+        if cond():
+            return True
+        time.sleep(0.02)
+    return False
+
+
+def test_kept_blocks_are_the_devices():
+    """All contexts of a device keep 512 MB together, and a request of one that
+    the device cannot serve takes back what another one keeps."""
+    csr = _csr(1_000_000, 40, 7)  # 320 MB
+    slack = 64 << 20
+    with A.Context(0) as a, A.Context(0) as b, A.Context(0) as c:
+        a.upload(*csr).close()
+        a.trim()
+        time.sleep(0.5)
+        before = _free_bytes()
+        for ctx in (a, b, c):
+            ctx.upload(*csr).close()
+        assert _settles(lambda: before - _free_bytes() < (512 << 20) + slack)
+        assert before - _free_bytes() > (200 << 20)
+        p = C.c_void_p()
+        assert A.lib().apspie_dev_alloc(c.h, C.c_int64(1 << 50), C.byref(p)) != 0
+        assert _settles(lambda: abs(before - _free_bytes()) < slack)
+        for ctx in (a, b, c):  # and the contexts go on
+            g = ctx.upload(*csr)
+            _check(g, csr)
+            g.close()
+        for ctx in (a, b, c):
+            ctx.trim()
+        assert _settles(lambda: abs(before - _free_bytes()) < slack)
