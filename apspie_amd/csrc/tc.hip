@@ -797,7 +797,7 @@ void tc_run(Ctx *c, const Graph *g0, uint64_t *total_out, int32_t *per_row) {
     c->stats.host_syncs++;
     *total_out = res[0];
     c->stats.edges_traversed = (int64_t)res[1];  // wedges probed
-    c->stats.vertices_reached = (int64_t)h[0] + h[1] + h[2] + h[3];
+    c->stats.vertices_reached = (int64_t)h[0] + h[1] + h[2] + h[3] + h[kTinyCount];
     c->stats.iterations = 1;
     kt.collect();
 }

@@ -39,3 +39,17 @@ def test_rows_at_tier_edges(m, lens):
             assert total == want and np.array_equal(rows, want_rows)
         assert ctx.tc(G, per_row=False)[0] == want
         G.close()
+
+
+@pytest.mark.parametrize("key", ["lattice", "rmat"])
+def test_rows_counted(key):
+    """vertices_reached is the number of rows with two lower neighbours or
+    more, whichever kernel takes them."""
+    rp, c = A.gen_lattice(60) if key == "lattice" else A.gen_rmat(12)
+    rows = np.repeat(np.arange(len(rp) - 1), np.diff(rp))
+    lower = np.bincount(rows[c < rows], minlength=len(rp) - 1)
+    with A.Context(0) as ctx:
+        G = ctx.upload(rp, c)
+        ctx.tc(G)
+        assert ctx.stats()["vertices_reached"] == int((lower >= 2).sum())
+        G.close()
