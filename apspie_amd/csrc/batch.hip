@@ -1077,14 +1077,21 @@ __global__ __launch_bounds__(256) void k_batch_depths(
     }
 }
 
-// One batched traversal pass for up to 32*W sources.
+// Width of a batch's near-far rounds (0: Bellman-Ford rounds): the option
+// batch_sssp_delta, at -1 chosen per graph.
+double sssp_batch_delta(Ctx *c, const Graph *g) {
+    const double d = (double)opt(c, "batch_sssp_delta", -1);
+    return d < 0 ? sssp_batch_auto_delta(c, const_cast<Graph *>(g)) : d;
+}
+
 // near-far rounds of a batch may pull (and keep their distances source-major)
 bool sssp_rounds_pull(Ctx *c, const Graph *g) {
-    return opt(c, "batch_sssp_pull_div", 4) > 0 &&
+    return sssp_batch_delta(c, g) > 0 && opt(c, "batch_sssp_pull_div", 4) > 0 &&
            graph_max_degree(c, const_cast<Graph *>(g)) <= 64 &&
            graph_is_symmetric_weighted(c, const_cast<Graph *>(g));
 }
 
+// One batched traversal pass for up to 32*W sources.
 template <int W, bool SSSP>
 void batch_pass(Ctx *c, const Graph *g, const int32_t *src_host, int32_t nsrc, int32_t *depth_out,
                 float *dist_out) {
@@ -1132,13 +1139,12 @@ void batch_pass(Ctx *c, const Graph *g, const int32_t *src_host, int32_t nsrc, i
     APSPIE_HIP(hipMemcpyAsync(ulist, uniq.data(), sizeof(int32_t) * uniq.size(),
                               hipMemcpyHostToDevice, c->stream));
     const int grid = fill_grid(c, kBlock, (int)opt(c, "batch_blocks_per_cu", 4));
-    // near-far rounds for SSSP (threshold step batch_sssp_delta, 0 = off,
-    // -1 = chosen per graph; passes of up to 128 sources take twice that
-    // width: fewer rounds, whose fixed cost weighs more on a narrow row --
-    // 2048^2 lattice, 32 / 64 / 128 sources: 0.876 -> 0.829 / 0.705 -> 0.682
-    // / 0.625 -> 0.616 ms per query; 512 sources 0.596 -> 0.603)
-    double bdelta = SSSP ? (double)opt(c, "batch_sssp_delta", -1) : 0;
-    if (bdelta < 0) bdelta = sssp_batch_auto_delta(c, const_cast<Graph *>(g)) * (W <= 4 ? 2 : 1);
+    // near-far rounds for SSSP; where the width is chosen per graph, passes of up
+    // to 128 sources take twice it: fewer rounds, whose fixed cost weighs more on
+    // a narrow row -- 2048^2 lattice, 32 / 64 / 128 sources: 0.876 -> 0.829 /
+    // 0.705 -> 0.682 / 0.625 -> 0.616 ms per query; 512 sources 0.596 -> 0.603
+    double bdelta = SSSP ? sssp_batch_delta(c, g) : 0;
+    if (SSSP && W <= 4 && opt(c, "batch_sssp_delta", -1) < 0) bdelta *= 2;
     const float delta = (float)bdelta;
     const bool near_far = SSSP && delta > 0;
     uint32_t *pend =
@@ -1165,7 +1171,7 @@ void batch_pass(Ctx *c, const Graph *g, const int32_t *src_host, int32_t nsrc, i
     // lattice, 32 / 64 sources: 0.94 -> 0.88 / 0.73 -> 0.71 ms per query;
     // 128 sources are best at the option's 4)
     const int32_t sssp_pull_div =
-        near_far && sssp_rounds_pull(c, g)
+        SSSP && sssp_rounds_pull(c, g)
             ? (int32_t)std::min<int64_t>(opt(c, "batch_sssp_pull_div", 4) * (W <= 2 ? 2 : 1),
                                          1 << 22)
             : 0;
@@ -1327,8 +1333,8 @@ void batch_run(Ctx *c, const Graph *g, const int32_t *src, int32_t nsrc, int32_t
     // ms per query in groups of 512 / 256 / 128: 2048^2 lattice 0.652 / 0.553 /
     // 0.508, 1024^2 0.167 / 0.150 / 0.151).  On smaller graphs the rounds' fixed
     // cost weighs more (724^2 0.067 / 0.071 / 0.077, 512^2 0.040 / 0.044 / 0.057)
-    if (SSSP && nsrc > kSourceMajorGroup && g->m >= kSourceMajorFrom &&
-        opt(c, "batch_sssp_delta", -1) != 0 && sssp_rounds_pull(c, g))
+    // (and Bellman-Ford batches, which are never source-major, stay whole)
+    if (SSSP && nsrc > kSourceMajorGroup && g->m >= kSourceMajorFrom && sssp_rounds_pull(c, g))
         group = kSourceMajorGroup;
     for (int32_t s0 = 0; s0 < nsrc; s0 += group) {
         const int32_t k = std::min(group, nsrc - s0);

@@ -115,3 +115,28 @@ def test_groups_of_a_large_graph(nsrc):
         for i in {0, 1, 127, nsrc - 1, min(128, nsrc - 1), min(256, nsrc - 1)}:
             assert np.array_equal(got[i], c.sssp(G, int(src[i])))
         G.close()
+
+
+@pytest.mark.parametrize("hi", [1, 255])
+def test_only_near_far_batches_are_grouped(hi):
+    """Equal weights mean Bellman-Ford rounds: a batch then stays one pass, and
+    300 copies of a source expand what the source alone does.  With weights
+    1..255 the batch is split in three."""
+    w, nsrc = 1024, 300
+    ids = np.arange(w * w).reshape(w, w)
+    u = np.concatenate([ids[:, :-1].ravel(), ids[:-1].ravel()]).astype(np.int32)
+    v = np.concatenate([ids[:, 1:].ravel(), ids[1:].ravel()]).astype(np.int32)
+    val = np.random.default_rng(1).integers(1, hi + 1, len(u)).astype(np.float32)
+    src = int(ids[w // 2, w // 2])
+    with A.Context(0) as c:
+        G = c.from_coo(w * w, u, v, val)
+        out = c.dev_alloc(4 * nsrc * w * w)
+        c.sssp_batch(G, [src], out=out.ptr, mem=A.DEVICE)
+        alone = c.stats()["vertices_reached"]
+        c.sssp_batch(G, [src] * nsrc, out=out.ptr, mem=A.DEVICE)
+        if hi == 1:
+            assert alone == w * w and c.stats()["vertices_reached"] == alone
+        else:
+            assert c.stats()["vertices_reached"] > 2 * alone
+        out.free()
+        G.close()
