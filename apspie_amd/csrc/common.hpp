@@ -139,6 +139,9 @@ int64_t opt(Ctx *c, const char *name, int64_t dflt);
 
 // Scratch buffer by name, grown on demand (contents not preserved on growth).
 void *scratch(Ctx *c, const std::string &name, size_t bytes);
+// Bytes of a scratch buffer as it stands, and its memory given back.
+size_t scratch_held(Ctx *c, const std::string &name);
+void scratch_drop(Ctx *c, const std::string &name);
 // Bytes a new scratch buffer could still take: the largest free range of the
 // arena, else what the HBM budget leaves (INT64_MAX without either).
 int64_t scratch_room(Ctx *c);

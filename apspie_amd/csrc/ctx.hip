@@ -307,19 +307,28 @@ void drop_scratch(Ctx *c) {
 
 }  // namespace
 
+size_t scratch_held(Ctx *c, const std::string &name) {
+    const auto it = c->scratch.find(name);
+    return it == c->scratch.end() || !it->second.ptr ? 0 : it->second.bytes;
+}
+
+void scratch_drop(Ctx *c, const std::string &name) {
+    const auto it = c->scratch.find(name);
+    if (it == c->scratch.end() || !it->second.ptr) return;
+    Buffer &b = it->second;
+    // pending work may still read the buffer
+    sync(c);
+    if (c->arena)
+        arena_give(c, b.ptr, b.bytes);
+    else
+        dev_free(c, b.ptr, b.bytes);
+    b = Buffer{};
+}
+
 void *scratch(Ctx *c, const std::string &name, size_t bytes) {
     Buffer &b = c->scratch[name];
     if (b.bytes >= bytes && b.ptr) return b.ptr;
-    if (b.ptr) {
-        // pending work may still read the old buffer
-        sync(c);
-        if (c->arena)
-            arena_give(c, b.ptr, b.bytes);
-        else
-            dev_free(c, b.ptr, b.bytes);
-        b.ptr = nullptr;
-        b.bytes = 0;
-    }
+    scratch_drop(c, name);
     if (c->arena) {
         const size_t want = granules(bytes);
         b.ptr = arena_take(c, want);

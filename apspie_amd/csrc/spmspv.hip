@@ -493,21 +493,14 @@ float host_identity(int sr) {
     }
 }
 
-}  // namespace
+size_t dense_bytes(const Graph *g) { return sizeof(float) * (size_t)g->n; }
 
-int64_t spmspv_run(Ctx *c, const Graph *g, int sr, int64_t nx, const int32_t *x_ind,
-                   const float *x_val, const int32_t *mask, int32_t *y_ind, float *y_val,
-                   int path) {
-    if (nx == 0 || g->nnz == 0) {
-        c->stats.iterations = 1;
-        return 0;
-    }
-    if (path == APSPIE_PATH_AUTO) path = (int)opt(c, "spmspv_path", 0);
-    SpvPath sp{opt(c, "spmspv_sort_max", 1 << 16), 0, 0};
-    if (path == APSPIE_PATH_SORT) sp.all_sort = 1;
-    else if (path != APSPIE_PATH_AUTO) sp.sort_max = -1;
+// One call, with the atomic path's dense row at hand (dense) or got when the edge
+// count asks for it, after a round trip.
+int64_t spmspv_call(Ctx *c, const Graph *g, int sr, int64_t nx, const int32_t *x_ind,
+                    const float *x_val, const int32_t *mask, int32_t *y_ind, float *y_val,
+                    SpvPath sp, bool dense) {
     const int64_t n = g->n, words = n / 32 + 1;
-    bool dense = !sp.all_sort;
     const int64_t gtiles = ceil_div(nx, kGatherTile), ftiles = ceil_div((n + 31) / 32, kBlock);
     FrontierBufs f;
     f.v = (int32_t *)scratch(c, "spv_v", sizeof(int32_t) * nx);
@@ -516,17 +509,10 @@ int64_t spmspv_run(Ctx *c, const Graph *g, int sr, int64_t nx, const int32_t *x_
     float *yd = nullptr;
     uint32_t *touched = nullptr;
     auto dense_row = [&] {
-        yd = (float *)scratch(c, "spv_dense", sizeof(float) * n);
+        yd = (float *)scratch(c, "spv_dense", dense_bytes(g));
         touched = (uint32_t *)scratch(c, "spv_touched", sizeof(uint32_t) * words);
     };
-    if (dense) {
-        try {
-            dense_row();
-        } catch (const Error &) {  // a call that turns out to sort needs no dense row
-            if (path != APSPIE_PATH_AUTO) throw;
-            dense = false;
-        }
-    }
+    if (dense) dense_row();
     const int64_t nctl = sizeof(SpvCtl) / 8 + 2 * gtiles + std::max<int64_t>(ftiles, 1);
     SpvCtl *ctl = (SpvCtl *)scratch(c, "spv_ctl", sizeof(uint64_t) * nctl);
     uint64_t *st = (uint64_t *)(ctl + 1), *st_fin = st + 2 * gtiles;
@@ -601,6 +587,38 @@ int64_t spmspv_run(Ctx *c, const Graph *g, int sr, int64_t nx, const int32_t *x_
     APSPIE_HIP(hipEventSynchronize(c->ev1));
     c->ev1_recorded = true;
     return (int64_t)h[2];
+}
+
+}  // namespace
+
+int64_t spmspv_run(Ctx *c, const Graph *g, int sr, int64_t nx, const int32_t *x_ind,
+                   const float *x_val, const int32_t *mask, int32_t *y_ind, float *y_val,
+                   int path) {
+    if (nx == 0 || g->nnz == 0) {
+        c->stats.iterations = 1;
+        return 0;
+    }
+    if (path == APSPIE_PATH_AUTO) path = (int)opt(c, "spmspv_path", 0);
+    SpvPath sp{opt(c, "spmspv_sort_max", 1 << 16), 0, 0};
+    if (path == APSPIE_PATH_SORT) sp.all_sort = 1;
+    else if (path != APSPIE_PATH_AUTO) sp.sort_max = -1;
+    auto call = [&](bool dense) {
+        return spmspv_call(c, g, sr, nx, x_ind, x_val, mask, y_ind, y_val, sp, dense);
+    };
+    if (path != APSPIE_PATH_AUTO) return call(!sp.all_sort);
+    // A call that may turn out to sort takes the dense row beforehand only where
+    // its memory is nobody else's loss: the context has it already, or has neither
+    // a budget nor an arena and the device is not full.
+    if ((c->budget > 0 || c->arena) && scratch_held(c, "spv_dense") < dense_bytes(g))
+        return call(false);
+    try {
+        return call(true);
+    } catch (const Error &e) {
+        if (e.status != APSPIE_ERR_OOM && e.status != APSPIE_ERR_BUDGET) throw;
+    }
+    scratch_drop(c, "spv_dense");
+    scratch_drop(c, "spv_touched");
+    return call(false);
 }
 
 // Dense mXv (mXv.cuh:110-247): the entries of x above 0.5 (bitify,

@@ -81,3 +81,35 @@ def test_scratch_without_room_for_a_dense_row(thin):
             ctx.spmspv(G, A.SR_PLUS_TIMES, np.arange(66_000, dtype=np.int32))
         assert e.value.status == -4
         G.close()
+
+
+def test_a_sorting_call_leaves_a_budget_alone(thin):
+    """Under a budget with room for the dense row, a call that sorts does not
+    take it: what fitted beside it before still does.  A call that needs the row
+    gets it, and those after it find it there."""
+    rp, col, a = thin
+    rng = np.random.default_rng(5)
+    x = np.sort(rng.choice(ROWS, 50, replace=False))
+    xv = rng.random(len(x)).astype(np.float32)
+    every = np.arange(ROWS, dtype=np.int32)
+    with A.Context(0) as ctx:
+        G = ctx.upload(rp.astype(np.int32), col, a)
+        ctx.spmspv(G, A.SR_BOOL, every, path=A.PATH_SORT)  # every other buffer
+        want = ctx.spmspv(G, A.SR_PLUS_TIMES, x, xv, path=A.PATH_SORT)
+        used = ctx.hbm_used()
+        ctx.set_hbm_budget(used + 5 * N)
+        for _ in range(2):
+            got = ctx.spmspv(G, A.SR_PLUS_TIMES, x, xv)
+            assert np.array_equal(got[0], want[0]) and np.array_equal(got[1], want[1])
+            assert ctx.hbm_used() < used + N
+        H = ctx.upload(np.arange(N + 1, dtype=np.int32) // 8, np.zeros(N // 8, np.int32))
+        H.close()
+        ctx.set_hbm_budget(used + 5 * N)
+        for _ in range(2):
+            yi, yv = ctx.spmspv(G, A.SR_MIN_PLUS, every, None)
+            wi, wv = O.spmspv(N, rp, col, a, A.SR_MIN_PLUS, every, np.ones(ROWS, np.float32), None)
+            assert np.array_equal(yi, wi) and np.array_equal(yv, wv)
+            assert ctx.hbm_used() > used + 4 * N
+        got = ctx.spmspv(G, A.SR_PLUS_TIMES, x, xv)
+        assert np.array_equal(got[0], want[0]) and np.array_equal(got[1], want[1])
+        G.close()
