@@ -230,7 +230,7 @@ __device__ __forceinline__ int32_t load_relaxed(const int32_t *p) {
 // ------------------------------------------------------- chained tiles
 // Exclusive prefix over tiles by decoupled look-back.  One status word per
 // tile, zero before the launch: bits 62-63 = 0 nothing, 1 aggregate, 2
-// inclusive prefix; bits 0-61 = value.  A tile's id must come from a ticket
+// inclusive prefix; bits 0-61 = value (signed).  A tile's id must come from a ticket
 // counter in launch order, so that every tile a block waits on belongs to a
 // block that started earlier and never waits on a later one: every wait
 // ends.  A tile looks back with a whole wave, 64 status words at a time: one
@@ -267,7 +267,7 @@ __device__ __forceinline__ uint64_t chain_tiles(uint64_t *status, int64_t tile, 
         }
     }
     if (lane_id() == 0) tile_post(status + tile, kTilePre | ((prefix + agg) & kTileVal));
-    return prefix;
+    return (uint64_t)((int64_t)(prefix << 2) >> 2);  // the value's sign bit is bit 61
 }
 
 // float <-> order-preserving int for non-negative floats (distances >= 0)

@@ -91,3 +91,16 @@ def test_build_refuses_an_index_out_of_range(ctx):
         for sym in (True, False):
             with pytest.raises(A.ApspieError):
                 ctx.from_coo(5, [1, r, 2], [2, c, 3], symmetrize=sym)
+
+
+@pytest.mark.parametrize("n", [1, 1024, 1025, 2048, 5000, 65_536, 65_537, 400_001])
+@pytest.mark.parametrize("lo,hi", [(-100, 0), (-100, 100), (-(1 << 31), -(1 << 30))])
+def test_scan_of_negative_values(n, lo, hi):
+    """Prefixes that are negative at a tile's edge: the 64-bit total and the
+    low words of the prefixes."""
+    x = np.random.default_rng(n).integers(lo, hi, n).astype(np.int32)
+    want = np.cumsum(x, dtype=np.int64)
+    with A.Context(0) as ctx:
+        out, total = ctx.scan_exclusive(x)
+        assert total == want[-1]
+        assert np.array_equal(out, np.concatenate([[0], want[:-1]]).astype(np.int32))
