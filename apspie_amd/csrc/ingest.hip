@@ -185,7 +185,7 @@ __global__ void k_entry_rows(const int32_t *rowptr, int32_t m, int64_t nnz, int3
          e += (int64_t)gridDim.x * blockDim.x) {
         int32_t lo = 0, hi = m;  // largest r with rowptr[r] <= e
         while (hi - lo > 1) {
-            const int32_t mid = (lo + hi) >> 1;
+            const int32_t mid = lo + ((hi - lo) >> 1);  // lo + hi can pass 2^31
             if (rowptr[mid] <= e) lo = mid; else hi = mid;
         }
         rows[e] = lo;
@@ -345,7 +345,7 @@ __global__ void k_check_mirror_values(const int32_t *rowptr, const int32_t *col,
             const int32_t v = col[e];
             int32_t lo = rowptr[v], hi = rowptr[v + 1];  // first entry of row v not below r
             while (lo < hi) {
-                const int32_t mid = (lo + hi) >> 1;
+                const int32_t mid = lo + ((hi - lo) >> 1);  // lo + hi can pass 2^31
                 if (col[mid] < r) lo = mid + 1; else hi = mid;
             }
             if (lo >= rowptr[v + 1] || col[lo] != r ||

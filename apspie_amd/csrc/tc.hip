@@ -50,7 +50,7 @@ __global__ void k_lowcnt(const int32_t *rowptr, const int32_t *col, int32_t m, i
         int32_t lo = rowptr[r], hi = rowptr[r + 1];
         const int32_t b = lo;
         while (lo < hi) {
-            const int32_t mid = (lo + hi) >> 1;
+            const int32_t mid = lo + ((hi - lo) >> 1);  // lo + hi can pass 2^31
             if (col[mid] < (int32_t)r) lo = mid + 1; else hi = mid;
         }
         lowcnt[r] = lo - b;
