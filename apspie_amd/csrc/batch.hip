@@ -218,7 +218,7 @@ __device__ __noinline__ dev::Pair32 pull_long(const LongRows &q, uint32_t nl,
     dev::Pair32 found{0, 0};
     for (uint32_t j = wave; j < nl; j += nwaves) {
         const int64_t v = q.v[j];
-        const int32_t rs = rowptr[v], re = rowptr[v + 1];
+        const uint32_t rs = rowptr[v], re = rowptr[v + 1];  // (a step can pass 2^31)
         uint32_t uv[W], acc[W];
         load_row<W>(vis + v * W, uv);
 #pragma unroll
@@ -226,10 +226,10 @@ __device__ __noinline__ dev::Pair32 pull_long(const LongRows &q, uint32_t nl,
             uv[w] = ~uv[w];
             acc[w] = 0;
         }
-        for (int32_t base = rs; base < re; base += kLongStep) {
+        for (uint32_t base = rs; base < re; base += kLongStep) {
 #pragma unroll
             for (int t = 0; t < kLongStep / 64; ++t) {
-                const int32_t e = base + t * 64 + lane;
+                const uint32_t e = base + t * 64 + lane;
                 if (e < re) {
                     uint32_t f[W];
                     load_row<W>(front + (int64_t)col[e] * W, f);
@@ -306,7 +306,7 @@ __device__ __forceinline__ void batch_pull(PullLds<LONG> &lds, const int32_t *__
     dev::Pair32 found{0, 0};
     for (int64_t pbase = (int64_t)blockIdx.x * VPB * KP; pbase < m;
          pbase += (int64_t)gridDim.x * VPB * KP) {
-        int32_t rs[KP], re[KP];
+        uint32_t rs[KP], re[KP];  // (a step past a row's end can pass 2^31)
         uint32_t uv[KP], acc[KP];
 #pragma unroll
         for (int k = 0; k < KP; ++k) {
@@ -350,7 +350,7 @@ __device__ __forceinline__ void batch_pull(PullLds<LONG> &lds, const int32_t *__
                     }
                 }
             }
-            for (int32_t e = rs[k] + Q; e < re[k] && (acc[k] & uv[k]) != uv[k]; e += Q) {
+            for (uint32_t e = rs[k] + Q; e < re[k] && (acc[k] & uv[k]) != uv[k]; e += Q) {
                 int32_t uu[Q];
 #pragma unroll
                 for (int t = 0; t < Q; ++t) uu[t] = e + t < re[k] ? col[e + t] : -1;
@@ -710,12 +710,12 @@ __device__ __forceinline__ void batch_sssp_pull(PullQueue &q, const int32_t *__r
             crs[k] = 0;
             cd[k] = 0;
             uint32_t near = 0, far = 0;
-            int32_t rs = 0, re = 0;
+            uint32_t rs = 0, re = 0;  // (a step past a row's end can pass 2^31)
             if (v < m) {
                 rs = rowptr[v];
                 re = rowptr[v + 1];
                 int32_t *dv_row = op.word_of(v, w);
-                for (int32_t e0 = rs; e0 < re; e0 += Q) {
+                for (uint32_t e0 = rs; e0 < re; e0 += Q) {
                     int32_t u[Q];
                     uint32_t f[Q], x = 0;
                     float we[Q];

@@ -265,7 +265,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(8))) voi
         for (int k = 0; k < kPullPer; ++k)
             if (open[k] && !hit[k] && re[k] - rs[k] > 1) pend |= 1u << k;
         {
-            int32_t e = 0, lim = 0, rend = 0;
+            int32_t e = 0, lim = 0, rend = 0;  // (e + kPullIlp can pass 2^31)
             uint32_t kbit = 0;
             for (;;) {
                 if (e >= lim) {
@@ -281,11 +281,11 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(8))) voi
                             rend = re[k];
                         }
                     e = r0 + 1;
-                    lim = min(rend, r0 + kPullLight);
+                    lim = r0 + min(rend - r0, kPullLight);
                 }
                 int32_t u[kPullIlp];
 #pragma unroll
-                for (int q = 0; q < kPullIlp; ++q) u[q] = e + q < lim ? col[e + q] : -1;
+                for (int q = 0; q < kPullIlp; ++q) u[q] = q < lim - e ? col[e + q] : -1;
                 uint32_t f[kPullIlp];
 #pragma unroll
                 for (int q = 0; q < kPullIlp; ++q)
@@ -299,8 +299,9 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(8))) voi
                     scanned += (uint64_t)(at + 1);
                     e = lim;
                 } else {
-                    scanned += (uint64_t)min(kPullIlp, lim - e);
-                    e += kPullIlp;
+                    const int32_t n = min(kPullIlp, lim - e);
+                    scanned += (uint64_t)n;
+                    e += n;
                     if (e >= lim && lim < rend) longm |= kbit;
                 }
             }
@@ -311,15 +312,15 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(8))) voi
         // row 64 entries at a time, coalesced, stopping at the first hit
 #pragma unroll
         for (int k = 0; k < kPullPer; ++k) {
-            const int32_t lim = min(re[k], rs[k] + kPullLight);
+            const int32_t lim = rs[k] + min(re[k] - rs[k], kPullLight);
             uint64_t heavy = __ballot((longm >> k) & 1u);
             while (heavy) {
                 const int h = __ffsll((unsigned long long)heavy) - 1;
                 heavy &= heavy - 1;
-                const int32_t hrs = __shfl(lim, h, 64), hre = __shfl(re[k], h, 64);
+                const uint32_t hrs = __shfl(lim, h, 64), hre = __shfl(re[k], h, 64);
                 bool found = false;
-                for (int32_t e0 = hrs; e0 < hre; e0 += 64) {
-                    const int32_t e = e0 + lane;
+                for (uint32_t e0 = hrs; e0 < hre; e0 += 64) {
+                    const uint32_t e = e0 + lane;
                     bool f = false;
                     if (e < hre) {
                         const int32_t u = col[e];

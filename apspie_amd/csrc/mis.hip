@@ -102,7 +102,8 @@ __global__ __launch_bounds__(kBlock) void k_mis_lose(const int32_t *__restrict__
         __syncthreads();
         const int64_t j = base + threadIdx.x;
         if (j < F) {
-            const int32_t u = cur.v[j], rs = cur.start[j], re = rowptr[u + 1];
+            const int32_t u = cur.v[j];
+            const uint32_t rs = cur.start[j], re = rowptr[u + 1];  // (rs + t can pass 2^31)
             const uint64_t ku = live[u];
             int32_t c[kLoseQ];
 #pragma unroll
@@ -122,14 +123,15 @@ __global__ __launch_bounds__(kBlock) void k_mis_lose(const int32_t *__restrict__
         __syncthreads();
         const int32_t n = s_n;
         for (int32_t q = wave; q < n; q += kBlock / 64) {
-            const int32_t u = s_u[q], re = s_end[q];
+            const int32_t u = s_u[q];
+            const uint32_t re = s_end[q];
             const uint64_t ku = live[u];
             bool lost = false;
-            for (int32_t e0 = s_e[q]; e0 < re && !lost; e0 += kLoseStep) {
+            for (uint32_t e0 = s_e[q]; e0 < re && !lost; e0 += kLoseStep) {
                 bool mine = false;
 #pragma unroll
                 for (int t = 0; t < kLoseStep / 64; ++t) {
-                    const int32_t e = e0 + t * 64 + lane;
+                    const uint32_t e = e0 + t * 64 + lane;
                     if (e < re && live[col[e]] > ku) mine = true;
                 }
                 lost = __ballot(mine) != 0;

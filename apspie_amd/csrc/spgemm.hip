@@ -67,11 +67,12 @@ __global__ __launch_bounds__(kBlock) void k_row_bound(const int32_t *__restrict_
     const int64_t i0 = (int64_t)blockIdx.x * (kBlock / 16) + threadIdx.x / 64 * 4;
     for (int64_t w = i0; w < m; w += step) {  // the wave's first row
         const int64_t i = w + (threadIdx.x / 16 & 3);
-        const int32_t b = i < m ? arp[i] : 0, e1 = i < m ? arp[i + 1] : 0;
+        // (unsigned: a step past a row's end can pass 2^31)
+        const uint32_t b = i < m ? arp[i] : 0, e1 = i < m ? arp[i + 1] : 0;
         const bool is_long = e1 - b > kBoundRow;
         uint64_t s = 0;
         if (!is_long)
-            for (int32_t e = b + j; e < e1; e += 16) {
+            for (uint32_t e = b + j; e < e1; e += 16) {
                 const int32_t k = acol[e];
                 s += (uint64_t)(brp[k + 1] - brp[k]);
             }
@@ -80,10 +81,10 @@ __global__ __launch_bounds__(kBlock) void k_row_bound(const int32_t *__restrict_
         if (j == 0 && i < m && !is_long) prods[i] = (int64_t)s;
         for (uint64_t todo = __ballot(is_long && j == 0); todo; todo &= todo - 1) {
             const int src = __ffsll((unsigned long long)todo) - 1;
-            const int32_t lb = __shfl(b, src, 64), le = __shfl(e1, src, 64);
+            const uint32_t lb = __shfl(b, src, 64), le = __shfl(e1, src, 64);
             uint64_t t = 0;
 #pragma unroll 8
-            for (int32_t e = lb + dev::lane_id(); e < le; e += 64) {
+            for (uint32_t e = lb + dev::lane_id(); e < le; e += 64) {
                 const int32_t k = acol[e];
                 t += (uint64_t)(brp[k + 1] - brp[k]);
             }
@@ -299,8 +300,8 @@ __device__ __forceinline__ void wave_row(int32_t r, const int32_t *arp, const in
     }
     dev::wave_sync();
     uint32_t created = 0;
-    const int32_t a1 = arp[r + 1];
-    for (int32_t e0 = arp[r]; e0 < a1; e0 += 64) {
+    const uint32_t a1 = arp[r + 1];  // (a step past the row's end can pass 2^31)
+    for (uint32_t e0 = arp[r]; e0 < a1; e0 += 64) {
         int32_t b0 = 0;
         uint32_t len = 0;
         float av = 1.0f;
@@ -403,18 +404,18 @@ struct Entry {
 // product is applied.
 template <int RUN, class F>
 __device__ __forceinline__ void wave_products(const int32_t *pre, const Entry *ent, int cn,
-                                              int32_t w0, int32_t W,
+                                              uint32_t w0, uint32_t W,  // W < 2^31
                                               const int32_t *__restrict__ bcol,
                                               const float *__restrict__ bval, F &&f) {
-    const int jl = __builtin_amdgcn_readfirstlane(wave_find(pre, cn, w0));
-    const int jh =
-        __builtin_amdgcn_readfirstlane(wave_find(pre, cn, min(w0 + 64 * RUN, W) - 1));
+    const int jl = __builtin_amdgcn_readfirstlane(wave_find(pre, cn, (int32_t)w0));
+    const int jh = __builtin_amdgcn_readfirstlane(
+        wave_find(pre, cn, (int32_t)(min(w0 + 64 * RUN, W) - 1)));
     int32_t x[RUN], key[RUN];
     int j[RUN];
     float a[RUN], b[RUN];
 #pragma unroll
     for (int q = 0; q < RUN; ++q) {
-        x[q] = min(w0 + q * 64 + dev::lane_id(), W - 1);
+        x[q] = (int32_t)min(w0 + q * 64 + dev::lane_id(), W - 1);
         j[q] = jl;
     }
     // the slices' searches side by side: a step is one LDS round trip for all
@@ -448,8 +449,8 @@ __device__ __forceinline__ void for_products(int32_t r, const int32_t *arp, cons
                                              int32_t *pre, Entry *ent, uint64_t *s_scan,
                                              F &&f) {
     const int32_t ab = arp[r], an = arp[r + 1] - ab;
-    for (int32_t c0 = 0; c0 < an; c0 += kChunk) {
-        const int32_t cn = min(kChunk, an - c0);
+    for (uint32_t c0 = 0; c0 < (uint32_t)an; c0 += kChunk) {
+        const int32_t cn = min(kChunk, an - (int32_t)c0);
         uint32_t carry = 0;
         for (int32_t x0 = 0; x0 < cn; x0 += BLOCK) {
             const int32_t x = x0 + threadIdx.x;
@@ -472,17 +473,16 @@ __device__ __forceinline__ void for_products(int32_t r, const int32_t *arp, cons
         }
         if (threadIdx.x == 0) pre[cn] = (int32_t)carry;
         __syncthreads();
-        const int32_t W = (int32_t)carry;
-        const int32_t wave = threadIdx.x / 64;
+        const uint32_t W = carry, wave = threadIdx.x / 64;
         // a chunk that does not give every wave half a run goes out in slices
         if (W >= BLOCK * RUN / 2) {
-            for (int32_t w0 = wave * 64 * RUN; w0 < W; w0 += BLOCK * RUN)
+            for (uint32_t w0 = wave * 64 * RUN; w0 < W; w0 += BLOCK * RUN)
                 wave_products<RUN>(pre, ent, cn, w0, W, bcol, bval, f);
         } else if (RUN > 4 && W >= BLOCK * 2) {
-            for (int32_t w0 = wave * 64 * 4; w0 < W; w0 += BLOCK * 4)
+            for (uint32_t w0 = wave * 64 * 4; w0 < W; w0 += BLOCK * 4)
                 wave_products<4>(pre, ent, cn, w0, W, bcol, bval, f);
         } else {
-            for (int32_t w0 = wave * 64; w0 < W; w0 += BLOCK)
+            for (uint32_t w0 = wave * 64; w0 < W; w0 += BLOCK)
                 wave_products<1>(pre, ent, cn, w0, W, bcol, bval, f);
         }
         __syncthreads();  // pre / ent are refilled by the next chunk

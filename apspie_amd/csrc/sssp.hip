@@ -193,7 +193,7 @@ k_sssp_do_round(const int32_t *__restrict__ rowptr, const int32_t *__restrict__ 
         }
         // each lane walks its short rows one after another, kDoIlp loads in flight
         {
-            int32_t e = 0, lim = 0, kk = -1, bk = 0;
+            int32_t e = 0, lim = 0, kk = -1, bk = 0;  // (e + kDoIlp can pass 2^31)
             for (;;) {
                 if (e >= lim) {
                     if (kk >= 0) {
@@ -214,7 +214,7 @@ k_sssp_do_round(const int32_t *__restrict__ rowptr, const int32_t *__restrict__ 
                 }
                 int32_t u[kDoIlp];
 #pragma unroll
-                for (int q = 0; q < kDoIlp; ++q) u[q] = e + q < lim ? col[e + q] : -1;
+                for (int q = 0; q < kDoIlp; ++q) u[q] = q < lim - e ? col[e + q] : -1;
                 bool f[kDoIlp];
 #pragma unroll
                 for (int q = 0; q < kDoIlp; ++q)
@@ -222,7 +222,7 @@ k_sssp_do_round(const int32_t *__restrict__ rowptr, const int32_t *__restrict__ 
 #pragma unroll
                 for (int q = 0; q < kDoIlp; ++q)
                     if (f[q]) bk = min(bk, dev::fbits(dev::bitsf(dist[u[q]]) + w[e + q]));
-                e += kDoIlp;
+                e += min(kDoIlp, lim - e);
             }
         }
         int32_t pc[kDoPer], prs[kDoPer], pcd[kDoPer];
@@ -247,7 +247,7 @@ k_sssp_do_round(const int32_t *__restrict__ rowptr, const int32_t *__restrict__ 
     const int32_t HF = (int32_t)cnt_entries(heavy_cnt), HE = (int32_t)cnt_edges(heavy_cnt);
     if (HF == 0) return;
     HeavyLds &L = lds.hv;
-    const int32_t ntiles = (HE + kHvTile - 1) / kHvTile;
+    const int32_t ntiles = (int32_t)(((int64_t)HE + kHvTile - 1) / kHvTile);
     for (int32_t t = blockIdx.x; t < ntiles; t += gridDim.x) {
         const int32_t i0 = min(max(heavy.tfirst[t], 0), HF - 1);
         const int32_t i1 = (t + 1 < ntiles) ? min(max(heavy.tfirst[t + 1], i0), HF - 1) : HF - 1;
@@ -262,17 +262,17 @@ k_sssp_do_round(const int32_t *__restrict__ rowptr, const int32_t *__restrict__ 
             }
         }
         __syncthreads();
-        const int32_t x0 = t * kHvTile + threadIdx.x * kHvPer;
-        if (x0 < HE) {
-            const int j = dev::upper_bound_m1(L.off, 0, nv, x0);
-            const int32_t split = L.off[j + 1];  // first entry of row j + 1
+        const uint32_t x0 = t * kHvTile + threadIdx.x * kHvPer;  // (x0 + k can pass 2^31)
+        if (x0 < (uint32_t)HE) {
+            const int j = dev::upper_bound_m1(L.off, 0, nv, (int32_t)x0);
+            const uint32_t split = L.off[j + 1];  // first entry of row j + 1
             int32_t idx[kHvPer], u[kHvPer];
 #pragma unroll
             for (int k = 0; k < kHvPer; ++k) {
-                const int32_t x = x0 + k;
+                const uint32_t x = x0 + k;
                 const int jj = x >= split ? j + 1 : j;
                 idx[k] = -1;
-                if (x < HE && jj < nv) idx[k] = L.start[jj] + (x - L.off[jj]);
+                if (x < (uint32_t)HE && jj < nv) idx[k] = L.start[jj] + (int32_t)(x - L.off[jj]);
                 if ((uint32_t)idx[k] >= (uint32_t)nnz) idx[k] = -1;  // guard only
                 u[k] = idx[k] >= 0 ? col[idx[k]] : -1;
             }
@@ -598,66 +598,67 @@ __global__ __launch_bounds__(kLfBlock) void k_light_first(const int32_t *__restr
     for (int64_t v0 = (blockIdx.x * (int64_t)(kLfBlock / 64) + threadIdx.x / 64) * kRows; v0 < m;
          v0 += step) {
         const int64_t v = v0 + lane / kLfLanes;
-        const int32_t rs = v < m ? rowptr[v] : 0, re = v < m ? rowptr[v + 1] : 0;
+        // (unsigned: a step past a row's end can pass 2^31)
+        const uint32_t rs = v < m ? rowptr[v] : 0, re = v < m ? rowptr[v + 1] : 0;
         const bool mine = re - rs <= kLfShort;
         float x[kLfPer];
         int32_t c[kLfPer];
 #pragma unroll
         for (int k = 0; k < kLfPer; ++k) {
-            const int32_t e = rs + k * kLfLanes + sub;
+            const uint32_t e = rs + k * kLfLanes + sub;
             const bool in = mine && e < re;
             x[k] = in ? val[e] : 0.0f;
             c[k] = in ? col[e] : 0;
         }
         uint64_t bl[kLfPer];
-        int32_t nl = 0;
+        uint32_t nl = 0;
 #pragma unroll
         for (int k = 0; k < kLfPer; ++k) {
             const bool in = mine && rs + k * kLfLanes + sub < re;
             bl[k] = __ballot(in && x[k] < delta) & group;
             nl += __popcll(bl[k]);
         }
-        int32_t lpos = rs, hpos = rs + nl;
+        uint32_t lpos = rs, hpos = rs + nl;
 #pragma unroll
         for (int k = 0; k < kLfPer; ++k) {
             const bool in = mine && rs + k * kLfLanes + sub < re;
             const bool light = in && x[k] < delta;
             const uint64_t bh = __ballot(in && !light) & group;
             if (in) {
-                const int32_t p = light ? lpos + __popcll(bl[k] & below) : hpos + __popcll(bh & below);
+                const uint32_t p = light ? lpos + __popcll(bl[k] & below) : hpos + __popcll(bh & below);
                 lcol[p] = c[k];
                 lval[p] = x[k];
             }
             lpos += __popcll(bl[k]);
             hpos += __popcll(bh);
         }
-        if (mine && sub == 0 && v < m) lend[v] = rs + nl;
+        if (mine && sub == 0 && v < m) lend[v] = (int32_t)(rs + nl);
         if (re - rs > kLfWave && sub == 0) hubs[dev::atomic_add_dev(nhubs, 1u)] = (int32_t)v;
         uint64_t longm = __ballot(!mine && re - rs <= kLfWave && sub == 0);
         while (longm) {
             const int from = __ffsll((unsigned long long)longm) - 1;
             longm &= longm - 1;
-            const int32_t ls = __shfl(rs, from, 64), le = __shfl(re, from, 64);
+            const uint32_t ls = __shfl(rs, from, 64), le = __shfl(re, from, 64);
             // kLfStep entries a step, their loads in flight; a row of one
             // step is counted from the registers it is written from
             uint32_t cnt = 0;
             if (le - ls > kLfStep) {
-                for (int32_t e0 = ls; e0 < le; e0 += kLfStep)
+                for (uint32_t e0 = ls; e0 < le; e0 += kLfStep)
 #pragma unroll
                     for (int k = 0; k < kLfPer; ++k) {
-                        const int32_t e = e0 + k * 64 + lane;
+                        const uint32_t e = e0 + k * 64 + lane;
                         cnt += e < le && val[e] < delta ? 1u : 0u;
                     }
                 cnt = (uint32_t)dev::wave_sum_u64(cnt);
             }
-            int32_t lp = ls, hp = ls + (int32_t)cnt;
-            for (int32_t e0 = ls; e0 < le; e0 += kLfStep) {
+            uint32_t lp = ls, hp = ls + cnt;
+            for (uint32_t e0 = ls; e0 < le; e0 += kLfStep) {
                 float y[kLfPer];
                 int32_t d[kLfPer];
                 uint64_t ml[kLfPer], mh[kLfPer];
 #pragma unroll
                 for (int k = 0; k < kLfPer; ++k) {
-                    const int32_t e = e0 + k * 64 + lane;
+                    const uint32_t e = e0 + k * 64 + lane;
                     y[k] = e < le ? val[e] : 0.0f;
                     d[k] = e < le ? col[e] : 0;
                 }
@@ -671,12 +672,12 @@ __global__ __launch_bounds__(kLfBlock) void k_light_first(const int32_t *__restr
                 }
                 if (le - ls <= kLfStep) {
                     cnt = step;
-                    hp = ls + (int32_t)cnt;
+                    hp = ls + cnt;
                 }
 #pragma unroll
                 for (int k = 0; k < kLfPer; ++k) {
                     if (e0 + k * 64 + lane < le) {
-                        const int32_t p = (ml[k] >> lane) & 1u ? lp + __popcll(ml[k] & below)
+                        const uint32_t p = (ml[k] >> lane) & 1u ? lp + __popcll(ml[k] & below)
                                                                : hp + __popcll(mh[k] & below);
                         lcol[p] = d[k];
                         lval[p] = y[k];
@@ -685,7 +686,7 @@ __global__ __launch_bounds__(kLfBlock) void k_light_first(const int32_t *__restr
                     hp += __popcll(mh[k]);
                 }
             }
-            if (lane == from) lend[v] = ls + (int32_t)cnt;
+            if (lane == from) lend[v] = (int32_t)(ls + cnt);
         }
     }
 }
@@ -701,29 +702,30 @@ __global__ __launch_bounds__(kLfHubBlock) void k_light_first_hubs(
     const uint64_t below = (1ull << lane) - 1;
     const uint32_t n = *nhubs;
     for (uint32_t q = blockIdx.x; q < n; q += gridDim.x) {
-        const int32_t v = hubs[q], rs = rowptr[v], re = rowptr[v + 1];
+        const int32_t v = hubs[q];
+        const uint32_t rs = rowptr[v], re = rowptr[v + 1];
         // a wave takes kLfHubPer * 64 consecutive entries of a step
-        const int32_t first = rs + (threadIdx.x & ~63) * kLfHubPer + lane;
+        const uint32_t first = rs + (threadIdx.x & ~63) * kLfHubPer + lane;
         uint32_t cnt = 0;
-        for (int32_t e0 = 0; first - lane + e0 < re; e0 += kStep)
+        for (uint32_t e0 = 0; first - lane + e0 < re; e0 += kStep)
 #pragma unroll
             for (int k = 0; k < kLfHubPer; ++k) {
-                const int32_t e = first + e0 + k * 64;
+                const uint32_t e = first + e0 + k * 64;
                 cnt += e < re && val[e] < delta ? 1u : 0u;
             }
         dev::Pair32 tot;
         (void)dev::block_exclusive_add_pair<kLfHubBlock>(cnt, 0u, s_scan, tot);
-        const int32_t nl = (int32_t)tot.a;
-        if (threadIdx.x == 0) lend[v] = rs + nl;
-        int32_t lp = rs, hp = rs + nl;
-        for (int32_t e0 = 0; rs + e0 < re; e0 += kStep) {
+        const uint32_t nl = tot.a;
+        if (threadIdx.x == 0) lend[v] = (int32_t)(rs + nl);
+        uint32_t lp = rs, hp = rs + nl;
+        for (uint32_t e0 = 0; rs + e0 < re; e0 += kStep) {
             float x[kLfHubPer];
             int32_t c[kLfHubPer];
             uint64_t ml[kLfHubPer], mh[kLfHubPer];
             uint32_t wl = 0, wh = 0;
 #pragma unroll
             for (int k = 0; k < kLfHubPer; ++k) {
-                const int32_t e = first + e0 + k * 64;
+                const uint32_t e = first + e0 + k * 64;
                 x[k] = e < re ? val[e] : 0.0f;
                 c[k] = e < re ? col[e] : 0;
             }
@@ -738,12 +740,12 @@ __global__ __launch_bounds__(kLfHubBlock) void k_light_first_hubs(
             __syncthreads();  // s_scan's last readers
             const dev::Pair32 ex = dev::block_exclusive_add_pair<kLfHubBlock>(
                 lane == 0 ? wl : 0u, lane == 0 ? wh : 0u, s_scan, tot);
-            int32_t l = lp + (int32_t)dev::wave_read_lane(ex.a, 0);
-            int32_t h = hp + (int32_t)dev::wave_read_lane(ex.b, 0);
+            uint32_t l = lp + dev::wave_read_lane(ex.a, 0);
+            uint32_t h = hp + dev::wave_read_lane(ex.b, 0);
 #pragma unroll
             for (int k = 0; k < kLfHubPer; ++k) {
                 if (first + e0 + k * 64 < re) {
-                    const int32_t p = (ml[k] >> lane) & 1u ? l + __popcll(ml[k] & below)
+                    const uint32_t p = (ml[k] >> lane) & 1u ? l + __popcll(ml[k] & below)
                                                            : h + __popcll(mh[k] & below);
                     lcol[p] = c[k];
                     lval[p] = x[k];
@@ -751,8 +753,8 @@ __global__ __launch_bounds__(kLfHubBlock) void k_light_first_hubs(
                 l += __popcll(ml[k]);
                 h += __popcll(mh[k]);
             }
-            lp += (int32_t)tot.a;
-            hp += (int32_t)tot.b;
+            lp += tot.a;
+            hp += tot.b;
         }
         __syncthreads();  // s_scan is written by the next row
     }

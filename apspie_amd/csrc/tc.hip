@@ -617,7 +617,8 @@ __global__ __launch_bounds__(kBitsBlock) __attribute__((amdgpu_waves_per_eu(8)))
         }
         __syncthreads();
         uint32_t c = 0;
-        int32_t pos = 0, end = 0, j = -1;
+        uint32_t pos = 0, end = 0;  // (a step past a pair's end can pass 2^31)
+        int32_t j = -1;
         for (;;) {
             if (pos >= end) {  // uniform in the group: its pair is done
                 if (!own && j >= 0) {
@@ -641,7 +642,7 @@ __global__ __launch_bounds__(kBitsBlock) __attribute__((amdgpu_waves_per_eu(8)))
             int32_t key[kScan];
 #pragma unroll
             for (int q = 0; q < kScan; ++q) {
-                const int32_t e = pos + sub + q * kGroup;
+                const uint32_t e = pos + sub + q * kGroup;
                 key[q] = e < end ? col[e] : -1;
             }
 #pragma unroll
