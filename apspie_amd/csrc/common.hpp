@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include <atomic>
+#include <chrono>
 #include <cstdint>
 #include <deque>
 #include <cstdio>
@@ -129,6 +130,8 @@ struct Ctx {
     std::deque<Buffer> spares;
     size_t spare_bytes = 0;
     std::map<void *, size_t> spare_sizes;  // handed out again: bytes of the block
+    bool ample_room = false;  // may_keep_blocks: the answer, and until when it stands
+    std::chrono::steady_clock::time_point room_until{};
     // graphs whose memory is accounted to this context
     std::set<Graph *> graphs;
     // event pairs of the kernel timer (option "profiling"), reused by calls
@@ -153,7 +156,7 @@ hipError_t device_malloc(Ctx *c, void **p, size_t bytes);
 // spare blocks where one fits.  A block is kept only where may_keep_blocks() has
 // waited for every stream.
 void *graph_alloc(Ctx *c, size_t bytes);
-bool may_keep_blocks();
+bool may_keep_blocks(Ctx *c);
 void graph_free(Ctx *c, void *p, size_t bytes, bool keep);
 // The arrays that a graph of context c has so far, if any.
 void graph_release(Ctx *c, Graph *g);
