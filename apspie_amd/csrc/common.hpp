@@ -215,6 +215,9 @@ void bfs_run_in(Ctx *c, const Graph *g, int32_t source, int32_t *depth_dev, void
                 int64_t bytes);
 void sssp_run(Ctx *c, const Graph *g, int32_t source, float *dist_dev);
 void mis_run(Ctx *c, const Graph *g, const uint32_t *prio_dev, int32_t *out_dev);
+// whether the tuned values of tc_medium_row / spgemm_*_ub move any row of such a call
+bool tc_uses_medium_row(const Graph *g);
+bool spgemm_uses_bounds(Ctx *c, int32_t n);
 void tc_run(Ctx *c, const Graph *g, uint64_t *total, int32_t *per_row_dev);
 int64_t spmspv_run(Ctx *c, const Graph *g, int semiring, int64_t nx, const int32_t *x_ind,
                    const float *x_val, const int32_t *mask, int32_t *y_ind, float *y_val,

@@ -37,9 +37,9 @@ static const char *kOptionNames[] = {
                            // symmetric weights (0 = never)
     "batch_long_row_group", // batched BFS on graphs with rows longer than 64: sources per
                             // pass (1..512)
-    "tc_medium_row",     // TC: rows with |L_r| up to this go to the 256-thread LDS tier, longer
-                         // ones to the 1024-thread tier (128..2048; 512 measured best or within
-                         // 4 % on R-MAT-18/20/22: 1.2-1.6x faster than 2048)
+    "tc_medium_row",     // TC above 2^20 vertices: rows with |L_r| up to this go to the 256-thread
+                         // LDS tier, longer ones to the 1024-thread tier (128..2048; R-MAT-22,
+                         // ms at 128 / 256 / 512 / 1024 / 2048: 60.4 / 58.9 / 58.4 / 61.6 / 72.2)
     "spgemm_wave_ub",    // SpGEMM: rows with at most this many products to the wave tier (<= 256; with the
                          // dense accumulator and up to 16384 columns, at most 64 of them)
     "spgemm_block_ub",   // SpGEMM: up to this to the block LDS tier (<= 4096) where B has more than

@@ -705,6 +705,13 @@ __global__ __launch_bounds__(BLOCK) void k_rows_dense(
 
 }  // namespace
 
+// the dense accumulator takes every row above the smallest (see spgemm_run)
+static bool spgemm_small_dense(Ctx *c, int32_t n) {
+    return n <= kDenseN / 2 && opt(c, "spgemm_dense", 1) != 0;
+}
+
+bool spgemm_uses_bounds(Ctx *c, int32_t n) { return !spgemm_small_dense(c, n); }
+
 Graph *spgemm_run(Ctx *c, const Graph *a, const Graph *b) {
     const int32_t m = a->m;
     const int grid = fill_grid(c, kBlock, 4);
@@ -731,7 +738,7 @@ Graph *spgemm_run(Ctx *c, const Graph *a, const Graph *b) {
         // R-MAT-12 in the block tier's tables 415 us + 152 symbolic, here 82 + 69;
         // the wave tier took 32 us for its rows of up to 256 products and takes
         // 9 for those of up to 64
-        const bool small_dense = dense_ok && b->n <= kDenseN / 2;
+        const bool small_dense = spgemm_small_dense(c, b->n);
         const int32_t wave_ub = (int32_t)std::min<int64_t>(
             std::max<int64_t>(opt(c, "spgemm_wave_ub", kWaveUb), 1),
             small_dense ? kDenseFrom : kWaveUb);

@@ -693,6 +693,8 @@ void graph_prepare_tc(Ctx *c, Graph *g) {
     }
 }
 
+bool tc_uses_medium_row(const Graph *g) { return g->m > kTcBitsMax; }
+
 void tc_run(Ctx *c, const Graph *g0, uint64_t *total_out, int32_t *per_row) {
     Graph *g = const_cast<Graph *>(g0);
     *total_out = 0;
@@ -714,7 +716,7 @@ void tc_run(Ctx *c, const Graph *g0, uint64_t *total_out, int32_t *per_row) {
     // up to 2^20 vertices every row above the small tier takes the
     // bit-per-vertex kernel, which k_tc_bits has the figures for; above that
     // its bits do not fit the LDS and the hash tables take them
-    const bool bits = m <= kTcBitsMax;
+    const bool bits = !tc_uses_medium_row(g);
     k_tc_bin<<<(int)std::min<int64_t>(grid, ceil_div(m, kBlock * kBinPer)), kBlock, 0,
                c->stream>>>(g->lowcnt, m, kSmallRow, bits ? kSmallRow : medium_row,
                             bits ? INT32_MAX : kBigRow, lists, ctl, per);

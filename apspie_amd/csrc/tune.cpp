@@ -15,10 +15,13 @@
 //     hipGraph chunk, then the pull threshold, and for a weighted graph the
 //     batched SSSP width (Bellman-Ford, 256, 1024);
 //   apspie_autotune_hash: TC's medium / big tier bound (a 256-thread block
-//     with a 4096-slot LDS table vs a 1024-thread block with 32768 slots),
-//     then SpGEMM's wave / block tier bounds (512- and 8192-slot tables) and
+//     with a 4096-slot LDS table vs a 1024-thread block with 32768 slots; above
+//     2^20 vertices), then SpGEMM's wave / block tier bounds (512- and 8192-slot
+//     tables; above 16384 columns, or without the dense accumulator) and
 //     whether rows beyond them use the dense accumulator or global tables
-//     (A * A; skipped when the product does not fit one call).
+//     (A * A; skipped when the product does not fit one call).  A bound that no
+//     row of the graph meets is left as it is: its candidates would differ by
+//     noise only.
 // Every candidate is timed three times (median of the calls' device time);
 // the buffers come from the context's scratch pool (its HBM budget applies)
 // and every copy runs on its stream.
@@ -199,7 +202,8 @@ extern "C" int apspie_autotune_hash(apspie_ctx *c, const apspie_graph *g) {
         set_device(c);
         // TC (rows sorted): the medium / big tier bound
         uint64_t total = 0;
-        if (apspie_tc(c, g, &total, nullptr, APSPIE_MEM_HOST) == APSPIE_OK)
+        if (tc_uses_medium_row(g) &&
+            apspie_tc(c, g, &total, nullptr, APSPIE_MEM_HOST) == APSPIE_OK)
             pick(c, "tc_medium_row", {256, 512, 1024, 2048},
                  [&] { return apspie_tc(c, g, &total, nullptr, APSPIE_MEM_HOST); });
         // SpGEMM A * A: the wave / block bounds jointly, then dense or global
@@ -229,18 +233,23 @@ extern "C" int apspie_autotune_hash(apspie_ctx *c, const apspie_graph *g) {
         if (first == APSPIE_ERR_OVERFLOW || first == APSPIE_ERR_OOM || first == APSPIE_ERR_BUDGET)
             return;
         APSPIE_CHECK(first == APSPIE_OK, first, "autotune run failed: " + c->last_error);
-        double best = 1e300;
-        int64_t bw = 256, bk = 4096;
-        for (int64_t wub : {64, 128, 256})
-            for (int64_t bub : {1024, 2048, 4096}) {
-                apspie_ctx_set_option(c, "spgemm_wave_ub", wub);
-                apspie_ctx_set_option(c, "spgemm_block_ub", bub);
-                const double t = median_ms(c, product);
-                if (t < best) { best = t; bw = wub; bk = bub; }
-            }
-        apspie_ctx_set_option(c, "spgemm_wave_ub", bw);
-        apspie_ctx_set_option(c, "spgemm_block_ub", bk);
+        auto bounds = [&] {
+            double best = 1e300;
+            int64_t bw = 256, bk = 4096;
+            for (int64_t wub : {64, 128, 256})
+                for (int64_t bub : {1024, 2048, 4096}) {
+                    apspie_ctx_set_option(c, "spgemm_wave_ub", wub);
+                    apspie_ctx_set_option(c, "spgemm_block_ub", bub);
+                    const double t = median_ms(c, product);
+                    if (t < best) { best = t; bw = wub; bk = bub; }
+                }
+            apspie_ctx_set_option(c, "spgemm_wave_ub", bw);
+            apspie_ctx_set_option(c, "spgemm_block_ub", bk);
+        };
+        const bool bounded = spgemm_uses_bounds(c, g->n);
+        if (bounded) bounds();
         if (g->n <= 32768) pick(c, "spgemm_dense", {0, 1}, product);
+        if (!bounded && spgemm_uses_bounds(c, g->n)) bounds();
     });
 }
 

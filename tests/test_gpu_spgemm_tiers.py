@@ -90,3 +90,23 @@ def test_float_sums_against_64_bits(ctx, n):
     assert np.array_equal(got[0], want.indptr) and np.array_equal(got[1], want.indices)
     err = np.abs(got[2].astype(np.float64) - want.data) / want.data
     assert np.all(err <= (terms.data + 1) * 2.0 ** -24)
+
+
+def test_autotune_leaves_bounds_that_move_no_row():
+    """4096 vertices: the bit-per-vertex triangle count and the dense accumulator
+    take all rows the bounds would bin, so their values stay the caller's."""
+    rp, c = A.gen_rmat(12)
+    with A.Context(0) as ctx:
+        G = ctx.upload(rp, c, np.ones(len(c), np.float32))
+        mine = {"tc_medium_row": 700, "spgemm_wave_ub": 100, "spgemm_block_ub": 3000}
+        for name, v in mine.items():
+            ctx.set_option(name, v)
+        ctx.autotune_hash(G)
+        assert ctx.get_option("tc_medium_row") == 700
+        if ctx.get_option("spgemm_dense"):  # else the tables win, and are tuned
+            assert {k: ctx.get_option(k) for k in mine} == mine
+        ctx.set_option("spgemm_dense", 0)
+        ctx.autotune_hash(G)
+        assert ctx.get_option("spgemm_wave_ub") in (64, 128, 256)
+        assert ctx.get_option("spgemm_block_ub") in (1024, 2048, 4096)
+        G.close()
