@@ -884,13 +884,23 @@ double sssp_weight_delta(Ctx *c, Graph *g) {
 // The width used when sssp_delta is left at -1.
 //
 // Sparse rows (the weights' width above every weight, so that no entry is
-// heavy): four times that width from kNfFrom vertices on -- the rounds'
-// fixed cost (about 8 us) weighs more than the re-expansions a wider bucket
-// adds -- and Bellman-Ford rounds (0) below.  Lattices at weights 1..255, ms
-// per source, Bellman-Ford / 512 / 2048 / 8192: 512^2 1.14 / 1.76 / 1.30 /
-// 1.28, 724^2 1.43 / - / 1.51 / -, 887^2 1.76 / - / 1.62 / -, 1024^2 2.06 / 2.28
-// / 1.73 / 2.17, 1500^2 3.40 / 2.87 / 2.33 / 3.36, 2048^2 5.68 / 3.27 / 2.84 /
-// 4.45.
+// heavy), kNfFrom vertices or more (fewer: Bellman-Ford rounds, 0): a wide
+// bucket, for the rounds' fixed cost (about 8 us) weighs more than the
+// re-expansions it adds, as long as the paths are long.  On graphs with short
+// paths four times the width is all of them, Bellman-Ford rounds in effect: no
+// loss against those below kNfWide vertices, but from there on the width itself
+// is better.  Long paths are told from short ones by the longest row: 8 entries
+// at most on lattices with a few far edges, 16 and more on random graphs of a
+// mean row of 3.  Weights 1..255, ms per source, Bellman-Ford / 256 / 512 / 1024 /
+// 2048 / 4096.  Lattices (width 512): 900^2 2.03 / 2.87 / 2.17 / 1.85 / 1.64 /
+// 1.67, 1024^2 2.16 / 3.05 / 2.36 / 1.98 / 1.85 / 1.81, 1774^2 4.52 / 3.77 / 3.02 /
+// 2.70 / 2.57 / 2.88, 2048^2 6.14 / 4.14 / 3.34 / 2.98 / 3.01 / 3.18, 2896^2 11.7 /
+// 5.42 / 4.51 / 4.17 / 4.36 / 4.59.  Random edges, mean row 4 (width 512), 2^20
+// vertices 0.79 / 0.80 / 0.70 / 0.68 / 0.83 / 0.84, 2^22 2.31 / 1.51 / 1.46 / 1.45 /
+// 2.38 / 2.37; mean row 8 (256), 2^20 1.27 / 0.86 / 0.88 / 1.32 / 1.31 / 1.32, 2^22
+// 4.43 / 1.86 / 1.85 / 4.43 / 4.47 / 4.46; mean row 12 (256), 2^22 6.02 / 3.37 /
+// 4.17 / 6.03 / 6.07 / 6.09.  Smaller lattices, Bellman-Ford / 2048: 512^2 1.14 /
+// 1.30, 724^2 1.43 / 1.51.
 //
 // Longer rows (light / heavy rounds): 1.42 * largest weight / sqrt(mean row),
 // narrower on large graphs by (2^20 / m)^0.4, from kNfFrom vertices on too.
@@ -904,13 +914,16 @@ double sssp_weight_delta(Ctx *c, Graph *g) {
 // 0.67 / 0.67 / 0.52 / 0.55 / 0.57, 2^20 1.39 / 1.15 / 1.08 / 1.07 / 1.12, 2^22
 // 4.44 / 2.67 / 2.76 / 2.93 / 3.23; edge factor 8: 2^20 1.09 / 0.99 / 0.87 / 0.92 /
 // 0.78, 2^22 2.95 / 1.99 / 1.94 / 2.00 / 2.19.
-constexpr int32_t kNfFrom = 3 << 18;
+constexpr int32_t kNfFrom = 3 << 18, kNfWide = 1 << 22, kLongPathRow = 8;
 double sssp_auto_delta(Ctx *c, Graph *g) {
     if (g->m < kNfFrom) return 0;
     const double d = sssp_weight_delta(c, g);
     float lo = 0.0f, hi = 0.0f;
     if (!(d > 0) || !graph_weight_range(c, g, &lo, &hi)) return 0;
-    if (d > hi) return 4 * d;
+    if (d > hi) {
+        if (g->m < kNfWide) return 4 * d;
+        return graph_max_degree(c, g) <= kLongPathRow ? 2 * d : d;
+    }
     if (opt(c, "sssp_light_heavy", 1) == 0) return g->m >= (1 << 22) ? d : 0;
     const double w = 1.42 * hi / std::sqrt(std::max(1.0, (double)g->nnz / g->m)) *
                      std::min(1.0, std::pow((double)(1 << 20) / g->m, 0.4));

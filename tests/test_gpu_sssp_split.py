@@ -53,3 +53,22 @@ def test_default_width_of_longer_rows(m, near_far):
         assert np.array_equal(ctx.sssp(G, 0), np.where(np.arange(m) == 0, 0, 200))
         assert (ctx.stats()["iterations"] != 2) == near_far
         G.close()
+
+
+@pytest.mark.parametrize("mean,most", [(4, 0.7), (8, 0.5)])
+def test_default_width_of_large_random_graphs(mean, most):
+    """2^22 vertices, short rows, short paths: a bucket as wide as the paths
+    would re-expand what Bellman-Ford rounds do (at most 0.4 of it at the
+    weights' own width)."""
+    m = 1 << 22
+    rng = np.random.default_rng(mean)
+    u, v = rng.integers(0, m, (2, m * mean // 2), dtype=np.int32)
+    w = rng.integers(1, 256, len(u)).astype(np.float32)
+    with A.Context(0) as ctx:
+        G = ctx.from_coo(m, u, v, w)
+        got = ctx.sssp(G, int(u[0]))
+        edges = ctx.stats()["edges_traversed"]
+        ctx.set_option("sssp_delta", 0)
+        assert np.array_equal(got, ctx.sssp(G, int(u[0])))
+        assert edges < most * ctx.stats()["edges_traversed"]
+        G.close()
