@@ -259,12 +259,13 @@ void graph_free(Ctx *c, void *p, size_t bytes, bool keep) {
 void graph_release(Ctx *c, Graph *g) {
     if (!g->rowptr && !g->col && !g->val) return;
     (void)hipSetDevice(c->device);
+    const size_t rows = sizeof(int32_t) * (g->m + 1), entries = sizeof(int32_t) * g->nnz;
     // every stream, as hipFree waits: another context or the caller's own
     // stream may still read the arrays, and they are given out again
-    const bool keep = may_keep_blocks(c);
-    graph_free(c, g->rowptr, sizeof(int32_t) * (g->m + 1), keep);
-    graph_free(c, g->col, sizeof(int32_t) * g->nnz, keep);
-    graph_free(c, g->val, sizeof(float) * g->nnz, keep);
+    const bool keep = std::max(rows, entries) >= kSpareMin && may_keep_blocks(c);
+    graph_free(c, g->rowptr, rows, keep);
+    graph_free(c, g->col, entries, keep);
+    graph_free(c, g->val, entries, keep);
     g->rowptr = g->col = nullptr;
     g->val = nullptr;
 }
