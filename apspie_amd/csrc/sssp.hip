@@ -773,7 +773,10 @@ Graph::LightFirst graph_light_first(Ctx *c, Graph *g, float delta) {
     const size_t bytes = 2 * ecol + sizeof(int32_t) * ((size_t)g->m + 1);
     void *mem = nullptr;
     // owned by the graph (freed with it), like its other derived arrays
-    APSPIE_HIP(device_malloc(c, (void **)&mem, bytes));
+    if (device_malloc(c, &mem, bytes) != hipSuccess) {
+        (void)hipGetLastError();
+        throw Error{APSPIE_ERR_OOM, "no room for the light-first rows"};
+    }
     int32_t *lcol = (int32_t *)mem;
     float *lval = (float *)((char *)mem + ecol);
     int32_t *lend = (int32_t *)((char *)mem + 2 * ecol);
@@ -943,14 +946,21 @@ double sssp_batch_auto_delta(Ctx *c, Graph *g) {
 }
 
 void sssp_run(Ctx *c, const Graph *g, int32_t source, float *dist) {
-    double delta = (double)opt(c, "sssp_delta", -1);
-    if (delta < 0) delta = sssp_auto_delta(c, const_cast<Graph *>(g));
+    const double asked = (double)opt(c, "sssp_delta", -1);
+    const double delta = asked < 0 ? sssp_auto_delta(c, const_cast<Graph *>(g)) : asked;
     if (delta > 0) {
-        switch (opt(c, "bfs_tile", 2048)) {
-        case 1024: sssp_near_far<1024>(c, g, source, dist, (float)delta); return;
-        case 4096: sssp_near_far<4096>(c, g, source, dist, (float)delta); return;
-        default: sssp_near_far<2048>(c, g, source, dist, (float)delta); return;
+        try {
+            switch (opt(c, "bfs_tile", 2048)) {
+            case 1024: sssp_near_far<1024>(c, g, source, dist, (float)delta); return;
+            case 4096: sssp_near_far<4096>(c, g, source, dist, (float)delta); return;
+            default: sssp_near_far<2048>(c, g, source, dist, (float)delta); return;
+            }
+        } catch (const Error &e) {
+            // near-far rounds need a byte per vertex more than Bellman-Ford rounds,
+            // and maybe the light-first rows: a default that does not fit gives way
+            if (asked >= 0 || (e.status != APSPIE_ERR_OOM && e.status != APSPIE_ERR_BUDGET)) throw;
         }
+        for (const char *name : {"sssp_pend", "sssp_hb", "sssp_hubs"}) scratch_drop(c, name);
     }
     // pulled rounds read w(v, u) for the edge u -> v: symmetric values only
     int32_t pull_div = (int32_t)opt(c, "sssp_pull_div", 0);

@@ -72,3 +72,32 @@ def test_default_width_of_large_random_graphs(mean, most):
         assert np.array_equal(got, ctx.sssp(G, int(u[0])))
         assert edges < most * ctx.stats()["edges_traversed"]
         G.close()
+
+
+@pytest.mark.parametrize("kind", ["lattice", "rmat"])
+def test_default_width_gives_way_to_a_budget(kind):
+    """Where only Bellman-Ford rounds fit the budget the default takes those; a
+    width that was asked for is refused."""
+    rp, c = A.gen_lattice(900) if kind == "lattice" else A.gen_rmat(20)
+    w = A.gen_weights(rp, c)
+    m, src = len(rp) - 1, int(np.argmax(np.diff(rp)))
+    with A.Context(0) as ctx:
+        G = ctx.upload(rp, c, w)
+        out = ctx.dev_alloc(4 * m)
+        ctx.set_option("sssp_delta", 0)
+        ctx.sssp(G, src, out=out.ptr, mem=A.DEVICE)
+        want = out.to_host(np.float32, m)
+        need = ctx.hbm_used()
+        ctx.trim()
+        ctx.set_hbm_budget(need)
+        ctx.set_option("sssp_delta", 64)
+        with pytest.raises(A.ApspieError):
+            ctx.sssp(G, src, out=out.ptr, mem=A.DEVICE)
+        ctx.trim()
+        ctx.set_option("sssp_delta", -1)
+        for _ in range(2):
+            out.from_host(np.zeros(m, np.float32))
+            ctx.sssp(G, src, out=out.ptr, mem=A.DEVICE)
+            assert np.array_equal(out.to_host(np.float32, m), want)
+        out.free()
+        G.close()
