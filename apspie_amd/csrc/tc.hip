@@ -561,7 +561,10 @@ __global__ __launch_bounds__(BLOCK) void k_tc_block(const int32_t *rowptr, const
 // pair from the item's LDS counter: no prefix sum and no search per wedge.
 // Against the hash tiers: R-MAT-18 1.76 -> 0.41 ms (of 380 M wedges in all,
 // 1.5 a cycle and CU), R-MAT-20 (the 32768-word instance, one block per CU) a
-// call 10.1 -> 4.3 ms.
+// call 10.1 -> 4.3 ms.  Up to 2^18 vertices the bits fit 32 KB and two blocks a
+// CU: R-MAT-18 a call 0.72 ms, with the large instance 0.99; above, only that one
+// holds them (2^18 + 4096 vertices 1.03 ms, 2^19 1.94, 2^20 4.2; one of 64 KB for
+// up to 2^19 is not built), and above 2^20 no CU's LDS does (2^20 + 4096: 9.4).
 constexpr int kTcBitsWords = 8192, kTcBitsMax = 1 << 20;
 constexpr int kBitsBlock = 1024;  // two blocks per CU at 8192 words, one at 32768
 constexpr int kBitsChunk = 512;
@@ -714,8 +717,7 @@ void tc_run(Ctx *c, const Graph *g0, uint64_t *total_out, int32_t *per_row) {
         (int32_t)std::min<int64_t>(std::max<int64_t>(opt(c, "tc_medium_row", 512), kSmallRow),
                                    kMediumRow);
     // up to 2^20 vertices every row above the small tier takes the
-    // bit-per-vertex kernel, which k_tc_bits has the figures for; above that
-    // its bits do not fit the LDS and the hash tables take them
+    // bit-per-vertex kernel (figures there); above, the hash tables take them
     const bool bits = !tc_uses_medium_row(g);
     k_tc_bin<<<(int)std::min<int64_t>(grid, ceil_div(m, kBlock * kBinPer)), kBlock, 0,
                c->stream>>>(g->lowcnt, m, kSmallRow, bits ? kSmallRow : medium_row,
