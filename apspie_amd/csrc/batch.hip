@@ -32,6 +32,7 @@ namespace {
 constexpr int kBlock = 256;
 constexpr int kTile = 2048;
 constexpr int kMaxBatch = 512;  // sources per pass (larger batches are split)
+constexpr int kPullStep = 4;    // row entries a pulled SSSP round loads at once
 
 // the W words of a vertex's bit row (16-byte loads when W is a multiple of 4;
 // rows of W words are W * 4-byte aligned)
@@ -306,7 +307,7 @@ __device__ __forceinline__ void batch_pull(PullLds<LONG> &lds, const int32_t *__
     dev::Pair32 found{0, 0};
     for (int64_t pbase = (int64_t)blockIdx.x * VPB * KP; pbase < m;
          pbase += (int64_t)gridDim.x * VPB * KP) {
-        uint32_t rs[KP], re[KP];  // (a step past a row's end can pass 2^31)
+        int32_t rs[KP], re[KP];
         uint32_t uv[KP], acc[KP];
 #pragma unroll
         for (int k = 0; k < KP; ++k) {
@@ -323,7 +324,7 @@ __device__ __forceinline__ void batch_pull(PullLds<LONG> &lds, const int32_t *__
         for (int k = 0; k < KP; ++k)
 #pragma unroll
             for (int t = 0; t < Q; ++t)
-                u[k][t] = uv[k] && rs[k] + t < re[k] ? col[rs[k] + t] : -1;
+                u[k][t] = uv[k] && t < re[k] - rs[k] ? col[rs[k] + t] : -1;
 #pragma unroll
         for (int k = 0; k < KP; ++k)
 #pragma unroll
@@ -350,10 +351,12 @@ __device__ __forceinline__ void batch_pull(PullLds<LONG> &lds, const int32_t *__
                     }
                 }
             }
-            for (uint32_t e = rs[k] + Q; e < re[k] && (acc[k] & uv[k]) != uv[k]; e += Q) {
+            // (offsets within the row: a step past its end can pass 2^31 in the CSR)
+            for (int32_t o = Q; o < re[k] - rs[k] && (acc[k] & uv[k]) != uv[k]; o += Q) {
                 int32_t uu[Q];
 #pragma unroll
-                for (int t = 0; t < Q; ++t) uu[t] = e + t < re[k] ? col[e + t] : -1;
+                for (int t = 0; t < Q; ++t)
+                    uu[t] = o + t < re[k] - rs[k] ? col[rs[k] + o + t] : -1;
 #pragma unroll
                 for (int t = 0; t < Q; ++t)
                     if (uu[t] >= 0) acc[k] |= front[(int64_t)uu[t] * W + w];
@@ -691,7 +694,7 @@ __device__ __forceinline__ void batch_sssp_pull(PullQueue &q, const int32_t *__r
     // four from four words on (128 / 256 / 512 sources: 0.616 / 0.598 /
     // 0.597 with two, 0.611 / 0.591 / 0.579 with four)
     constexpr int KP = W == 1 ? 1 : W == 2 ? 2 : 4;
-    constexpr int Q = 4;  // row entries loaded at once
+    constexpr int Q = kPullStep;
     constexpr int S = 4;  // sources relaxed at once
     constexpr int kPasses = kQueue / (VPB * KP);
     static_assert(kPasses >= 1, "one pass's claims fit the LDS queue");
@@ -710,12 +713,12 @@ __device__ __forceinline__ void batch_sssp_pull(PullQueue &q, const int32_t *__r
             crs[k] = 0;
             cd[k] = 0;
             uint32_t near = 0, far = 0;
-            uint32_t rs = 0, re = 0;  // (a step past a row's end can pass 2^31)
+            int32_t rs = 0, re = 0;
             if (v < m) {
                 rs = rowptr[v];
                 re = rowptr[v + 1];
                 int32_t *dv_row = op.word_of(v, w);
-                for (uint32_t e0 = rs; e0 < re; e0 += Q) {
+                for (int32_t e0 = rs; e0 < re; e0 += Q) {
                     int32_t u[Q];
                     uint32_t f[Q], x = 0;
                     float we[Q];
@@ -1084,9 +1087,12 @@ double sssp_batch_delta(Ctx *c, const Graph *g) {
     return d < 0 ? sssp_batch_auto_delta(c, const_cast<Graph *>(g)) : d;
 }
 
-// near-far rounds of a batch may pull (and keep their distances source-major)
+// near-far rounds of a batch may pull (and keep their distances source-major).  Not
+// on a graph whose last offsets a step of kPullStep entries would carry past 2^31
+// (comparing by the row's rest instead cost the 2048^2 lattice 1 %).
 bool sssp_rounds_pull(Ctx *c, const Graph *g) {
     return sssp_batch_delta(c, g) > 0 && opt(c, "batch_sssp_pull_div", 4) > 0 &&
+           g->nnz <= INT32_MAX - kPullStep &&
            graph_max_degree(c, const_cast<Graph *>(g)) <= 64 &&
            graph_is_symmetric_weighted(c, const_cast<Graph *>(g));
 }
